@@ -1,0 +1,48 @@
+"""The whole-lattice sums at the sizes where their kernels' work splits can go
+wrong: rows of one word and of more words than a workgroup has threads, more
+rows than the grid covers at once."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+Q = {0: 4, 1: 6, 2: 7, 3: 7}
+
+
+def make(model, dx, dy, r, solids):
+    from lgca_amd import Lattice
+    rng = np.random.default_rng(dx * 7 + dy + model)
+    state = rng.integers(0, 1 << Q[model], dx * dy, dtype=np.uint8)
+    types = rng.choice(np.array([0, 0, 0, 1, 2], np.uint8), dx * dy) if solids else np.zeros(dx * dy, np.uint8)
+    lat = Lattice(model, dim_x=dx, dim_y=dy, coarse_graining_radius=r)
+    if solids:
+        lat.set_cell_types(types)
+    lat.set_state_u8(state)
+    lat.copy_data_to_output_buffer()
+    return lat, state, types
+
+
+@pytest.mark.parametrize("model,dx,dy,solids", [
+    (0, 2, 3, False), (1, 31, 2, True), (2, 33, 8200, True), (3, 1000, 66, False),
+    (2, 32768 + 40, 4, True), (0, 70000, 5, True), (1, 4096, 300, False), (2, 2048, 2050, False)])
+def test_particle_count_and_mean_velocity_are_exact(model, dx, dy, solids):
+    print(f"[sum] model={model} {dx}x{dy} solids={solids}", flush=True)
+    lat, state, types = make(model, dx, dy, 1, solids)
+    assert lat.get_n_particles() == orc.count_particles(state)
+    b = [((state >> d) & 1).astype(np.int64) for d in range(Q[model])]
+    rho = sum(b)
+    if model == 0:
+        kx, ky, ux, uy = b[0] - b[2], b[1] - b[3], 1.0, 1.0
+    else:
+        kx, ky = 2 * b[0] + b[1] - b[2] - 2 * b[3] - b[4] + b[5], b[1] + b[2] - b[4] - b[5]
+        ux, uy = 0.5, float(np.float32(0.866025388240814208984375))
+    fluid = types == 0
+    n = float(fluid.sum())
+    per = np.where(fluid & (rho > 0), 840 // np.maximum(rho, 1), 0)
+    sx, sy = int((kx * per).sum()), int((ky * per).sum())
+    # the sums are exact integers, then one double division and one rounding
+    want = [float(np.float32(sx * ux / (840.0 * n))), float(np.float32(sy * uy / (840.0 * n)))] if n else [0.0, 0.0]
+    assert lat.get_mean_velocity() == want
+    lat.close()
