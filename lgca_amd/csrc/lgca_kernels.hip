@@ -465,12 +465,161 @@ hipError_t launch_cell_fields(int kind, const uint32_t* planes, const Geometry& 
 // of columns x0..x0+r on rows y0..y0+2r that exist, plus -- only when
 // dim_x == 2r -- the candidate x = 2r of each row, which wraps to column 0 of
 // the next row.  Sums are sequential FP32 in that order; one divide by the
-// count.  One thread per coarse cell keeps the order.
+// count.
+//
+// Density and x momentum (and HPP's y momentum) are sums of multiples of 1/2
+// that FP32 holds exactly for r up to kCoarseExactRadius, so any order gives
+// their bits and popcounts give the sums.  The y momentum of FHP rounds at
+// every cell: its chain of (2r + 1)(r + 1) dependent adds is the kernel's
+// bound (2145 adds at r = 32).  So one wave of a workgroup does nothing else,
+// one chain per lane for 64 coarse cells, with the addends already in LDS in
+// the order it needs; the other kCoarseProducers waves read the planes, up
+// to 16 columns of a row at a time (a unit), turn them into addends and keep the
+// popcounts.  An 8192 x 4096 lattice at r = 32: 242 us with one thread per
+// coarse cell doing all of it, waiting out a memory latency per word; 52 us so
+// (4400 x 2200 at r = 20: 113 and 25 us; 1480 x 740 at r = 10: 36 and 9.9 us).
+constexpr uint32_t kCoarseExactRadius = 1023;
+constexpr uint32_t kCoarseProducers = 7;
+
+// Addends of the y-momentum chain for the cells of one unit: bit j of the
+// four planes is cell j; out[j] = ky * sin(pi/3), ky = a1 + a2 - a4 - a5,
+// exact.  The float's bits are put together from three planes: zero or not,
+// |ky| == 2 (exponent one up), sign.
+__device__ __forceinline__ void y_addends(uint32_t a1, uint32_t a2, uint32_t a4, uint32_t a5, uint32_t quads,
+                                          float4* out)
+{
+    const uint32_t p1 = a1 ^ a2, p2 = a1 & a2, n1 = a4 ^ a5, n2 = a4 & a5;
+    uint32_t nz = (p1 ^ n1) | (p2 ^ n2);
+    uint32_t two = (p2 & ~(n1 | n2)) | (n2 & ~(p1 | p2));
+    uint32_t neg = (n2 & ~p2) | (n1 & ~(p1 | p2));
+    const uint32_t one = __float_as_uint(kSin60);
+    for (uint32_t k = 0; k < quads; ++k) {
+        float f[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t v = ((neg << (31 - j)) & 0x80000000u) | ((two << (23 - j)) & 0x00800000u) | one;
+            f[j] = __uint_as_float(v & (uint32_t)__builtin_amdgcn_sbfe((int)nz, j, 1));
+        }
+        out[k * 64] = make_float4(f[0], f[1], f[2], f[3]);
+        nz >>= 4;
+        two >>= 4;
+        neg >>= 4;
+    }
+}
+
 template <int KIND>
-__global__ __launch_bounds__(64) void coarse_kernel(const uint32_t* __restrict__ planes,
-                                                    Geometry g, uint32_t r,
-                                                    float* __restrict__ md, float* __restrict__ mm,
-                                                    float* __restrict__ vel)
+__global__ __launch_bounds__(64 * (1 + kCoarseProducers))
+void coarse_kernel(const uint32_t* __restrict__ planes, Geometry g, uint32_t r, uint32_t chunks, uint32_t chunk,
+                   float* __restrict__ md, float* __restrict__ mm, float* __restrict__ vel)
+{
+    constexpr int Q = num_dir_of_kind(KIND);
+    constexpr bool kChain = KIND != kHPP;
+    // [2 stages][producer][chunk / 4 quads][64 coarse cells] addends
+    extern __shared__ float4 addends[];
+    __shared__ int sums[kCoarseProducers][3][64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t cdx = g.dim_x / (2 * r), cdy = g.dim_y / (2 * r), nc = cdx * cdy;
+    const uint32_t c = blockIdx.x * 64 + lane;
+    const bool live = c < nc;
+    const uint32_t x0 = live ? (c % cdx) * 2 * r : 0u, y0 = live ? (c / cdx) * 2 * r : 0u;
+    const bool wrap_col = g.dim_x == 2 * r;
+    const uint32_t per_row = chunks + (wrap_col ? 1u : 0u), units = (2 * r + 1) * per_row;
+    const uint32_t stages = (units + kCoarseProducers - 1) / kCoarseProducers;
+    const uint32_t slot = chunk / 4 * 64;  // float4s of one unit
+    // cells of a unit: `chunk` columns of the row, the rest of the r + 1 in
+    // the last chunk, and the wrapped cell
+    auto unit_cells = [&](uint32_t i) {
+        return i >= chunks ? 1u : i + 1 == chunks ? r + 1 - (chunks - 1) * chunk : chunk;
+    };
+
+    int rho = 0, kx = 0, ky = 0;  // producers: density, x momentum in halves (HPP: ones), HPP y momentum
+    float sy = 0.0f;              // wave 0: the chain
+    uint32_t lo[Q], hi[Q];        // producers: the unit's plane words, loaded a stage ahead
+    auto load_unit = [&](uint32_t u) {
+        const uint32_t i = u % per_row, n = unit_cells(i);
+        const uint32_t y = y0 + u / per_row + (i >= chunks ? 1u : 0u), x = i >= chunks ? 0u : x0 + i * chunk;
+        const bool ok = live && u < units && y < g.dim_y;
+        const uint32_t* p = planes + (size_t)y * Q * g.P + (x >> 5);
+        const bool two = ok && (x & 31u) + n > 32;
+#pragma unroll
+        for (int d = 0; d < Q; ++d) {
+            lo[d] = ok ? p[(size_t)d * g.P] : 0u;
+            hi[d] = two ? p[(size_t)d * g.P + 1] : 0u;
+        }
+    };
+    if (wave) load_unit(wave - 1);
+    for (uint32_t st = 0; st <= stages; ++st) {
+        if (wave && st < stages) {
+            const uint32_t u = st * kCoarseProducers + wave - 1, i = u % per_row, n = unit_cells(i);
+            const uint32_t sh = i >= chunks ? 0u : (x0 + i * chunk) & 31u;
+            const uint32_t valid = n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u;
+            uint32_t a[Q];
+#pragma unroll
+            for (int d = 0; d < Q; ++d) a[d] = __builtin_amdgcn_alignbit(hi[d], lo[d], sh) & valid;
+            if (st + 1 < stages) load_unit(u + kCoarseProducers);
+#pragma unroll
+            for (int d = 0; d < Q; ++d) rho += __popc(a[d]);
+            if (KIND == kHPP) {
+                kx += __popc(a[0]) - __popc(a[2]);
+                ky += __popc(a[1]) - __popc(a[3]);
+            } else {
+                kx += 2 * (__popc(a[0]) - __popc(a[3])) + __popc(a[1]) - __popc(a[2]) - __popc(a[4]) + __popc(a[5]);
+                y_addends(a[1], a[2], a[4], a[5], (n + 3) / 4,
+                          addends + ((st & 1u) * kCoarseProducers + wave - 1) * slot + lane);
+            }
+        }
+        if (kChain && !wave && st) {
+            for (uint32_t p = 0; p < kCoarseProducers; ++p) {
+                const uint32_t u = (st - 1) * kCoarseProducers + p;
+                if (u >= units) break;
+                const uint32_t quads = (unit_cells(u % per_row) + 3) / 4;
+                const float4* a = addends + (((st - 1) & 1u) * kCoarseProducers + p) * slot + lane;
+#pragma unroll 4
+                for (uint32_t k = 0; k < quads; ++k) {
+                    const float4 v = a[k * 64];
+                    sy += v.x;
+                    sy += v.y;
+                    sy += v.z;
+                    sy += v.w;
+                }
+            }
+        }
+        if (kChain) __syncthreads();
+    }
+    if (wave) {
+        sums[wave - 1][0][lane] = rho;
+        sums[wave - 1][1][lane] = kx;
+        sums[wave - 1][2][lane] = ky;
+    }
+    __syncthreads();
+    if (wave || !live) return;
+    for (uint32_t p = 0; p < kCoarseProducers; ++p) {
+        rho += sums[p][0][lane];
+        kx += sums[p][1][lane];
+        ky += sums[p][2][lane];
+    }
+    const uint32_t rows = min(2 * r + 1, g.dim_y - y0);
+    const uint32_t wrapped = wrap_col ? min(rows, g.dim_y - 1 - y0) : 0u;
+    const float fc = (float)(int)(rows * (r + 1) + wrapped);
+    const float sd = (float)rho, sx = KIND == kHPP ? (float)kx : 0.5f * (float)kx;
+    if (KIND == kHPP) sy = (float)ky;
+    const float den = sd / fc, ux = sx / fc, uy = sy / fc;
+    md[c] = den;
+    mm[2 * c] = ux;
+    mm[2 * c + 1] = uy;
+    if (vel) {
+        vel[2 * c] = den > 0.0f ? ux / den : 0.0f;
+        vel[2 * c + 1] = den > 0.0f ? uy / den : 0.0f;
+    }
+}
+
+// The same one cell at a time, one thread per coarse cell, for radii whose
+// density sums FP32 may round (more than 2^24 particles in a window).
+template <int KIND>
+__global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __restrict__ planes,
+                                                          Geometry g, uint32_t r,
+                                                          float* __restrict__ md, float* __restrict__ mm,
+                                                          float* __restrict__ vel)
 {
     constexpr int Q = num_dir_of_kind(KIND);
     const uint32_t cdx = g.dim_x / (2 * r), cdy = g.dim_y / (2 * r);
@@ -524,10 +673,25 @@ hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, ui
 {
     const uint32_t n = (g.dim_x / (2 * r)) * (g.dim_y / (2 * r));
     const dim3 grid(div_up(n, 64));
+    if (r > kCoarseExactRadius) {
+        switch (kind) {
+        case kHPP: hipLaunchKernelGGL(coarse_large_kernel<kHPP>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
+        case kFHP1: hipLaunchKernelGGL(coarse_large_kernel<kFHP1>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
+        default: hipLaunchKernelGGL(coarse_large_kernel<kFHP2>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
+        }
+        return hipGetLastError();
+    }
+    // the r + 1 columns in units of at most 16, of about equal size, whole
+    // quads of addends: two stages of them take 56 KiB of LDS at most
+    const uint32_t chunks = (r + 1 + 15) / 16;
+    const uint32_t chunk = ((r + 1 + chunks - 1) / chunks + 3) & ~3u;
+    const uint32_t used = (r + chunk) / chunk;  // chunks that hold a column
+    const dim3 block(64 * (1 + kCoarseProducers));
+    const size_t lds = kind == kHPP ? 0 : (size_t)2 * kCoarseProducers * chunk * 64 * sizeof(float);
     switch (kind) {
-    case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
-    case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
-    default: hipLaunchKernelGGL(coarse_kernel<kFHP2>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
+    case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
+    case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
+    default: hipLaunchKernelGGL(coarse_kernel<kFHP2>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
     }
     return hipGetLastError();
 }

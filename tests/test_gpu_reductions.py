@@ -1,6 +1,8 @@
-"""The whole-lattice sums at the sizes where their kernels' work splits can go
-wrong: rows of one word and of more words than a workgroup has threads, more
-rows than the grid covers at once."""
+"""The whole-lattice sums and the coarse fields at the sizes where their
+kernels' work splits can go wrong: rows of one word and of more words than a
+workgroup has threads, more rows than the grid covers at once, more coarse
+cells than one workgroup's 64, radii on both sides of a unit of 16 columns and
+of the largest radius the popcounts serve, and the wrapped column."""
 import numpy as np
 import pytest
 
@@ -45,4 +47,18 @@ def test_particle_count_and_mean_velocity_are_exact(model, dx, dy, solids):
     # the sums are exact integers, then one double division and one rounding
     want = [float(np.float32(sx * ux / (840.0 * n))), float(np.float32(sy * uy / (840.0 * n)))] if n else [0.0, 0.0]
     assert lat.get_mean_velocity() == want
+    lat.close()
+
+
+@pytest.mark.parametrize("model", [0, 1, 2])
+@pytest.mark.parametrize("dx,dy,r", [
+    (2, 2, 1), (300, 130, 1), (640, 96, 7), (480, 64, 15), (512, 96, 16), (612, 70, 17), (1000, 130, 31),
+    (2112, 132, 32), (132, 200, 33), (64, 100, 32), (130, 260, 65), (2046, 2046, 1023), (2048, 2050, 1024)])
+def test_coarse_fields_bit_exact_at_unit_edges(model, dx, dy, r):
+    print(f"[coarse] model={model} {dx}x{dy} r={r}", flush=True)
+    lat, state, _ = make(model, dx, dy, r, False)
+    lat.post_process(cells=False)
+    _, _, md, mm = orc.post_process(model, dx, dy, r, state)
+    np.testing.assert_array_equal(lat.mean_density().view(np.uint32), md.view(np.uint32))
+    np.testing.assert_array_equal(lat.mean_momentum().view(np.uint32), mm.view(np.uint32))
     lat.close()
