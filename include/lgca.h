@@ -61,16 +61,17 @@ typedef struct lgca_info {
     uint32_t tile_rows;      /* rows per tile of the tiled kernel's steps_per_pass
                                 launches: lgca_set_tuning's value, else the height
                                 the timed trial of the first launches chose (0
-                                until it has)                                   */
+                                until it has); lattices that run in blocks
+                                (lgca_set_tuning) report the fixed rule's       */
     uint64_t num_cells;
     uint64_t num_coarse_cells;
     uint64_t state_bytes;    /* one state buffer: dim_y * Q * row_pitch * 4   */
     uint64_t device_bytes;   /* everything the handle holds on the GPU        */
     uint64_t step;           /* absolute step counter (hash input)            */
     uint64_t seed;
-    int32_t steps_per_pass;  /* steps per pass of lgca_step: lgca_set_tuning's
-                                value, else the one the trial chose (2, 4 or 8;
-                                -1 until it has)                                */
+    int32_t steps_per_pass;  /* steps per pass of the tiled kernel: lgca_set_tuning's
+                                value, else the one the trial chose (4 or 8; -1
+                                until it has; 4 on lattices that run in blocks) */
     uint32_t pass_pipeline;  /* 1 when lgca_set_pipeline has turned on launches
                                 of several passes                               */
 } lgca_info;
@@ -153,12 +154,13 @@ LGCA_API lgca_status lgca_step_noalloc(lgca_lattice* h, uint64_t nsteps);
 
 /* Launch shape of lgca_step: steps fused per pass over HBM (1, 2, 4 or 8; 0
  * selects the one-step kernel that keeps a 128-cell quad per thread; -1, the
- * default, lets the trial choose: 4, 8 on a lattice that fills the GPU where
- * 8-step passes are faster, or 2 where 2-step passes are faster on a lattice
- * too small to fill it) and rows per tile (0 = automatic: a timed trial
+ * default, is automatic) and rows per tile (0 = automatic: a timed trial
  * of a few shapes on the first launches, kept thereafter and restarted by this
- * call, lgca_set_forcing, new cell types or a new stream).  Results do not
- * depend on it.  No counterpart in the reference; used by the autotuner and
+ * call, lgca_set_forcing, new cell types or a new stream).  With both
+ * automatic, the trial chooses 4 or 8 steps per pass on a lattice large enough
+ * to fill the GPU with tiles; smaller ones run in blocks of rows held in
+ * registers, up to 28 steps per pass, in shapes predicted from the size (and
+ * timed by lgca_tune).  Results do not depend on it.  No counterpart in the reference; used by the autotuner and
  * benchmarks. */
 LGCA_API lgca_status lgca_set_tuning(lgca_lattice* h, int steps_per_pass, uint32_t tile_rows);
 /* Several passes of 4 or 8 steps per launch (on = 1; 0, the default, launches
@@ -183,8 +185,9 @@ LGCA_API lgca_status lgca_set_pipeline(lgca_lattice* h, int on);
  * 4-step shape for the shorter passes that finish calls of an 8-step choice.
  * Candidates include tile heights whose passes fill the GPU's wave slots
  * once or twice.  Each kernel the kept shapes use then runs once untimed, at
- * every offset of the first step within its four-step group.  The state and
- * the step do not change.  Does nothing when lgca_set_tuning fixed the rows
+ * every offset of the first step within its four-step group.  On a lattice
+ * that runs in blocks, the block shapes predicted fastest are timed instead.
+ * The state and the step do not change.  Does nothing when lgca_set_tuning fixed the rows
  * per tile or selected the one-step kernel.  No counterpart in the
  * reference; benchmarks call it before their warm-up, so that timed steps
  * run the kept shapes from the first. */

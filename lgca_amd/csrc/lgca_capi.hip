@@ -117,11 +117,14 @@ struct lgca_lattice {
     std::vector<hipEvent_t> trial_ev;  // start / end of every timed group of launches
     std::vector<uint32_t> trial_steps; // steps launched inside each group
     uint32_t trial_issued = 0;      // candidate launches queued so far
-    uint32_t trial_group = 1;       // launches per timed group
     int trial_open = -1;            // group whose end event is still to come
     LaunchShape tuned{0, 0};        // the chosen shape, th 0 while undecided
     uint32_t tuned_rem4 = 0;        // rows of the fastest 4-step candidate, for the
                                     // 4-step remainders of an 8-step choice (0: rule)
+    // Passes held in blocks (block_lattice): steps per pass (0 while undecided)
+    // and the shape for every number of steps
+    uint32_t block_k = 0;
+    BlockShape block[kBlockMaxSteps + 1];
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     // forcing controller of the viewers (lgca_controller_*)
@@ -179,6 +182,7 @@ void reset_trial(lgca_lattice* h)
     h->trial_open = -1;
     h->tuned = LaunchShape{0, 0};
     h->tuned_rem4 = 0;
+    h->block_k = 0;
 }
 
 template <typename T>
@@ -854,6 +858,7 @@ static lgca_status prepare_decisions(lgca_lattice* h, uint64_t remaining, uint32
     size_t k = (size_t)(64ull << 20) / 4 / per_step;
     if (k > 64) k = 64;
     if (k > remaining) k = (size_t)remaining;
+    else if (k > need) k -= k % need;  // whole passes: a window's rest would be drawn again
     if (k < need) k = need;
     if (h->dec_cap < k * per_step) {
         if (h->dec) {
@@ -937,20 +942,15 @@ static int steps_for_launch(int want, uint64_t left)
 // Shape of the next tiled launch (steps k, rows per tile th), and the trial
 // group whose start event goes before it and whose end event goes after it
 // (-1: none).  With automatic rows, the first launches run candidate shapes,
-// each twice in a group of consecutive launches between two events on the
-// lattice's stream: at the configured steps per pass (4 when automatic) the
-// rule's height, then 4, 8, 12, 16, 20, 24, 32 rows; with automatic steps on
-// a lattice that fills the GPU (the rule's height is 4 rows or more), 8-step
-// passes of 16 to 64 rows, which move the state through HBM half as often
-// (the 32768 x 8192 Karman lattice runs 8-step passes of 40 rows 1.4x faster
-// than 4-step passes of 16), and on a lattice the rule gives 2-row tiles,
-// 2-step passes of 2 and 4 rows, whose shorter walks suit lattices too
-// small to fill the GPU (the 2048 x 512 pipe runs 10 % faster so).  Groups are single launches, or four
-// when 2-step passes compete: then the gaps between launches must count as
-// they do in a long run, and timing each launch alone penalised the shorter
-// 2-step launches.  Once the last group has finished (queried, never waited
-// for) the fastest per step is kept, the rule's unless another beats it by
-// more than 2 %.  Results do not depend on the shape.
+// each twice between events on the lattice's stream: at the configured steps
+// per pass (4 when automatic) the rule's height, then 4, 8, 12, 16, 20, 24, 32
+// rows; with automatic steps also 8-step passes of 16 to 64 rows, which move
+// the state through HBM half as often (the 32768 x 8192 Karman lattice runs
+// 8-step passes of 40 rows 1.4x faster than 4-step passes of 16).  (Lattices
+// too small to fill the GPU with walks run in blocks when the steps are
+// automatic and make no trial.)  Once the last launch has finished (queried,
+// never waited for) the fastest per step is kept, the rule's unless another
+// beats it by more than 2 %.  Results do not depend on the shape.
 constexpr uint32_t kTrialReps = 2;
 
 // The trial's candidate shapes, the rule's own first.
@@ -1005,16 +1005,7 @@ static std::vector<LaunchShape> trial_candidates(const lgca_lattice* h)
         c.push_back(LaunchShape{ck, cth});
     };
     for (uint32_t r : {4u, 8u, 12u, 16u, 20u, 24u, 32u}) add(base_k, r);
-    if (h->tile_k == kAutoSteps && c[0].th == 2) {
-        // small lattices: their walks are short chains of dependent steps, and
-        // fewer or more steps per launch can win (the 2048 x 512 pipe keeps
-        // 2-step passes, the 256 x 256 HPP lattice 8-step ones: 0.84 against
-        // 1.14 us per step at 4)
-        add(2, 2);
-        add(2, 4);
-        add(8, 2);
-    }
-    if (h->tile_k == kAutoSteps && c[0].th >= 4) {
+    if (h->tile_k == kAutoSteps) {  // (smaller lattices run in blocks)
         for (uint32_t r : {16u, 24u, 32u, 40u, 48u, 64u}) add(8, r);
         // Tiles tall enough that a pass's waves fill the GPU's wave slots
         // once (or twice) and no more: a pass with a few waves past a whole
@@ -1045,9 +1036,6 @@ static lgca_status plan_launch(lgca_lattice* h, uint64_t left, int* k, uint32_t*
     }
     if (!h->tuned.th && h->trial.empty()) {
         h->trial = trial_candidates(h);
-        h->trial_group = 1;
-        for (const LaunchShape& s : h->trial)
-            if (s.k == 2 && base_k != 2) h->trial_group = 4;
         h->trial_issued = 0;
         h->trial_open = -1;
         const size_t groups = kTrialReps * h->trial.size();
@@ -1059,8 +1047,7 @@ static lgca_status plan_launch(lgca_lattice* h, uint64_t left, int* k, uint32_t*
         h->trial_steps.assign(groups, 0);
     }
     const uint32_t groups = kTrialReps * (uint32_t)h->trial.size();
-    const uint32_t n = h->trial_group * groups;  // candidate launches in all
-    if (!h->tuned.th && h->trial_issued == n && h->trial_open < 0) {
+    if (!h->tuned.th && h->trial_issued == groups && h->trial_open < 0) {
         const hipError_t q = hipEventQuery(h->trial_ev[2 * (groups - 1) + 1]);
         if (q != hipErrorNotReady) {
             HIPCHK(h, q);
@@ -1083,16 +1070,13 @@ static lgca_status plan_launch(lgca_lattice* h, uint64_t left, int* k, uint32_t*
         *th = *k == h->tuned.k ? h->tuned.th : other_tile_rows(h, *k);
         return LGCA_OK;
     }
-    if (h->trial_issued < n) {
-        const uint32_t e = h->trial_issued / h->trial_group, pos = h->trial_issued % h->trial_group;
+    if (h->trial_issued < groups) {
+        const uint32_t e = h->trial_issued;
         const LaunchShape& c = h->trial[e / kTrialReps];
         *k = steps_for_launch(c.k, left);
         if (*k == c.k) {
-            // a launch that the steps left force to another k inside a
-            // group is timed with it, and its steps are counted
             *th = c.th;
-            if (pos == 0) *ev_start = (int)e;
-            if (pos + 1 == h->trial_group) *ev_end = (int)e;
+            *ev_start = *ev_end = (int)e;
             ++h->trial_issued;
             return LGCA_OK;
         }
@@ -1256,8 +1240,129 @@ static const PipeCache* pipe_plan(lgca_lattice* h, int k, const TileArgs& a)
     return &h->pipes.back();
 }
 
+// Whether lgca_step runs passes in blocks (lgca_block.hpp): with automatic
+// steps and rows, on lattices that walks cannot fill the GPU with.
+static bool uses_blocks(const lgca_lattice* h)
+{
+    return h->tile_k == kAutoSteps && !h->tile_th && block_lattice(h->g);
+}
+
+// Decides the block shapes from the pass-time model: the best for every number
+// of steps, and the steps per pass with the least time per step.  lgca_info
+// reports the walk's rule for such lattices, which run no trial.
+static void plan_blocks(lgca_lattice* h)
+{
+    if (h->block_k) return;
+    const bool feat = h->mask || h->force_dir != LGCA_FORCE_NONE;
+    float best = 0.0f;
+    for (uint32_t k = 1; k <= kBlockMaxSteps; ++k) {
+        float us = -1.0f;
+        for (const BlockShape& s : block_shapes(h->g, h->kind, k)) {
+            const float t = block_pass_us(h->g, h->kind, feat, h->ncu, k, s);
+            if (t > 0.0f && (us < 0.0f || t < us)) {
+                us = t;
+                h->block[k] = s;
+            }
+        }
+        if (us < 0.0f) h->block[k] = BlockShape{0, 0, 0};
+        else if (!h->block_k || us / (float)k < best) {
+            best = us / (float)k;
+            h->block_k = k;
+        }
+    }
+    if (!h->tuned.th) h->tuned = LaunchShape{4, auto_tile_rows(h, 4)};
+}
+
+// Steps of the next block pass of `left` steps to go: whole passes, the rest
+// spread evenly over as many (an even split costs less than a short last
+// pass, whose launch and loads are the same).
+static uint32_t block_steps(const lgca_lattice* h, uint64_t left)
+{
+    const uint64_t passes = (left + h->block_k - 1) / h->block_k;
+    return (uint32_t)((left + passes - 1) / passes);
+}
+
+// A pass of k steps in blocks of shape s from the live state into the other
+// buffer.
+static hipError_t launch_block_pass(lgca_lattice* h, uint32_t k, const BlockShape& s, const uint32_t* fdec,
+                                    uint32_t t0)
+{
+    BlockArgs b{};
+    b.a = with_k(tile_args(h, s.th, fdec), (int)k);
+    b.a.t0 = t0;
+    b.k = k;
+    b.hk = block_halo(s.m, k);
+    b.nstrips = tile_segments(h->g, (int)k) ? 1 : tile_strips(h->g, (int)k);
+    return launch_block(h->kind, s, b, h->stream);
+}
+
 static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_dec = nullptr,
                                size_t ext_words = 0);
+
+// lgca_tune on a lattice that runs in blocks: the kTuneBlocks shapes with the
+// least predicted time per step, timed over passes of about 24 steps that
+// read the live state and write the other buffer (two interleaved rounds,
+// the best of each kept), and the fastest is kept.  Every kernel that calls of
+// any length use then runs once.
+constexpr size_t kTuneBlocks = 8;
+static lgca_status tune_blocks(lgca_lattice* h)
+{
+    plan_blocks(h);
+    const bool forcing = h->force_dir != LGCA_FORCE_NONE, feat = h->mask || forcing;
+    struct Candidate {
+        uint32_t k;
+        BlockShape s;
+        float us;  // per step: predicted, then measured
+    };
+    std::vector<Candidate> cand;
+    for (uint32_t k = 2; k <= kBlockMaxSteps; ++k)
+        for (const BlockShape& s : block_shapes(h->g, h->kind, k)) {
+            const float t = block_pass_us(h->g, h->kind, feat, h->ncu, k, s);
+            if (t > 0.0f) cand.push_back(Candidate{k, s, t / (float)k});
+        }
+    std::sort(cand.begin(), cand.end(), [](const Candidate& x, const Candidate& y) { return x.us < y.us; });
+    if (cand.size() > kTuneBlocks) cand.resize(kTuneBlocks);
+    const uint32_t* fdec = nullptr;
+    if (forcing) {
+        const uint32_t need = kBlockMaxSteps;
+        if (h->dec_count == 0 || h->step < h->dec_step0 || h->step + need > h->dec_step0 + h->dec_count) {
+            lgca_status st = prepare_decisions(h, 64, need);
+            if (st) return st;
+        }
+        fdec = h->dec + (size_t)(h->step - h->dec_step0) * decision_words_per_step(h);
+    }
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    hipError_t e = hipEventCreate(&ev[0]);
+    if (e == hipSuccess) e = hipEventCreate(&ev[1]);
+    const uint32_t t0 = (uint32_t)h->step;
+    for (uint32_t rep = 0; rep <= 2 && e == hipSuccess; ++rep)
+        for (Candidate& c : cand) {
+            // the first round loads the code: untimed
+            const int n = rep ? (int)((24 + c.k - 1) / c.k) : 1;
+            if (rep) e = hipEventRecord(ev[0], h->stream);
+            for (int i = 0; i < n && e == hipSuccess; ++i) e = launch_block_pass(h, c.k, c.s, fdec, t0);
+            if (!rep || e != hipSuccess) continue;
+            float ms = 0.0f;
+            if ((e = hipEventRecord(ev[1], h->stream)) != hipSuccess) break;
+            if ((e = hipEventSynchronize(ev[1])) != hipSuccess) break;
+            if ((e = hipEventElapsedTime(&ms, ev[0], ev[1])) != hipSuccess) break;
+            const float us = ms * 1e3f / (float)(n * (int)c.k);
+            c.us = rep == 1 ? us : std::min(c.us, us);
+        }
+    if (e == hipSuccess && !cand.empty()) {
+        const Candidate& best =
+            *std::min_element(cand.begin(), cand.end(), [](const Candidate& x, const Candidate& y) { return x.us < y.us; });
+        h->block_k = best.k;
+        h->block[best.k] = best.s;
+        for (uint32_t k = 1; k < best.k && e == hipSuccess; ++k)
+            if (h->block[k].m) e = launch_block_pass(h, k, h->block[k], fdec, t0);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    for (hipEvent_t v : ev)
+        if (v) (void)hipEventDestroy(v);
+    if (e != hipSuccess) return hip_fail(h, e, "lgca_tune (blocks)");
+    return LGCA_OK;
+}
 
 // The launch-shape trial of plan_launch, run at once and waited for: each
 // candidate shape is timed over groups of consecutive passes covering eight
@@ -1275,6 +1380,7 @@ extern "C" lgca_status lgca_tune(lgca_lattice* h)
     std::lock_guard<std::mutex> lk(h->mu);
     DeviceGuard dg(h->device);
     if (h->tile_k == 0 || h->tile_th) return LGCA_OK;  // no automatic choice to make
+    if (uses_blocks(h)) return tune_blocks(h);
     const std::vector<LaunchShape> cand = trial_candidates(h);
     int kmax = 1;
     for (const LaunchShape& c : cand) kmax = std::max(kmax, c.k);
@@ -1432,10 +1538,15 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
     uint64_t ext_step0 = 0;  // window held in ext_dec
     uint32_t ext_count = 0;
     uint64_t left = nsteps;
+    const bool blocks = uses_blocks(h);
+    if (blocks) plan_blocks(h);
     while (left > 0) {
         int k = 1, ev_start = -1, ev_end = -1;
         uint32_t th = 0;
-        if (h->tile_k != 0 && ext_dec) {
+        if (blocks) {
+            k = (int)block_steps(h, left);
+            if (forcing && ext_dec) k = (int)std::min<uint64_t>((uint64_t)k, ext_words / per_step);
+        } else if (h->tile_k != 0 && ext_dec) {
             const LaunchShape sh = kept_shape(h);
             k = steps_for_launch(sh.k, left);
             th = k == sh.k ? sh.th : other_tile_rows(h, k);
@@ -1447,7 +1558,7 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
         // descriptor of under 2 GiB: lattices whose forced region is larger
         // than that per pass (some 2 G forced cells at 8 steps) take fewer
         // steps per pass (a trial launch so cut is timed with its group).
-        if (forcing && h->tile_k != 0 && (uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes) {
+        if (forcing && !blocks && h->tile_k != 0 && (uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes) {
             while (k > 1 && (uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes) k /= 2;
             if ((uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes)
                 return fail(h, LGCA_ERR_INVALID_ARGUMENT, "lgca_step: the force region's decisions of one step exceed 2 GiB");
@@ -1458,7 +1569,7 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
         // times single launches, nor without allocating)
         uint64_t npass = 1;
         const PipeCache* pc = nullptr;
-        if (h->pipe && !ext_dec && h->tile_k != 0 && ev_start < 0 && ev_end < 0 && h->trial_open < 0 &&
+        if (h->pipe && !ext_dec && !blocks && h->tile_k != 0 && ev_start < 0 && ev_end < 0 && h->trial_open < 0 &&
             (k == 4 || k == 8) && left >= 2 * (uint64_t)k) {
             uint64_t np = left / (uint64_t)k;
             if (forcing) np = std::min<uint64_t>(np, pipe_window_steps(h, k) / (uint64_t)k);
@@ -1473,6 +1584,7 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
         if (forcing && ext_dec) {
             if (ext_count == 0 || h->step + k > ext_step0 + ext_count) {
                 uint64_t kw = std::min<uint64_t>(ext_words / per_step, 64);
+                if (kw < left && kw > (uint64_t)k) kw -= kw % (uint64_t)k;
                 kw = std::max<uint64_t>(std::min<uint64_t>(kw, left), (uint64_t)k);
                 lgca_status st = draw_decisions(h, ext_dec, (uint32_t)kw);
                 if (st) return st;
@@ -1521,7 +1633,9 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
             left -= span;
             continue;
         }
-        if (h->tile_k == 0) {
+        if (blocks) {
+            HIPCHK(h, launch_block_pass(h, (uint32_t)k, h->block[k], fdec, (uint32_t)h->step));
+        } else if (h->tile_k == 0) {
             StepArgs a{};
             a.g = h->g;
             a.mask = h->mask;

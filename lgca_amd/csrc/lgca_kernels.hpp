@@ -142,6 +142,36 @@ size_t tile_pipe_exch_words(const Geometry& g, int k, uint32_t nband);
 hipError_t launch_tile_pipe(int kind, int k, const TileArgs& a, const PipeArgs& p, uint32_t nwaves,
                             hipStream_t s);
 
+// Passes that hold a block of rows per workgroup (lgca_block.hpp).
+constexpr uint32_t kBlockMaxWaves = 16;
+struct BlockArgs {
+    TileArgs a;        // a.th: rows a block stores (even)
+    uint32_t k;        // steps of the pass
+    uint32_t hk;       // halo rows either side, >= k, even unless m is 1
+    uint32_t nstrips;  // x-strips (1 in segment mode)
+};
+// Shape of a pass: m rows per wave and segment, `waves` waves per workgroup, th
+// stored rows per block.
+struct BlockShape {
+    uint32_t m, waves, th;
+};
+constexpr uint32_t kBlockMaxSteps = 28;  // steps per pass the planner considers
+// Halo rows either side of a block for k-step passes.
+inline uint32_t block_halo(uint32_t m, uint32_t k) { return m == 1 ? k : (k + 1) & ~1u; }
+// LDS bytes of a workgroup.
+uint32_t block_lds_bytes(int kind, uint32_t m, uint32_t waves);
+// Predicted time (us) of a k-step pass of shape s, or a negative number where
+// the shape cannot run it.  feat: the lattice has solids or forcing.
+float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32_t k, const BlockShape& s);
+// The shapes that can run k-step passes, th chosen so that the row tiles come
+// out equal.
+std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k);
+// Whether passes of this lattice are better held in blocks than walked.
+bool block_lattice(const Geometry& g);
+hipError_t launch_block(int kind, const BlockShape& s, const BlockArgs& b, hipStream_t st);
+template <int KIND, int M>
+hipError_t launch_block_km(const BlockArgs& b, uint32_t waves, uint32_t blocks, bool ragged, int seg, hipStream_t s);
+
 // Batched ensembles.  BatchJob is a job's static descriptor (its TileArgs
 // without src/dst/t0/th/halo, which come from BatchState and WorkItem);
 // BatchState is the job's dynamic state on the device; a WorkItem is one

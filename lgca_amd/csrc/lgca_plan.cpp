@@ -196,4 +196,77 @@ size_t tile_pipe_exch_words(const Geometry& g, int k, uint32_t nband)
     return (size_t)2 * nband * 2 * (size_t)k * g.Q * g.P;
 }
 
+// ------------------------------------------------- block passes (lgca_block.hpp)
+
+uint32_t block_lds_bytes(int kind, uint32_t m, uint32_t waves)
+{
+    // two buffers of the exchanged planes, and the chirality words of every row
+    return waves * 64u * 4u * (kind == 0 ? 4u : 8u + 4u * m);
+}
+
+// Lattices whose walks the fixed rule gives 2-row tiles, about 25 wave-rows (64
+// words of a row) per SIMD.  FHP-II on
+// torus lattices, us per step in blocks / walked: 2048 x 1024 1.02 / 2.06,
+// 4400 x 2200 1.93 / 3.90, 8192 x 4096 (20,480 wave-rows) 4.05 / 4.93, 16384 x
+// 4096 (36,864) 6.85 / 6.82, 32768 x 8192 22 / 19: the larger ones fill the
+// GPU with walks, which read and compute fewer halo rows.
+bool block_lattice(const Geometry& g)
+{
+    const bool seg = tile_segments(g, 8);
+    const uint64_t wave_rows = seg ? (uint64_t)g.dim_y / (64 / g.W) : (uint64_t)g.dim_y * tile_strips(g, 8);
+    return wave_rows < 3 * 8704;
+}
+
+std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k)
+{
+    std::vector<BlockShape> out;
+    const uint32_t S = tile_segments(g, (int)k) ? 64 / g.W : 1;
+    for (uint32_t m : {1u, 2u, 4u, 6u})
+        for (uint32_t waves : {4u, 8u, 12u, 16u}) {
+            const uint32_t held = m * waves * S, halo = 2 * block_halo(m, k);
+            if (held < halo + 2 || block_lds_bytes(kind, m, waves) > 160u * 1024u) continue;
+            const uint32_t most = (held - halo) & ~1u;
+            const uint32_t tiles = (g.dim_y + most - 1) / most;
+            uint32_t th = (g.dim_y + tiles - 1) / tiles;
+            th += th & 1u;
+            out.push_back(BlockShape{m, waves, th});
+        }
+    return out;
+}
+
+// A pass takes its launch, loads and stores (3.2 us, 1.3 more where masks and
+// decisions are read), then per step a barrier with the exchange through LDS
+// and the rows' work: at least one wave's chain of m rows, at most the VALU
+// time of the rows a SIMD still works on.  Constants from passes of 5 to 28
+// steps on 256 x 256 HPP (0.12 us a step), the 2048 x 512 FHP-II pipe (0.45)
+// and 4400 x 2200 FHP-II (1.6); the best predicted shape was within 10 % of
+// the best measured one on each.
+float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32_t k, const BlockShape& s)
+{
+    const bool seg = tile_segments(g, (int)k);
+    const uint32_t S = seg ? 64 / g.W : 1, held = s.m * s.waves * S, hk = block_halo(s.m, k);
+    if (!k || !s.th || held < s.th + 2 * hk || (!seg && k > 32)) return -1.0f;
+    const uint64_t blocks = (uint64_t)((g.dim_y + s.th - 1) / s.th) * (seg ? 1 : tile_strips(g, (int)k));
+    // workgroups a CU holds: 128 registers allow 16 waves, half of them 32
+    const uint32_t waves_cu = feat && s.m > 2 ? 16 : 32;
+    const uint32_t fit = std::max(1u, std::min(waves_cu / s.waves, 160u * 1024u / block_lds_bytes(kind, s.m, s.waves)));
+    const uint32_t cus = std::max(ncu, 1u);
+    const uint32_t per_cu = (uint32_t)std::min<uint64_t>(fit, (blocks + cus - 1) / cus);
+    const uint64_t rounds = (blocks + (uint64_t)cus * per_cu - 1) / ((uint64_t)cus * per_cu);
+    float row = kind == 0 ? 0.045f : kind == 1 ? 0.090f : 0.119f;  // us of a SIMD per wave-row
+    if (feat) row *= 1.15f;
+    if (g.nb != 32) row *= 1.1f;
+    const float chain = (kind == 0 ? 0.04f : 0.16f) * (float)s.m;
+    float us = 0.0f;
+    for (uint32_t left = 0; left < k; ++left) {
+        const uint32_t rows = std::min(held, s.th + 2 * left);
+        const float work = (float)per_cu * (float)((rows + S * s.m - 1) / (S * s.m) * s.m) / 4.0f * row;
+        us += 0.08f * (float)per_cu + std::max(work, chain);
+    }
+    // reads of the held rows and writes of the stored ones, at 4.5 TB/s: half of
+    // them overlap other blocks' steps
+    const float bytes = (float)blocks * (float)((s.m * s.waves) + (s.th + S - 1) / S) * 256.0f * (float)g.Q;
+    return 3.2f + (feat ? 1.3f : 0.0f) + (float)rounds * us + 0.5f * bytes / 4.5e6f;
+}
+
 }  // namespace lgca

@@ -50,6 +50,31 @@ int tile_waves_per_cu(int kind, int k, bool ragged)
     return 0;
 }
 
+hipError_t launch_block(int kind, const BlockShape& sh, const BlockArgs& b, hipStream_t s)
+{
+    const uint32_t m = sh.m, waves = sh.waves;
+    const Geometry& g = b.a.g;
+    const bool seg = tile_segments(g, (int)b.k);
+    const uint32_t S = seg ? 64 / g.W : 1, held = waves * S * m;
+    if (!b.k || !waves || waves > kBlockMaxWaves || b.nstrips == 0) return hipErrorInvalidValue;
+    if (b.a.th < 2 || (b.a.th & 1u) || (m > 1 && (b.hk & 1u)) || b.hk < b.k || held < b.a.th + 2 * b.hk)
+        return hipErrorInvalidValue;
+    if (!seg && (b.a.halo < tile_halo(g, (int)b.k) || b.a.halo > 16 || b.k > 32)) return hipErrorInvalidValue;
+    if (b.a.fdec && (uint64_t)b.k * b.a.fdec_stride * 4u >= ((uint64_t)1 << 31)) return hipErrorInvalidValue;
+    const uint64_t blocks = (uint64_t)((g.dim_y + b.a.th - 1) / b.a.th) * b.nstrips;
+    if (blocks >= ((uint64_t)1 << 31)) return hipErrorInvalidValue;
+    const bool ragged = g.nb != 32;
+    const int seg_mode = !seg ? 0 : (g.W == 64 && !ragged) ? 2 : 1;
+#define LGCA_BLOCK_CASE(KD, MM) \
+    if (kind == KD && m == MM) return launch_block_km<KD, MM>(b, waves, (uint32_t)blocks, ragged, seg_mode, s);
+    LGCA_BLOCK_CASE(kHPP, 1) LGCA_BLOCK_CASE(kHPP, 2) LGCA_BLOCK_CASE(kHPP, 4)
+    LGCA_BLOCK_CASE(kFHP1, 1) LGCA_BLOCK_CASE(kFHP1, 2) LGCA_BLOCK_CASE(kFHP1, 4)
+    LGCA_BLOCK_CASE(kFHP2, 1) LGCA_BLOCK_CASE(kFHP2, 2) LGCA_BLOCK_CASE(kFHP2, 4)
+    LGCA_BLOCK_CASE(kHPP, 6) LGCA_BLOCK_CASE(kFHP1, 6) LGCA_BLOCK_CASE(kFHP2, 6)
+#undef LGCA_BLOCK_CASE
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_tile(int kind, int k, const TileArgs& a, hipStream_t s, const uint32_t* order, uint32_t n_order)
 {
     const bool seg = tile_segments(a.g, k);
