@@ -135,41 +135,40 @@ __global__ __launch_bounds__(256) void setup_kernel(const JobInstall* __restrict
     }
 }
 
-// Force windows of many jobs: blockIdx.y picks the job, threads stride over
-// its force region's (row, word) pairs and draw every four-step group of the
-// window for theirs.  The window starts at the job's current device step,
-// which becomes its fdec_step0.  (A thread per (group, row, word) triple paid
-// two 32-bit divisions per triple to find its row and word.)
-__global__ __launch_bounds__(256) void batch_draw_kernel(const BatchJob* __restrict__ jobs,
-                                                         BatchState* state,
-                                                         const uint32_t* __restrict__ slots,
-                                                         uint32_t nsteps)
+// Force windows of many jobs: blockIdx.y picks the job, workgroups stride over
+// its (chunk of (row, word) pairs, four-step group) items (draw_chunk).  The
+// window starts at the job's current device step, which becomes its
+// fdec_step0.
+__global__ __launch_bounds__(kDrawThreads) void batch_draw_kernel(const BatchJob* __restrict__ jobs,
+                                                                  BatchState* state,
+                                                                  const uint32_t* __restrict__ slots,
+                                                                  uint32_t nsteps)
 {
-    __shared__ uint32_t Qt[32];
+    __shared__ DrawShared sh;
     const uint32_t slot = slots[blockIdx.y];
     const BatchJob& j = jobs[slot];
-    force_table(Qt, j.force_q);
-    const uint32_t step0 = state[slot].step;
-    const uint32_t rows = j.a.fy1 - j.a.fy0, fwn = j.a.fwn;
-    const uint32_t groups = ((step0 & 3u) + nsteps + 3u) / 4u;
-    const uint64_t plane = (uint64_t)rows * fwn;
-    uint32_t* dec = const_cast<uint32_t*>(j.a.fdec);
-    for (uint64_t it = (uint64_t)blockIdx.x * 256 + threadIdx.x; it < plane; it += (uint64_t)gridDim.x * 256) {
-        uint32_t yy, ww;
-        if (plane < ((uint64_t)1 << 32)) {  // 32-bit division, the usual case
-            yy = (uint32_t)it / fwn;
-            ww = (uint32_t)it - yy * fwn;
-        } else {
-            yy = (uint32_t)(it / fwn);
-            ww = (uint32_t)(it - (uint64_t)yy * fwn);
-        }
-        const uint32_t w = j.a.fw0 + ww;
-        const uint32_t cols = force_columns(w, j.fx0, j.fx1, j.a.g.dim_x);
-        for (uint32_t g = 0; g < groups; ++g)
-            draw_group(dec + it, plane, nsteps, step0, g, w, j.a.fy0 + yy, j.a.key0, j.a.key1, Qt, cols);
+    force_table(sh.nQ, j.force_q);
+    DrawRegion r{};
+    r.dec = const_cast<uint32_t*>(j.a.fdec);
+    r.plane = (uint64_t)(j.a.fy1 - j.a.fy0) * j.a.fwn;
+    r.nsteps = nsteps;
+    r.step0 = state[slot].step;
+    r.key0 = j.a.key0;
+    r.key1 = j.a.key1;
+    r.fx0 = j.fx0;
+    r.fx1 = j.fx1;
+    r.fy0 = j.a.fy0;
+    r.fw0 = j.a.fw0;
+    r.fwn = j.a.fwn;
+    r.dim_x = j.a.g.dim_x;
+    const uint32_t groups = ((r.step0 & 3u) + nsteps + 3u) / 4u;
+    const uint64_t items = (r.plane + kDrawWords - 1) / kDrawWords * groups;
+    for (uint64_t it = blockIdx.x; it < items; it += gridDim.x) {
+        const uint64_t chunk = it / groups;
+        draw_chunk(r, chunk * kDrawWords, (uint32_t)(it - chunk * groups), sh);
     }
     // fdec_step0 is not the field the other blocks read
-    if (blockIdx.x == 0 && threadIdx.x == 0) state[slot].fdec_step0 = step0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) state[slot].fdec_step0 = r.step0;
 }
 
 }  // namespace lgca
@@ -943,11 +942,13 @@ void draw_windows(lgca_batch* b, const std::vector<int>& ks)
         const Job* j = b->slot_job[s];
         most = std::max<uint64_t>(most, (uint64_t)(j->p.fy1 - j->p.fy0) * j->p.fwn);
     }
-    const uint32_t bx = (uint32_t)std::min<uint64_t>((most + 255) / 256, 128);
+    // one workgroup per item of the largest region (9 groups when the window
+    // starts inside one), as far as 1024
+    const uint32_t bx = (uint32_t)std::min<uint64_t>((most + kDrawWords - 1) / kDrawWords * (kWindow / 4 + 1), 1024);
     // blockIdx.y covers at most 65535 jobs per launch
     for (size_t o = 0; o < slots.size(); o += 65535) {
         const uint32_t ny = (uint32_t)std::min<size_t>(65535, slots.size() - o);
-        hipLaunchKernelGGL(batch_draw_kernel, dim3(bx, ny), dim3(256), 0, b->stream, b->d_jobs, b->d_state,
+        hipLaunchKernelGGL(batch_draw_kernel, dim3(bx, ny), dim3(kDrawThreads), 0, b->stream, b->d_jobs, b->d_state,
                            b->d_draw + o, kWindow);
         hipchk(hipGetLastError(), "batch_draw_kernel");
     }

@@ -253,61 +253,36 @@ __device__ __forceinline__ uint32_t fill_word(uint32_t w, uint32_t y, uint32_t d
 // philox({w, y, G, 1})[step & 3] (one call serves the group).  Further
 // uniforms, needed only after a fire, are the group's extras
 // E_e = philox({w, y, G, 5 + 4 (e >> 2)})[e & 3], e = 0, 1, ..., shared by the
-// group's steps in step order: `used` counts the extras the group's earlier
-// steps took and `ext` holds block used >> 2 (the caller loads block 0 when
-// any step of the group fires).  Qt[k] = Q_{k+1}, where Q_1 = q = 2^32 - thr
-// and Q_{k+1} = floor(Q_k q / 2^32) (force_table); the first of the next n
-// cells to fire is the smallest m < n with u + Q_{m+1} < 2^32, and there is
-// none when u + Q_n >= 2^32.
-__device__ __forceinline__ bool force_fires(uint32_t u0, const uint32_t* Qt)
-{
-    return (uint64_t)u0 + Qt[31] < ((uint64_t)1 << 32);
-}
+// group's steps in step order, each step starting after the extras that the
+// group's earlier steps took.  With Q_1 = q = 2^32 - thr and
+// Q_{k+1} = floor(Q_k q / 2^32), the first of the next n cells to fire is the
+// smallest m < n with u + Q_{m+1} < 2^32, and there is none when
+// u + Q_n >= 2^32.  The table holds the complements ~Q_1..~Q_32 (force_table):
+// u + Q >= 2^32 exactly when u > ~Q.
+__device__ __forceinline__ bool force_fires(uint32_t u0, const uint32_t* nQ) { return u0 <= nQ[31]; }
 
 // Offset of the first fire among 32 cells for uniform u, 32 when none fires:
-// the number of k in [0, 32) with u + Qt[k] >= 2^32, a prefix because Qt
-// decreases.  Five fixed lifting steps find it up to 31, and Qt[31] adds the
-// last; no branches, so the lanes of a wave stay in step.  For the next n
-// cells of a word the first fire is this offset when it is < n, else there is
-// none (the prefix covers the first n cells).
-__device__ __forceinline__ uint32_t force_first(uint32_t u, const uint32_t* Qt)
+// the number of k in [0, 32) with u > nQ[k], a prefix because Q decreases.
+// Five fixed lifting steps find it up to 31, and nQ[31] adds the last; no
+// branches, so the lanes of a wave stay in step.  For the next n cells of a
+// word the first fire is this offset when it is < n, else there is none (the
+// prefix covers the first n cells).
+__device__ __forceinline__ uint32_t force_first(uint32_t u, const uint32_t* nQ)
 {
-    constexpr uint64_t kTwo32 = (uint64_t)1 << 32;
     uint32_t m = 0;
 #pragma unroll
-    for (uint32_t step = 16; step; step >>= 1)
-        m += ((uint64_t)u + Qt[m + step - 1] >= kTwo32) ? step : 0u;
-    return m + (((uint64_t)u + Qt[31] >= kTwo32) ? 1u : 0u);
+    for (uint32_t step = 16; step; step >>= 1) m += u > nQ[m + step - 1] ? step : 0u;
+    return m + (u > nQ[31] ? 1u : 0u);
 }
 
-__device__ __forceinline__ uint32_t force_word(uint32_t u0, uint32_t w, uint32_t y, uint32_t group,
-                                               uint32_t key0, uint32_t key1, const uint32_t* Qt,
-                                               uint32_t& used, U4& ext)
-{
-    if (!force_fires(u0, Qt)) return 0;  // no fire among all 32 cells
-    uint32_t word = 0, pos = 0, u = u0;
-    for (;;) {
-        const uint32_t m = force_first(u, Qt);
-        if (m >= 32 - pos) break;  // no fire among the word's remaining cells
-        word |= 1u << (pos + m);
-        pos += m + 1;
-        if (pos == 32) break;
-        if ((used & 3u) == 0 && used != 0) ext = philox4x32_10(w, y, group, 5u + used, key0, key1);
-        const uint32_t i = used & 3u;
-        u = i == 0 ? ext.x : (i == 1 ? ext.y : (i == 2 ? ext.z : ext.w));
-        ++used;
-    }
-    return word;
-}
-
-// Fills Qt[0..31] = Q_1..Q_32 for q = 2^32 - thr (exact integer steps, the
+// Fills nQ[0..31] = ~Q_1..~Q_32 for q = 2^32 - thr (exact integer steps, the
 // same on every platform) and makes it visible to the whole workgroup.
-__device__ __forceinline__ void force_table(uint32_t* Qt, uint32_t q)
+__device__ __forceinline__ void force_table(uint32_t* nQ, uint32_t q)
 {
     if (threadIdx.x == 0) {
         uint32_t Qk = q;
         for (int k = 0; k < 32; ++k) {
-            Qt[k] = Qk;
+            nQ[k] = ~Qk;
             Qk = __umulhi(Qk, q);
         }
     }
@@ -325,38 +300,126 @@ __device__ __forceinline__ uint32_t force_columns(uint32_t w, uint32_t fx0, uint
     return (nbits == 32 ? 0xFFFFFFFFu : ((1u << nbits) - 1u)) << sh;
 }
 
-// One thread's share of a force draw: the decision words of word w of row y
-// for the steps of group `group` (steps sharing (step & ~3), counted from
-// step0 & ~3) that fall in [step0, step0 + nsteps), stored at dec[k * plane]
-// for window index k; cols masks the forced columns of the word.  Steps of
-// the group before step0 are walked too: they take extras before the later
-// steps do.
-__device__ __forceinline__ void draw_group(uint32_t* dec, uint64_t plane, uint32_t nsteps,
-                                           uint32_t step0, uint32_t group, uint32_t w, uint32_t y,
-                                           uint32_t key0, uint32_t key1, const uint32_t* Qt,
-                                           uint32_t cols)
+// Force draws.  A workgroup of kDrawThreads threads draws the decision words of
+// kDrawWords consecutive (row, word) pairs of a force region for one group of
+// four steps.  At p <= 5e-3 a word fires in at most 15 % of its steps, but of
+// the 64 words of a wave one almost always does, so a thread per word had
+// every wave make the second Philox call and walk every step for a few lanes:
+// about 500 instructions a wave.  So the first pass only makes the first call,
+// stores zeros for the words that never fire in the group and lists the
+// others in LDS; the second takes the listed words, 64 to a wave again, each
+// lane stepping through its own fires, one search of the table each.
+// 6000 x 3000 cells forced at p = 5e-3, 28 steps: 59 -> 32 us (searching the
+// table by a logarithm and two reads: 41 for 39 at the time; results through
+// LDS to whole-line stores: 42).
+constexpr uint32_t kDrawThreads = 256, kDrawWords = 1024;
+struct DrawShared {
+    uint32_t nQ[32];
+    uint32_t count;
+    uint32_t idx[kDrawWords];   // of the region's (row, word) pairs, from the chunk's first
+    uint32_t u[4][kDrawWords];  // the group's first uniforms
+};
+struct DrawRegion {
+    uint32_t* dec;              // decision word of step step0 + k and pair i at dec[k * plane + i]
+    uint64_t plane;             // (row, word) pairs
+    uint32_t nsteps, step0, key0, key1;
+    uint32_t fx0, fx1, fy0, fw0, fwn, dim_x;
+};
+
+// force_table has filled sh.nQ.  Group `group` is counted from step0 & ~3;
+// steps of the group before step0 are walked too: they take extras before
+// the later steps do.
+__device__ __forceinline__ void draw_chunk(const DrawRegion& a, uint64_t first_pair, uint32_t group, DrawShared& sh)
 {
-    const uint32_t first = step0 & 3u;
-    const uint32_t G = ((step0 & ~3u) + 4u * group) >> 2;  // of the group's steps mod 2^32
-    uint32_t u[4] = {0, 0, 0, 0};
-    U4 ext{0, 0, 0, 0};
-    if (cols) {
-        const U4 r = philox4x32_10(w, y, G, 1u, key0, key1);
-        u[0] = r.x; u[1] = r.y; u[2] = r.z; u[3] = r.w;
-        // one call for the first four extras of the whole group, made up front
-        // so that a wave whose lanes fire at different steps makes it once
-        if (force_fires(u[0], Qt) || force_fires(u[1], Qt) || force_fires(u[2], Qt) ||
-            force_fires(u[3], Qt))
-            ext = philox4x32_10(w, y, G, 5u, key0, key1);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t skip = a.step0 & 3u;
+    const uint32_t G = ((a.step0 & ~3u) + 4u * group) >> 2;  // of the group's steps mod 2^32
+    const uint32_t i0 = group == 0 ? skip : 0u;                   // the group's steps in the window
+    const uint32_t i1 = min(4u, skip + a.nsteps - 4u * group);
+    // (i0 may lie past the first steps, so the pointer arithmetic is signed)
+    uint32_t* dec = a.dec + (int64_t)(4 * (int64_t)group - (int64_t)skip) * (int64_t)a.plane;
+    const uint32_t magic = 0xFFFFFFFFu / a.fwn;  // at * magic >> 32 is at / fwn or one less
+    auto pair = [&](uint64_t at, uint32_t& w, uint32_t& y) {
+        if (a.plane < ((uint64_t)1 << 32)) {  // the usual case
+            y = __umulhi((uint32_t)at, magic);
+            w = (uint32_t)at - y * a.fwn;
+            if (w >= a.fwn) {
+                w -= a.fwn;
+                ++y;
+            }
+        } else {
+            y = (uint32_t)(at / a.fwn);
+            w = (uint32_t)(at - (uint64_t)y * a.fwn);
+        }
+        w += a.fw0;
+        y += a.fy0;
+    };
+    if (tid == 0) sh.count = 0;
+    __syncthreads();
+    for (uint32_t k = 0; k < kDrawWords; k += kDrawThreads) {
+        const uint64_t at = first_pair + k + tid;
+        bool fires = false;
+        U4 r{0, 0, 0, 0};
+        if (at < a.plane) {
+            uint32_t w, y;
+            pair(at, w, y);
+            r = philox4x32_10(w, y, G, 1u, a.key0, a.key1);
+            fires = force_fires(min(min(r.x, r.y), min(r.z, r.w)), sh.nQ);
+            if (!fires)
+                for (uint32_t i = i0; i < i1; ++i) dec[i * a.plane + at] = 0u;
+        }
+        const unsigned long long any = __ballot(fires);
+        uint32_t base = 0;
+        if (lane == 0 && any) base = atomicAdd(&sh.count, (uint32_t)__popcll(any));
+        base = __builtin_amdgcn_readfirstlane(base);
+        if (fires) {
+            const uint32_t e = base + (uint32_t)__popcll(any & ((1ull << lane) - 1ull));
+            sh.idx[e] = k + tid;
+            sh.u[0][e] = r.x;
+            sh.u[1][e] = r.y;
+            sh.u[2][e] = r.z;
+            sh.u[3][e] = r.w;
+        }
     }
-    uint32_t used = 0;
+    __syncthreads();
+    const uint32_t n = sh.count;
+    for (uint32_t e = tid; e < n; e += kDrawThreads) {
+        const uint64_t at = first_pair + sh.idx[e];
+        uint32_t w, y, left = 0;  // left: steps still to walk, those that fire
+        pair(at, w, y);
+        const uint32_t cols = force_columns(w, a.fx0, a.fx1, a.dim_x);
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t k = 4u * group + i - first;  // window index of step 4G + i
-        if (4u * group + i >= first + nsteps) break;
-        const uint32_t word = cols ? (force_word(u[i], w, y, G, key0, key1, Qt, used, ext) & cols) : 0u;
-        if (4u * group + i >= first) dec[(size_t)k * plane] = word;
+        for (uint32_t i = 0; i < 4; ++i) {
+            const bool f = force_fires(sh.u[i][e], sh.nQ);
+            left |= f ? 1u << i : 0u;
+            if (!f && i >= i0 && i < i1) dec[i * a.plane + at] = 0u;
+        }
+        U4 ext = philox4x32_10(w, y, G, 5u, a.key0, a.key1);
+        uint32_t used = 0, pos = 0, word = 0, i = __ffs(left) - 1;
+        uint32_t u = sh.u[i][e];
+        for (;;) {
+            // u fires among the step's remaining 32 - pos cells
+            const uint32_t m = force_first(u, sh.nQ);
+            word |= 1u << (pos + m);
+            pos += m + 1u;
+            bool again = false;
+            if (pos < 32u) {
+                if ((used & 3u) == 0 && used) ext = philox4x32_10(w, y, G, 5u + used, a.key0, a.key1);
+                const uint32_t j = used & 3u;
+                u = j == 0 ? ext.x : (j == 1 ? ext.y : (j == 2 ? ext.z : ext.w));
+                ++used;
+                again = u <= sh.nQ[31u - pos];
+            }
+            if (again) continue;
+            if (i >= i0 && i < i1) dec[i * a.plane + at] = word & cols;
+            left &= left - 1u;
+            if (!left) break;
+            i = __ffs(left) - 1;
+            u = sh.u[i][e];
+            pos = word = 0;
+        }
     }
+    __syncthreads();  // the list is free for the next chunk
 }
 
 }  // namespace lgca

@@ -202,37 +202,36 @@ hipError_t launch_step(int kind, const StepArgs& a, hipStream_t s)
 
 // ------------------------------------------------------------ force draws
 // Decision words of steps [step0, step0 + nsteps) of the forced rows and
-// words: bit b of word (step, y, w) forces cell 32w + b (see force_word).
-// A thread owns one word of one row for one group of four steps that share
-// the word's first Philox call; groups follow step >> 2 (steps mod 2^32).
+// words: bit b of word (step, y, w) forces cell 32w + b (see draw_chunk).
+// Groups of four steps follow step >> 2 (steps mod 2^32).
 
-__global__ __launch_bounds__(256) void force_draw_kernel(ForceDrawArgs a)
+__global__ __launch_bounds__(kDrawThreads) void force_draw_kernel(ForceDrawArgs a)
 {
-    // grid: x over the (row, word) pairs of the force region, y over groups
-    __shared__ uint32_t Qt[32];
-    force_table(Qt, a.q);
-    const uint64_t plane = (uint64_t)(a.fy1 - a.fy0) * a.fwn;
-    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= plane) return;
-    uint32_t yy, ww;
-    if (plane < ((uint64_t)1 << 32)) {  // 32-bit division, the usual case
-        yy = (uint32_t)idx / a.fwn;
-        ww = (uint32_t)idx - yy * a.fwn;
-    } else {
-        yy = (uint32_t)(idx / a.fwn);
-        ww = (uint32_t)(idx - (uint64_t)yy * a.fwn);
-    }
-    const uint32_t w = a.fw0 + ww;
-    draw_group(a.dec + idx, plane, a.nsteps, a.step0, blockIdx.y, w, a.fy0 + yy, a.key0, a.key1, Qt,
-               force_columns(w, a.fx0, a.fx1, a.dim_x));
+    // grid: x over chunks of (row, word) pairs of the force region, y over groups
+    __shared__ DrawShared sh;
+    force_table(sh.nQ, a.q);
+    DrawRegion r{};
+    r.dec = a.dec;
+    r.plane = (uint64_t)(a.fy1 - a.fy0) * a.fwn;
+    r.nsteps = a.nsteps;
+    r.step0 = a.step0;
+    r.key0 = a.key0;
+    r.key1 = a.key1;
+    r.fx0 = a.fx0;
+    r.fx1 = a.fx1;
+    r.fy0 = a.fy0;
+    r.fw0 = a.fw0;
+    r.fwn = a.fwn;
+    r.dim_x = a.dim_x;
+    draw_chunk(r, (uint64_t)blockIdx.x * kDrawWords, blockIdx.y, sh);
 }
 
 hipError_t launch_force_draw(const ForceDrawArgs& a, hipStream_t s)
 {
     const uint32_t groups = ((a.step0 & 3u) + a.nsteps + 3u) / 4u;
     const uint64_t n = (uint64_t)(a.fy1 - a.fy0) * a.fwn;
-    if ((n + 255) / 256 >= ((uint64_t)1 << 31) || groups > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(force_draw_kernel, dim3(div_up(n, 256), groups), dim3(256), 0, s, a);
+    if ((n + kDrawWords - 1) / kDrawWords >= ((uint64_t)1 << 31) || groups > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(force_draw_kernel, dim3(div_up(n, kDrawWords), groups), dim3(kDrawThreads), 0, s, a);
     return hipGetLastError();
 }
 

@@ -240,7 +240,7 @@ inline uint64_t hash_threshold(double p)
 }
 
 // First-fire parameter of the per-cell force for threshold thr in [1, 2^32]:
-// q = 2^32 - thr (see force_word in lgca_dev.hpp).
+// q = 2^32 - thr (see force_first in lgca_dev.hpp).
 inline uint32_t force_q(uint64_t thr) { return (uint32_t)(((uint64_t)1 << 32) - thr); }
 
 hipError_t launch_pack(const uint8_t* state, uint32_t* planes, const Geometry& g,
