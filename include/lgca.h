@@ -272,7 +272,7 @@ LGCA_API lgca_status lgca_load_checkpoint(lgca_lattice** out, const char* path, 
  * time; the worker admits them in order while their device memory fits the
  * batch's HBM budget (and their cells the active-cell cap), and advances
  * all admitted jobs together, a few steps per round, in one kernel launch per
- * (model, steps per pass, ragged width) class.  A finished job's outputs stay
+ * (steps per pass, ragged width) class.  A finished job's outputs stay
  * on the GPU until released.  All batch entry points are thread-safe.
  * ---------------------------------------------------------------------- */
 typedef struct lgca_batch lgca_batch;
@@ -317,7 +317,8 @@ typedef struct lgca_batch_stats {
     uint64_t bytes_in_use;     /* device bytes of admitted, unreleased jobs            */
     uint64_t arena_bytes;      /* device memory reserved by the batch                  */
     int32_t steps_per_pass;    /* current tuning                                       */
-    uint32_t wave_target;      /* waves per round the tile height aims at              */
+    uint32_t wave_target;      /* waves per round the tile height aims at; in rounds of
+                                  blocks, waves per workgroup (at most 16)             */
     uint64_t tunings;          /* autotuner decisions taken                            */
 } lgca_batch_stats;
 

@@ -22,8 +22,9 @@ SOURCES = ["lgca_kernels.hip", "lgca_tile.hip", "lgca_capi.hip", "lgca_batch.hip
 # the single-lattice kernels and once per steps per pass of the batch kernel
 # (kind -1), which lets the template-heavy tiled kernels compile in parallel
 TILE_INST = [(kind, k) for k in (8, 4, 2, 1) for kind in (-1, 0, 1, 2)]
-# lgca_block_inst.hip once per (model kind, rows per wave)
-BLOCK_INST = [(kind, m) for m in (6, 4, 2, 1) for kind in (2, 1, 0)]
+# lgca_block_inst.hip once per (model kind, rows per wave); kind -1 is the
+# batch kernel
+BLOCK_INST = [(-1, 4), (-1, 2)] + [(kind, m) for m in (6, 4, 2, 1) for kind in (2, 1, 0)]
 ARCH = os.environ.get("LGCA_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
@@ -59,7 +60,7 @@ def _jobs():
     jobs = [(f"lgca_tile_inst.hip", [f"-DLGCA_INST_KIND={kind}", f"-DLGCA_INST_K={k}"],
              f"lgca_tile_{'batch' if kind < 0 else f'm{kind}'}_k{k}") for kind, k in TILE_INST]
     jobs += [("lgca_block_inst.hip", [f"-DLGCA_INST_KIND={kind}", f"-DLGCA_INST_M={m}"],
-              f"lgca_block_m{kind}_r{m}") for kind, m in BLOCK_INST]
+              f"lgca_block_{'batch' if kind < 0 else f'm{kind}'}_r{m}") for kind, m in BLOCK_INST]
     jobs += [(src, [], os.path.splitext(src)[0]) for src in SOURCES]
     return jobs
 

@@ -19,11 +19,17 @@
 // passed their completion event.  Client calls touch only host-side tables,
 // except lgca_batch_result, which copies on a stream of its own.
 //
-// Tiles: every job in a round uses the same tile height th, chosen so the
-// round has about `wave_target` waves; the autotuner times rounds with each
-// (steps per pass, wave target) candidate on the live mix and keeps the
-// fastest per site update, and tunes again when the mix has changed by 2x.
-// Results never depend on the tuning: the hash is keyed by (seed, step, cell).
+// Rounds are walks (lgca_tile.hpp) or blocks (lgca_block.hpp).  In a round of
+// walks every job uses the same tile height th, chosen so the round has about
+// `wave_target` waves; in a round of blocks every workgroup has the same rows
+// per wave and waves.  Mixes too small to fill the GPU with walks take the
+// block shape predicted fastest for the jobs still running; on larger ones the
+// autotuner times rounds of the best predicted blocks and of a few walks on
+// the live mix and keeps the fastest per site update, and tunes again when the
+// mix has changed by 2x.  16 FHP-II ensemble jobs of 1000-4000 steps: 24 ms in
+// walks, 9 ms with blocks; 120 serving jobs 380 and 300 ms; 512 ensemble jobs
+// 280 and 273 ms.
+// Results never depend on the shape: the hash is keyed by (seed, step, cell).
 #include "lgca.h"
 
 #include "lgca_dev.hpp"
@@ -359,15 +365,19 @@ struct Arena {
 };
 
 struct ClassRange {
-    int k;
+    int k;           // steps (0 in a round of blocks, whose items hold them)
     bool ragged;
     uint32_t offset, count;
     uint32_t heavy;  // leading items that can take the general walk
 };
 
+// Launch shape of a round: k steps per pass; walks (m 0) with tiles tall enough
+// for about `waves` waves, or blocks of m rows per wave and `waves` waves per
+// workgroup.
 struct Candidate {
     int k;
     uint32_t waves;
+    uint32_t m = 0;
 };
 
 }  // namespace
@@ -430,8 +440,8 @@ struct lgca_batch {
     std::vector<Job*> finishing;        // post-processed, waiting for their event
 
     // autotuner (worker-private)
-    int k_cur = 4;
-    uint32_t waves_cur = 4096;
+    Candidate cur{4, 4096, 0};
+    uint64_t mix_key = 0;               // jobs the block shape was predicted for
     std::vector<Candidate> cands;
     size_t cand_i = 0;
     int cand_rounds = 0;
@@ -807,6 +817,74 @@ uint32_t tile_rows_for(uint64_t wave_rows_total, uint32_t waves)
     return (uint32_t)th;
 }
 
+// Blocks of a job's k-step round: rows per block and blocks.
+struct JobBlocks {
+    uint32_t th, tiles, strips;
+};
+JobBlocks job_blocks(const Geometry& g, const Candidate& c, int k)
+{
+    const bool seg = tile_segments(g, k);
+    const uint32_t held = c.m * c.waves * (seg ? 64 / g.W : 1);
+    const uint32_t most = (held - 2 * block_halo(c.m, (uint32_t)k)) & ~1u;
+    JobBlocks b;
+    b.tiles = (g.dim_y + most - 1) / most;
+    b.th = (g.dim_y + b.tiles - 1) / b.tiles;
+    b.th += b.th & 1u;
+    b.tiles = (g.dim_y + b.th - 1) / b.th;
+    b.strips = seg ? 1 : tile_strips(g, k);
+    return b;
+}
+
+// Predicted time (us) of a round of the running jobs in blocks of shape c:
+// block_pass_us over a mix, whose blocks share the CUs.
+float mix_round_us(const lgca_batch* b, const Candidate& c)
+{
+    const uint32_t fit = std::max(1u, std::min(16u / c.waves, 160u * 1024u / block_lds_bytes(kFHP2, c.m, c.waves)));
+    float work = 0.0f, wait = 0.0f, most = 0.0f, bytes = 0.0f;
+    for (const Job* j : b->active) {
+        const Geometry& g = j->p.g;
+        const int k = (int)std::min<uint64_t>((uint64_t)c.k, j->d.steps - j->step);
+        const JobBlocks n = job_blocks(g, c, k);
+        const uint32_t S = tile_segments(g, k) ? 64 / g.W : 1, group = S * c.m, held = group * c.waves;
+        float row = j->p.kind == kHPP ? 0.045f : j->p.kind == kFHP1 ? 0.090f : 0.119f;
+        if (j->p.has_mask || j->p.forced) row *= 1.1f;
+        const float chain = (j->p.kind == kHPP ? 0.04f : 0.16f) * (float)c.m;
+        float bw = 0.0f, bl = 0.0f;  // one block's VALU time, and its time alone on a CU
+        for (int left = 0; left < k; ++left) {
+            const uint32_t rows = std::min(held, n.th + 2 * (uint32_t)left);
+            const float w = (float)((rows + group - 1) / group * c.m) / 4.0f * row;
+            bw += w;
+            bl += 0.08f + std::max(w, chain);
+        }
+        const float blocks = (float)n.tiles * (float)n.strips;
+        work += blocks * bw;
+        wait += blocks * (bl - bw + 1.5f);
+        most = std::max(most, bl);
+        bytes += blocks * (float)(held + n.th) / (float)S * 256.0f * (float)g.Q;
+    }
+    return 4.5f + std::max(most, work / 256.0f + wait / (256.0f * (float)fit)) + 0.5f * bytes / 4.5e6f;
+}
+
+// The block shapes a round may take, those with the least predicted time per
+// step first.  Steps are multiples of 4, so that a round of walks may follow,
+// and divide the force window when a job is forced.
+std::vector<Candidate> block_candidates(const lgca_batch* b)
+{
+    std::vector<std::pair<float, Candidate>> v;
+    const bool forced = std::any_of(b->active.begin(), b->active.end(), [](const Job* j) { return j->p.forced; });
+    for (int k = 4; k <= 24; k += 4)
+        for (uint32_t m : {2u, 4u})
+            for (uint32_t waves : {4u, 8u, 12u, 16u}) {
+                const Candidate c{k, waves, m};
+                if (m * waves < 2 * (uint32_t)k + 2 || (forced && kWindow % (uint32_t)k)) continue;
+                v.emplace_back(mix_round_us(b, c) / (float)k, c);
+            }
+    std::sort(v.begin(), v.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+    std::vector<Candidate> out;
+    for (const auto& x : v) out.push_back(x.second);
+    return out;
+}
+
 // Whether a work item reading rows [a, b) of a job (on the torus) can take
 // the general walk: rows with walls, the disc, given cell types or forcing.
 // It only orders the items of a class (those first, so that waves that run
@@ -837,7 +915,7 @@ bool rows_heavy(const Job* j, int64_t a, int64_t b)
 }
 
 // Builds this round's work items if the mix changed.
-void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th)
+void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th, const Candidate& shape)
 {
     const size_t n = b->active.size();
     b->sig.clear();
@@ -846,6 +924,7 @@ void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th)
     // later job of another size: the signature names jobs by their ids, never
     // reused, so that a new job in an old slot always rebuilds the items.
     b->sig.push_back(th);
+    b->sig.push_back(((uint64_t)shape.m << 32) | (shape.m ? shape.waves : 0u));
     for (size_t i = 0; i < n; ++i) {
         b->sig.push_back(b->active[i]->id);
         b->sig.push_back(((uint64_t)b->active[i]->slot << 8) | (uint64_t)ks[i]);
@@ -861,6 +940,21 @@ void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th)
         const int k = ks[i];
         const bool seg = tile_segments(g, k);
         const uint32_t halo = seg ? 0u : tile_halo(g, k);
+        if (shape.m) {
+            // a launch for every k: the items hold their job's
+            const JobBlocks n = job_blocks(g, shape, k);
+            const uint64_t key = g.nb != 32 ? 1u : 0u;
+            std::vector<WorkItem>& vh = cls[key];
+            std::vector<WorkItem>& vl = light[key];
+            const uint32_t bits = block_shape_bits(n.th, halo, (uint32_t)k, seg);
+            for (uint32_t t = 0; t < n.tiles; ++t) {
+                const int64_t y0 = (int64_t)t * n.th, rows = std::min<int64_t>(n.th, g.dim_y - y0);
+                std::vector<WorkItem>& v = rows_heavy(j, y0 - k, y0 + rows + k) ? vh : vl;
+                for (uint32_t st = 0; st < n.strips; ++st)
+                    v.push_back(WorkItem{(uint32_t)j->slot, st, t, bits, n.tiles * n.strips});
+            }
+            continue;
+        }
         const uint32_t jth = std::min<uint32_t>(th, g.dim_y + (g.dim_y & 1u));
         const uint32_t tiles = (g.dim_y + jth - 1) / jth;
         const uint64_t key = ((uint64_t)k << 8) | (g.nb != 32 ? 1u : 0u);
@@ -960,11 +1054,20 @@ void start_tuning(lgca_batch* b, int user_k, uint32_t user_waves, uint64_t wr)
     b->cands.clear();
     const int ks[2] = {4, 8};
     const uint32_t ws[4] = {2048, 4096, 8192, 16384};
-    for (int k : ks) {
-        if (user_k && k != user_k) continue;
-        for (uint32_t w : ws) {
-            if (user_waves && w != user_waves) continue;
-            b->cands.push_back(Candidate{k, w});
+    if (!user_k && !user_waves) {
+        // the blocks predicted fastest against the walks that win on mixes
+        // which fill the GPU
+        const std::vector<Candidate> blocks = block_candidates(b);
+        for (size_t i = 0; i < blocks.size() && i < 3; ++i) b->cands.push_back(blocks[i]);
+        for (int k : ks)
+            for (uint32_t w : {2048u, 4096u}) b->cands.push_back(Candidate{k, w});
+    } else {
+        for (int k : ks) {
+            if (user_k && k != user_k) continue;
+            for (uint32_t w : ws) {
+                if (user_waves && w != user_waves) continue;
+                b->cands.push_back(Candidate{k, w});
+            }
         }
     }
     if (user_k && b->cands.empty())
@@ -974,10 +1077,7 @@ void start_tuning(lgca_batch* b, int user_k, uint32_t user_waves, uint64_t wr)
     b->tuned_wave_rows = wr;
     b->rounds_since_tune = 0;
     if (b->cands.size() <= 1) {
-        if (!b->cands.empty()) {
-            b->k_cur = b->cands[0].k;
-            b->waves_cur = b->cands[0].waves;
-        }
+        if (!b->cands.empty()) b->cur = b->cands[0];
         b->tuning = false;
         return;
     }
@@ -988,8 +1088,7 @@ void start_tuning(lgca_batch* b, int user_k, uint32_t user_waves, uint64_t wr)
     b->tune_ev.assign(2 * b->cands.size(), nullptr);
     for (auto& e : b->tune_ev) hipchk(hipEventCreate(&e), "hipEventCreate");
     b->tune_su.assign(b->cands.size(), 0);
-    b->k_cur = b->cands[0].k;
-    b->waves_cur = b->cands[0].waves;
+    b->cur = b->cands[0];
 }
 
 // Picks the fastest candidate once the GPU has passed the last timing event.
@@ -1006,8 +1105,7 @@ void evaluate_tuning(lgca_batch* b, bool block)
         const double rate = ms > 0.0f ? (double)b->tune_su[c] / ms : 0.0;
         if (rate > best) {
             best = rate;
-            b->k_cur = b->cands[c].k;
-            b->waves_cur = b->cands[c].waves;
+            b->cur = b->cands[c];
         }
     }
     b->evaluating = false;
@@ -1031,10 +1129,26 @@ void run_round(lgca_batch* b)
     // A mix that has doubled since the last tuning (jobs still arriving) is
     // tuned again at once, a shrinking one after 64 rounds; a tuning under way
     // restarts only when the mix has grown 4x since it began.
-    if (!b->tuning && !b->evaluating) {
+    // A mix too small to fill the GPU with walks takes the block shape predicted
+    // fastest for the jobs still running, untimed: its rounds are short and its
+    // jobs keep ending.
+    if (!user_k && !user_waves && wr_now < 3 * 8704) {
+        if (b->tuning || b->evaluating) {
+            b->tuning = b->evaluating = false;
+            b->mix_key = 0;
+        }
+        uint64_t key = b->active.size();
+        for (const Job* j : b->active) key = key * 0x100000001B3ull ^ j->id;
+        if (key != b->mix_key) {
+            b->mix_key = key;
+            b->cur = block_candidates(b).front();
+        }
+        b->tuned_wave_rows = 0;  // a mix that grows past this is tuned at once
+    } else if (!b->tuning && !b->evaluating) {
         const bool grown = b->tuned_wave_rows != 0 && wr_now > 2 * b->tuned_wave_rows;
         const bool shrunk = b->rounds_since_tune >= 64 && wr_now * 2 < b->tuned_wave_rows;
         if (retune || b->tuned_wave_rows == 0 || shrunk || grown) start_tuning(b, user_k, user_waves, wr_now);
+        b->mix_key = 0;
     } else if (retune || wr_now > 4 * b->tuned_wave_rows) {
         start_tuning(b, user_k, user_waves, wr_now);
     }
@@ -1045,11 +1159,14 @@ void run_round(lgca_batch* b)
     uint64_t su = 0;
     for (size_t i = 0; i < n; ++i) {
         const Job* j = b->active[i];
-        ks[i] = pick_k(b->k_cur, j->d.steps - j->step, j->step);
+        // (blocks may start a pass at any step)
+        ks[i] = b->cur.m ? (int)std::min<uint64_t>((uint64_t)b->cur.k, j->d.steps - j->step)
+                         : pick_k(b->cur.k, j->d.steps - j->step, j->step);
         su += (uint64_t)j->d.dim_x * j->d.dim_y * (uint64_t)ks[i];
     }
-    const uint32_t th = tile_rows_for(wave_rows(b, b->k_cur), b->waves_cur);
-    build_round(b, ks, th);
+    const uint32_t th = b->cur.m ? 0 : tile_rows_for(wave_rows(b, b->cur.k), b->cur.waves);
+    const Candidate shape = b->cur;
+    build_round(b, ks, th, shape);
     draw_windows(b, ks);
 
     if (b->tuning && b->cand_rounds == 0)
@@ -1059,9 +1176,14 @@ void run_round(lgca_batch* b)
     // only jobs at their last steps add a short one.
     uint64_t nl = 0;
     for (const ClassRange& c : b->classes) {
-        hipchk(launch_tile_batch(c.k, c.ragged, b->d_jobs, b->d_state, b->d_items[b->items_buf] + c.offset,
-                                 c.count, c.heavy, b->stream),
-               "tile_batch_kernel");
+        const WorkItem* items = b->d_items[b->items_buf] + c.offset;
+        if (shape.m)
+            hipchk(launch_block_batch(shape.m, shape.waves, c.ragged, b->d_jobs, b->d_state, items, c.count, c.heavy,
+                                      b->stream),
+                   "block_batch_kernel");
+        else
+            hipchk(launch_tile_batch(c.k, c.ragged, b->d_jobs, b->d_state, items, c.count, c.heavy, b->stream),
+                   "tile_batch_kernel");
         ++nl;
     }
     if (b->tuning) {
@@ -1073,8 +1195,7 @@ void run_round(lgca_batch* b)
                 b->tuning = false;
                 b->evaluating = true;
             } else {
-                b->k_cur = b->cands[b->cand_i].k;
-                b->waves_cur = b->cands[b->cand_i].waves;
+                b->cur = b->cands[b->cand_i];
             }
         }
     }
@@ -1102,8 +1223,8 @@ void run_round(lgca_batch* b)
         ++b->rounds;
         b->launches += nl;
         b->site_updates += su;
-        b->stat_k = b->k_cur;
-        b->stat_waves = b->waves_cur;
+        b->stat_k = shape.k;
+        b->stat_waves = shape.waves;
         b->stat_tunings = b->n_tunings;
     }
     while ((int)b->inflight.size() > kInflight) {

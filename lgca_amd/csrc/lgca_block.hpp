@@ -48,25 +48,18 @@ __device__ __forceinline__ uint32_t block_shift_p1(uint32_t v, const LaneCtx& c,
     return bit3<kMux>(last_bit, R << (c.nb - 1u), o);
 }
 
-// One workgroup's block.  FEAT: 0 no solids and no forcing on the lattice, 1
-// either.
+// One workgroup's block: strip `strip` of row tile `tile`, k steps with hk halo
+// rows.  FEAT: 0 no solids and no forcing on the lattice, 1 either.  Every
+// wave of the workgroup makes k + 1 barriers.
 template <int KIND, int M, bool RAGGED, int SEG, int FEAT>
-__global__ __launch_bounds__(kBlockMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 8)))
-void block_kernel(BlockArgs b)
+__device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32_t hk, uint32_t strip, uint32_t tile,
+                                           uint32_t* lds)
 {
     constexpr int Q = num_dir_of_kind(KIND);
     constexpr uint32_t NX = KIND == kHPP ? 1 : 2;  // planes exchanged per direction
-    extern __shared__ uint32_t lds[];
-    const TileArgs& a = b.a;
     const Geometry& g = a.g;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwave = blockDim.x >> 6;
-
-    // Workgroups go to the 8 XCDs round-robin; each XCD takes a contiguous
-    // run of blocks, whose halo rows meet in its L2.
-    const uint32_t xcd = blockIdx.x & 7u, xq = gridDim.x >> 3, xr = gridDim.x & 7u;
-    const uint32_t item = xcd * xq + min(xcd, xr) + (blockIdx.x >> 3);
-    const uint32_t tile = item / b.nstrips, strip = item - tile * b.nstrips;
     const uint32_t y0 = tile * a.th, rows = min(a.th, g.dim_y - y0);
 
     // this lane's word and the group of M rows it works on
@@ -102,7 +95,7 @@ void block_kernel(BlockArgs b)
     uint32_t j[M];
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-        int r = (int)y0 - (int)b.hk + (int)(group * M + m);
+        int r = (int)y0 - (int)hk + (int)(group * M + m);
         if (r < 0) r += dy;
         else if (r >= dy) r -= dy;
         if (r < 0 || r >= dy) r = (r % dy + dy) % dy;  // (blocks taller than the lattice)
@@ -113,8 +106,8 @@ void block_kernel(BlockArgs b)
     // with `left` steps to go: the wave works on its rows [wave_lo, wave_hi)
     // for the pass's first `act` steps.
     const int wave_lo = (int)(wave * S * M), wave_hi = wave_lo + (int)(S * M);
-    const int idle = max(0, max(wave_lo - (int)(b.hk + rows) + 1, (int)b.hk - wave_hi + 1));
-    const int act = (int)b.k - idle;
+    const int idle = max(0, max(wave_lo - (int)(hk + rows) + 1, (int)hk - wave_hi + 1));
+    const int act = (int)k - idle;
     const bool work = act >= 0;  // (at 0 its initial planes are still read)
 
     const uint32_t plane_b = g.P * 4u, row_b = (uint32_t)Q * plane_b;
@@ -136,7 +129,7 @@ void block_kernel(BlockArgs b)
     auto load_force = [&](int m, uint32_t step) {
         const uint32_t off = SEG ? foff[SEG ? m : 0] : (frow(m) ? foff[0] : kOutside);
         const uint32_t row = !SEG && frow(m) ? (j[m] - a.fy0) * a.fwn * 4u : 0u;
-        return bload(make_rsrc(a.fdec, b.k * fplane_b), off, step * fplane_b + row);
+        return bload(make_rsrc(a.fdec, k * fplane_b), off, step * fplane_b + row);
     };
     if (work) {
 #pragma unroll
@@ -267,11 +260,11 @@ void block_kernel(BlockArgs b)
                     if (m & 1) odd_row();
                     else even_row();
                 } else if (SEG != kSegments) {  // one row per wave: wave-uniform
-                    if ((wave + b.hk) & 1u) odd_row();
+                    if ((wave + hk) & 1u) odd_row();
                     else even_row();
                 } else {
                     // one row per segment: each lane shifts the way its row does
-                    const bool odd = ((group + b.hk) & 1u) != 0;
+                    const bool odd = ((group + hk) & 1u) != 0;
                     auto shifted = [&](uint32_t even_v, uint32_t odd_v) {
                         const uint32_t v = odd ? odd_v : even_v;
                         uint32_t n = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(odd ? c.rsrc : c.lsrc), (int)v);
@@ -320,7 +313,7 @@ void block_kernel(BlockArgs b)
                 else if (forced) apply_force<KIND, uint32_t>(st, f, a.force_dir);
                 // the next step's decisions (the last step's again after it: a
                 // test would wait for the load at its join)
-                if (FRC == 1 || forced) fd[m] = load_force(m, min(step + 1u, b.k - 1u));
+                if (FRC == 1 || forced) fd[m] = load_force(m, min(step + 1u, k - 1u));
             }
 #pragma unroll
             for (int d = 0; d < Q; ++d) s[m][d] = st[d];
@@ -330,19 +323,19 @@ void block_kernel(BlockArgs b)
     // A loop per mode, so that the force decisions of the next step stay in
     // flight across the barrier (with one loop and tests in it, the paths
     // without loads made every step wait for them).  The mode and the steps
-    // that a wave works on are wave-uniform, and every wave makes b.k barriers.
+    // that a wave works on are wave-uniform, and every wave makes k barriers.
     auto pass = [&](auto sol_tag, auto frc_tag) {
         for (int step = 0; step < act; ++step) {
             advance(sol_tag, frc_tag, (uint32_t)step);
             __syncthreads();
         }
-        for (int step = max(act, 0); step < (int)b.k; ++step) __syncthreads();
+        for (int step = max(act, 0); step < (int)k; ++step) __syncthreads();
         if (idle) return;  // the wave holds no stored row
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             const uint32_t l = group * M + m;
-            const bool wr = writer && l >= b.hk && l < b.hk + rows;
-            if (!SEG && !(l >= b.hk && l < b.hk + rows)) continue;  // wave-uniform
+            const bool wr = writer && l >= hk && l < hk + rows;
+            if (!SEG && !(l >= hk && l < hk + rows)) continue;  // wave-uniform
 #pragma unroll
             for (int d = 0; d < Q; ++d) {
                 if (RAGGED) s[m][d] &= c.vmask;
@@ -359,6 +352,68 @@ void block_kernel(BlockArgs b)
     else if (!solid_rows) pass(I0{}, I1{});
     else if (!forced) pass(I1{}, I0{});
     else pass(I1{}, I1{});
+}
+
+template <int KIND, int M, bool RAGGED, int SEG, int FEAT>
+__global__ __launch_bounds__(kBlockMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void block_kernel(BlockArgs b)
+{
+    extern __shared__ uint32_t block_lds[];
+    // Workgroups go to the 8 XCDs round-robin; each XCD takes a contiguous
+    // run of blocks, whose halo rows meet in its L2.
+    const uint32_t xcd = blockIdx.x & 7u, xq = gridDim.x >> 3, xr = gridDim.x & 7u;
+    const uint32_t item = xcd * xq + min(xcd, xr) + (blockIdx.x >> 3);
+    const uint32_t tile = item / b.nstrips, strip = item - tile * b.nstrips;
+    block_body<KIND, M, RAGGED, SEG, FEAT>(b.a, b.k, b.hk, strip, tile, block_lds);
+}
+
+// Batched form (tile_batch_kernel's): every workgroup takes one work item.  A
+// job's steps in the round are in its items (block_shape_bits), so jobs at
+// their last steps share the launch, and a pass may start at any step.
+template <int M, bool RAGGED>
+__global__ __launch_bounds__(kBlockMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void block_batch_kernel(const BatchJob* __restrict__ jobs, BatchState* state, const WorkItem* __restrict__ items,
+                        uint32_t n_heavy)
+{
+    extern __shared__ uint32_t block_lds[];
+    // the leading (heavy) items and the rest each map to contiguous runs per XCD
+    const bool in_heavy = blockIdx.x < n_heavy;
+    const uint32_t i = in_heavy ? blockIdx.x : blockIdx.x - n_heavy, n = in_heavy ? n_heavy : gridDim.x - n_heavy;
+    const uint32_t xcd = i & 7u, q = n >> 3, r = n & 7u;
+    const uint32_t wi = __builtin_amdgcn_readfirstlane((in_heavy ? 0u : n_heavy) + xcd * q + min(xcd, r) + (i >> 3));
+    const WorkItem it = items[wi];
+    const BatchState bs = state[it.job];
+    TileArgs a = jobs[it.job].a;
+    a.t0 = bs.step;
+    a.th = it.shape & 0xFFFFu;
+    a.halo = (it.shape >> 16) & 0xFFu;
+    a.src = bs.cur ? jobs[it.job].buf1 : jobs[it.job].buf0;
+    a.dst = bs.cur ? jobs[it.job].buf0 : jobs[it.job].buf1;
+    if (a.fdec) a.fdec += (size_t)(bs.step - bs.fdec_step0) * a.fdec_stride;
+    const uint32_t k = (it.shape >> 24) & 0x7Fu, hk = block_halo(M, k);
+    const bool seg = (it.shape >> 31) != 0;
+    const uint32_t Q = __builtin_amdgcn_readfirstlane(a.g.Q);
+    if (Q == 4) {
+        if (seg) block_body<kHPP, M, RAGGED, kSegments, 1>(a, k, hk, it.strip, it.tile, block_lds);
+        else block_body<kHPP, M, RAGGED, kStrips, 1>(a, k, hk, it.strip, it.tile, block_lds);
+    } else if (Q == 6) {
+        if (seg) block_body<kFHP1, M, RAGGED, kSegments, 1>(a, k, hk, it.strip, it.tile, block_lds);
+        else block_body<kFHP1, M, RAGGED, kStrips, 1>(a, k, hk, it.strip, it.tile, block_lds);
+    } else {
+        if (seg) block_body<kFHP2, M, RAGGED, kSegments, 1>(a, k, hk, it.strip, it.tile, block_lds);
+        else block_body<kFHP2, M, RAGGED, kStrips, 1>(a, k, hk, it.strip, it.tile, block_lds);
+    }
+    // The job's last workgroup of the round advances it.  Every wave of every
+    // other one has read the state by now: a wave comes here after the body's
+    // barriers, which its workgroup's waves pass with the state read.
+    if (threadIdx.x == 0) {
+        BatchState& st = state[it.job];
+        if (atomicAdd(&st.done, 1u) + 1u == it.job_items) {
+            st.done = 0;
+            st.step = bs.step + k;
+            st.cur = bs.cur ^ 1u;
+        }
+    }
 }
 
 template <int KIND, int M>
@@ -381,6 +436,17 @@ hipError_t launch_block_km(const BlockArgs& b, uint32_t waves, uint32_t blocks, 
         else LGCA_BLOCK_LAUNCH(false, kStrips);
     }
 #undef LGCA_BLOCK_LAUNCH
+    return hipGetLastError();
+}
+
+template <int M>
+hipError_t launch_block_batch_m(const BatchJob* jobs, BatchState* state, const WorkItem* items, uint32_t n_items,
+                                uint32_t n_heavy, uint32_t waves, bool ragged, hipStream_t s)
+{
+    const dim3 grid(n_items), block(64 * waves);
+    const size_t lds = block_lds_bytes(kFHP2, M, waves);
+    if (ragged) hipLaunchKernelGGL((block_batch_kernel<M, true>), grid, block, lds, s, jobs, state, items, n_heavy);
+    else hipLaunchKernelGGL((block_batch_kernel<M, false>), grid, block, lds, s, jobs, state, items, n_heavy);
     return hipGetLastError();
 }
 

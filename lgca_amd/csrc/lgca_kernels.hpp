@@ -157,7 +157,7 @@ struct BlockShape {
 };
 constexpr uint32_t kBlockMaxSteps = 28;  // steps per pass the planner considers
 // Halo rows either side of a block for k-step passes.
-inline uint32_t block_halo(uint32_t m, uint32_t k) { return m == 1 ? k : (k + 1) & ~1u; }
+__host__ __device__ inline uint32_t block_halo(uint32_t m, uint32_t k) { return m == 1 ? k : (k + 1) & ~1u; }
 // LDS bytes of a workgroup.
 uint32_t block_lds_bytes(int kind, uint32_t m, uint32_t waves);
 // Predicted time (us) of a k-step pass of shape s, or a negative number where
@@ -199,6 +199,17 @@ struct WorkItem {
 // finishes a job's last item of the round moves the job K steps on and swaps
 // its buffers, for the next round's launches to read.
 // n_heavy: the class's leading items that can take the general walk.
+// The same in blocks of m rows per wave, `waves` waves per workgroup (one per
+// item; item shapes are block_shape_bits, steps included).
+hipError_t launch_block_batch(uint32_t m, uint32_t waves, bool ragged, const BatchJob* jobs, BatchState* state,
+                              const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s);
+template <int M>
+hipError_t launch_block_batch_m(const BatchJob* jobs, BatchState* state, const WorkItem* items, uint32_t n_items,
+                                uint32_t n_heavy, uint32_t waves, bool ragged, hipStream_t s);
+inline uint32_t block_shape_bits(uint32_t th, uint32_t halo, uint32_t k, bool seg)
+{
+    return th | (halo << 16) | (k << 24) | (seg ? 1u << 31 : 0u);
+}
 hipError_t launch_tile_batch(int k, bool ragged, const BatchJob* jobs, BatchState* state,
                              const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s);
 

@@ -24,6 +24,19 @@ hipError_t launch_tile_batch(int k, bool ragged, const BatchJob* jobs, BatchStat
     }
 }
 
+hipError_t launch_block_batch(uint32_t m, uint32_t waves, bool ragged, const BatchJob* jobs, BatchState* state,
+                              const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s)
+{
+    if (!n_items) return hipSuccess;
+    if (!waves || waves > kBlockMaxWaves) return hipErrorInvalidValue;
+    n_heavy = std::min(n_heavy, n_items);
+    switch (m) {
+    case 2: return launch_block_batch_m<2>(jobs, state, items, n_items, n_heavy, waves, ragged, s);
+    case 4: return launch_block_batch_m<4>(jobs, state, items, n_items, n_heavy, waves, ragged, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_tile_pipe(int kind, int k, const TileArgs& a, const PipeArgs& p, uint32_t nwaves, hipStream_t s)
 {
     if (tile_segments(a.g, k) || a.g.nb != 32 || a.th < (uint32_t)k || (a.th & 1u) || a.th > 65535)

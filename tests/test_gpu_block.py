@@ -97,3 +97,28 @@ def test_block_shapes_of_larger_lattices(model, dx, dy, geom, force, n):
 @pytest.mark.parametrize("dx,dy,geom", [(256, 256, None), (1001, 300, "mixed"), (2048, 130, "pipe")])
 def test_tuned_block_shapes(dx, dy, geom):
     check(2, dx, dy, geom, dict(dir="x", p=0.03), calls=(7, 64, 20), step0=1, tune=True)
+
+
+def test_batch_blocks_match_the_oracle():
+    """A batch small enough to run in blocks: every model, rows of several
+    strips and segments, short last words, forcing, given cell types, and steps
+    that end in the middle of a round."""
+    from lgca_amd import Batch, Job
+    rng = np.random.default_rng(8)
+    jobs, want = [], []
+    for i, (model, dx, dy, geom, force) in enumerate(
+            [c for c in CASES if c[1] > 16] + [(2, 2100, 90, "mixed", None), (0, 4160, 33, "slip", None)]):
+        types = make_types(rng, dx, dy, geom)
+        state = rng.integers(0, 1 << Q[model], dx * dy, dtype=np.uint8)
+        f = force or {}
+        jobs.append(Job(model, dx, dy, 17 + 5 * i, seed=60 + i, geometry="types", cell_types=types, state=state,
+                        force_dir=f.get("dir"), force_p=f.get("p", 0.0),
+                        force_region=(f.get("x0", 0), f.get("x1") or dx, f.get("y0", 0), f.get("y1") or dy)))
+        want.append(orc.run(model, dx, dy, types, state, 60 + i, 0, jobs[-1].steps, force, nthreads=8))
+    print(f"[block batch] {len(jobs)} jobs", flush=True)
+    with Batch(hbm_budget=4 * 10**9) as b:
+        ids = [b.submit(j) for j in jobs]
+        b.wait(timeout=60)
+        assert b.stats()["wave_target"] <= 16  # waves per workgroup: the rounds ran in blocks
+        for i, w in zip(ids, want):
+            np.testing.assert_array_equal(b.result(i)[0], w)
