@@ -22,16 +22,6 @@
 using namespace lgca;
 
 namespace lgca {
-// Device-resident state of the viewers' forcing controller.
-struct Controller {
-    long long acc[3];   // mean-velocity sums of the snapshot: x, y (units of 1/840), FLUID cells
-    long long forcing;  // the controller's current forcing amount
-    long long amount;   // this tick: amount to apply, or -1
-    long long reverted; // particles reverted by the last applied force
-    uint32_t calls;     // count-mode force call counter (hash stream 3)
-    float v[2];         // mean velocity the last decision saw
-};
-
 // Steps per pass and rows per tile of one tiled launch.
 struct LaunchShape {
     int k;
@@ -132,6 +122,9 @@ struct lgca_lattice {
     int ctrl_dir = LGCA_FORCE_NONE;
     float ctrl_u = 0.0f;
     int64_t ctrl_eq = 0;
+    int64_t ctrl_most = 0;          // the larger of the controller's two amounts
+    void* force_ws = nullptr;       // count-mode force: listed tries (count_force_bytes)
+    size_t force_ws_bytes = 0;
     bool calls_on_device = false;   // the count-mode call counter lives in ctrl
     std::string err;
     std::mutex mu;
@@ -238,209 +231,7 @@ lgca_status sync_force_calls(lgca_lattice* h)
 
 }  // namespace
 
-// -------------------------------------------------------------- count force
-// apply_body_force(int forcing), src/omp_lattice.cpp:254-346.  The sequential
-// loop's result depends on the order of its tries only through where it stops:
-// a cell that has been visited never flips again (its visit makes its flip
-// rules infeasible, or they were so already), so after M tries exactly the
-// feasible rules of the distinct cells among them have been applied.  One
-// workgroup therefore takes the candidate sequence 4096 tries at a time.  It
-// counts the feasible rules of a batch with repeats; while even that many
-// reverts stay below `forcing` the sequence cannot stop inside the batch, and
-// its lanes apply their flips at once, a repeated cell going to whichever
-// lane clears its bit first.  The batch that may hold the stop is replayed in
-// order, 1024 tries at a time: repeats of a feasible cell are dropped, a
-// prefix sum over the lanes finds the first try whose running total reaches
-// `forcing` (always after at least one try), and the flips up to it apply.
-//
-// Bound: two rounds of L2 latency per batch.  Finding 10,952 reverts on a
-// 1480 x 740 lattice (some 90,000 tries) took 8.2 ms with one wave, 64 tries
-// and a visited bitmap at a time; 0.47 ms so.
 namespace lgca {
-
-constexpr uint32_t kForceThreads = 1024, kForceTries = 4;
-
-// floor(a / n) and a - n * floor(a / n) from m = floor((2^64 - 1) / n): the
-// product's high half is the quotient or one less.
-__device__ __forceinline__ uint64_t divmod_magic(uint64_t a, uint64_t n, uint64_t m, uint64_t& rem)
-{
-    uint64_t q = __umul64hi(a, m);
-    rem = a - q * n;
-    if (rem >= n) {
-        rem -= n;
-        ++q;
-    }
-    return q;
-}
-
-struct CountForceArgs {
-    uint32_t* planes;
-    const uint32_t* mask;
-    Geometry g;
-    uint32_t key0, key1;
-    int dir;
-    uint64_t cells_magic, row_magic;  // of the cell count and of dim_x
-};
-
-template <int KIND>
-__device__ __forceinline__ void count_force_body(const CountForceArgs& a, uint32_t call, long long forcing,
-                                                 long long* result)
-{
-    constexpr int Q = num_dir_of_kind(KIND);
-    constexpr uint32_t kWaves = kForceThreads / 64;
-    __shared__ uint32_t part[2][kWaves];   // per-wave sums of the two barriers of a batch
-    __shared__ uint32_t first_hit;
-    __shared__ uint64_t list[kForceThreads];
-    const Geometry& g = a.g;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint64_t n = (uint64_t)g.dim_x * g.dim_y, it_max = 2 * n;
-    // the flip rules (src/omp_lattice.cpp:293-337): a particle moves from
-    // plane `from` to plane `to` where `to` is empty
-    const bool x = a.dir == 1;
-    const uint32_t rules = KIND != kHPP && !x ? 2u : 1u;
-    const uint32_t from[2] = {KIND == kHPP ? (x ? 2u : 1u) : (x ? 3u : 1u), 2u};
-    const uint32_t to[2] = {KIND == kHPP ? (x ? 0u : 3u) : (x ? 0u : 5u), 4u};
-
-    struct Try {
-        uint64_t cell;
-        uint32_t* word;   // word 0 of the cell's row and column in plane 0
-        uint32_t bit;     // 0: not a FLUID cell, or past the last try
-    };
-    auto make_try = [&](uint64_t i) {
-        Try t;
-        const U4 r = philox4x32_10((uint32_t)i, (uint32_t)(i >> 32), call, 3u, a.key0, a.key1);
-        uint64_t xx;
-        divmod_magic(((uint64_t)r.y << 32) | r.x, n, a.cells_magic, t.cell);
-        const uint32_t y = (uint32_t)divmod_magic(t.cell, g.dim_x, a.row_magic, xx);
-        const uint32_t w = (uint32_t)xx >> 5;
-        t.word = a.planes + (size_t)y * Q * g.P + w;
-        t.bit = i < it_max ? 1u << ((uint32_t)xx & 31u) : 0u;
-        if (a.mask)
-            t.bit &= ~(a.mask[((size_t)y * 2 + 0) * g.P + w] | a.mask[((size_t)y * 2 + 1) * g.P + w]);
-        return t;
-    };
-    // the planes change under the loop: read past the L1
-    auto plane = [&](const Try& t, uint32_t d) {
-        return __hip_atomic_load(t.word + (size_t)d * g.P, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    // feasible rules of a try, bit r for rule r
-    auto feasible = [&](const Try& t) {
-        // (every cell is on the lattice, so the loads need no test)
-        uint32_t f = (plane(t, from[0]) & ~plane(t, to[0]) & t.bit) ? 1u : 0u;
-        if (rules == 2) f |= (plane(t, from[1]) & ~plane(t, to[1]) & t.bit) ? 2u : 0u;
-        return f;
-    };
-    // applies the feasible rules f of a try; the number that this lane applied
-    auto flip = [&](const Try& t, uint32_t f) {
-        uint32_t k = 0;
-        for (uint32_t r = 0; r < rules; ++r) {
-            if (!((f >> r) & 1u)) continue;
-            if (atomicAnd(t.word + (size_t)from[r] * g.P, ~t.bit) & t.bit) {
-                atomicOr(t.word + (size_t)to[r] * g.P, t.bit);
-                ++k;
-            }
-        }
-        return k;
-    };
-    // sum of v over the workgroup; every lane gets it.  Flips made before it
-    // are in the L2 after it.
-    auto block_sum = [&](uint32_t v, uint32_t slot) {
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (lane == 0) part[slot][wave] = v;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        uint32_t s = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < kWaves; ++k) s += part[slot][k];
-        return s;
-    };
-
-    long long reverted = 0;
-    bool stop = false;
-    for (uint64_t base = 0; base < it_max && !stop; base += kForceThreads * kForceTries) {
-        Try t[kForceTries];
-        uint32_t f[kForceTries], most = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < kForceTries; ++u) t[u] = make_try(base + u * kForceThreads + tid);
-#pragma unroll
-        for (uint32_t u = 0; u < kForceTries; ++u) f[u] = feasible(t[u]);
-#pragma unroll
-        for (uint32_t u = 0; u < kForceTries; ++u) most += __popc(f[u]);
-        if (reverted + (long long)block_sum(most, 0) < forcing) {
-            uint32_t k = 0;
-#pragma unroll
-            for (uint32_t u = 0; u < kForceTries; ++u) k += flip(t[u], f[u]);
-            reverted += block_sum(k, 1);
-            continue;
-        }
-        // the sequence may stop here: in order, kForceThreads tries at a time
-#pragma unroll 1
-        for (uint32_t u = 0; u < kForceTries && !stop; ++u) {
-            const uint64_t i = base + u * kForceThreads + tid;
-            const Try c = make_try(i);
-            uint32_t fu = feasible(c);
-            // list the feasible tries in order, then drop repeats of a cell
-            const unsigned long long here = __ballot(fu != 0);
-            const uint32_t below = (uint32_t)__popcll(here & ((1ull << lane) - 1ull));
-            if (tid == 0) first_hit = kForceThreads;
-            block_sum(fu != 0, 0);
-            uint32_t pos = below;
-            for (uint32_t k = 0; k < wave; ++k) pos += part[0][k];
-            if (fu) list[pos] = c.cell;
-            __syncthreads();
-            if (fu)
-                for (uint32_t k = 0; k < pos; ++k)
-                    if (list[k] == c.cell) {
-                        fu = 0;
-                        break;
-                    }
-            // inclusive running total of the reverts
-            uint32_t incl = __popc(fu);
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t v = __shfl_up(incl, off, 64);
-                if ((int)lane >= off) incl += v;
-            }
-            const uint32_t total = block_sum(__popc(fu), 1);
-            for (uint32_t k = 0; k < wave; ++k) incl += part[1][k];
-            if (i < it_max && reverted + (long long)incl >= forcing) atomicMin(&first_hit, tid);
-            __syncthreads();
-            const uint32_t limit = first_hit;
-            if (fu && tid <= limit) flip(c, fu);
-            stop = limit < kForceThreads;
-            // (when limit is the last lane, its total is the block's)
-            if (stop) {
-                if (tid == limit) list[0] = incl;
-                __syncthreads();
-                reverted += (long long)list[0];
-            } else {
-                reverted += total;
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-        }
-    }
-    if (tid == 0) *result = reverted;
-}
-
-template <int KIND>
-__global__ __launch_bounds__(kForceThreads) void body_force_count_kernel(CountForceArgs a, uint32_t call,
-                                                                         long long forcing, long long* result)
-{
-    count_force_body<KIND>(a, call, forcing, result);
-}
-
-// The same, with the amount and call number the controller left on the GPU;
-// nothing happens (and no call is counted) when the amount is negative.
-template <int KIND>
-__global__ __launch_bounds__(kForceThreads) void controlled_force_kernel(CountForceArgs a, Controller* c)
-{
-    const long long amount = c->amount;
-    if (amount < 0) return;
-    const uint32_t call = c->calls;
-    __syncthreads();
-    count_force_body<KIND>(a, call, amount, &c->reverted);
-    if (threadIdx.x == 0) c->calls = call + 1;
-}
 
 // The viewers' decision (apps/pipe/pipe_viewer.cpp:107-125): the mean x
 // velocity of the snapshot, in the FP32 value lgca_mean_velocity returns; if
@@ -539,7 +330,7 @@ extern "C" lgca_status lgca_destroy(lgca_lattice* h)
         if (h->stream && h->stream != h->own_stream) (void)hipStreamSynchronize(h->stream);
         void* ptrs[] = {h->state[0], h->state[1], h->snap, h->mask, h->row_range, h->dec,
                         h->cell_density, h->cell_momentum, h->mean_density, h->mean_momentum,
-                        h->velocity, h->bytes, h->counters, h->ctrl};
+                        h->velocity, h->bytes, h->counters, h->ctrl, h->force_ws};
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
         for (const WaveOrder& o : h->orders) (void)hipFree(o.dev);
@@ -1674,18 +1465,33 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
     return LGCA_OK;
 }
 
-static CountForceArgs count_force_args(const lgca_lattice* h, int dir)
+// Queues a count-mode force of the live state (lgca_force.hip).  most: the
+// largest amount that may be asked for.
+static lgca_status queue_count_force(lgca_lattice* h, CountForceArgs a, int dir, int64_t most)
 {
-    CountForceArgs a{};
+    const uint64_t n = (uint64_t)h->dim_x * h->dim_y;
     a.planes = h->state[h->cur];
     a.mask = h->mask;
     a.g = h->g;
     a.key0 = (uint32_t)h->seed;
     a.key1 = (uint32_t)(h->seed >> 32);
     a.dir = dir;
-    a.cells_magic = UINT64_MAX / ((uint64_t)h->dim_x * h->dim_y);
+    a.cells_magic = UINT64_MAX / n;
     a.row_magic = UINT64_MAX / h->dim_x;
-    return a;
+    a.tries = count_force_tries(n, most);
+    if (a.tries && h->force_ws_bytes < count_force_bytes(a.tries)) {
+        if (h->force_ws) {
+            HIPCHK(h, hipStreamSynchronize(h->stream));
+            HIPCHK(h, hipFree(h->force_ws));
+        }
+        h->force_ws = nullptr;
+        h->force_ws_bytes = 0;
+        HIPCHK(h, dalloc(&h->force_ws, count_force_bytes(a.tries)));
+        h->force_ws_bytes = count_force_bytes(a.tries);
+    }
+    a.ws = h->force_ws;
+    HIPCHK(h, launch_count_force(h->kind, a, h->stream));
+    return LGCA_OK;
 }
 
 extern "C" lgca_status lgca_apply_body_force_count(lgca_lattice* h, int dir, int64_t forcing,
@@ -1705,15 +1511,11 @@ extern "C" lgca_status lgca_apply_body_force_count(lgca_lattice* h, int dir, int
     if (st0) return st0;
     lgca_status st = clear_counters(h);
     if (st) return st;
-    const uint32_t call = (uint32_t)h->force_calls++;
-    const CountForceArgs a = count_force_args(h, dir);
-    long long* res = (long long*)h->counters;
-    switch (h->kind) {
-    case kHPP: hipLaunchKernelGGL(body_force_count_kernel<kHPP>, dim3(1), dim3(kForceThreads), 0, h->stream, a, call, target, res); break;
-    case kFHP1: hipLaunchKernelGGL(body_force_count_kernel<kFHP1>, dim3(1), dim3(kForceThreads), 0, h->stream, a, call, target, res); break;
-    default: hipLaunchKernelGGL(body_force_count_kernel<kFHP2>, dim3(1), dim3(kForceThreads), 0, h->stream, a, call, target, res); break;
-    }
-    HIPCHK(h, hipGetLastError());
+    CountForceArgs a{};
+    a.call = (uint32_t)h->force_calls++;
+    a.amount = target;
+    a.result = (long long*)h->counters;
+    if ((st = queue_count_force(h, a, dir, target))) return st;
     unsigned long long v = 0;
     if ((st = read_counters(h, &v, 1))) return st;
     if (reverted) *reverted = (int64_t)v;
@@ -2022,6 +1824,7 @@ extern "C" lgca_status lgca_load_checkpoint(lgca_lattice** out, const char* path
             h->ctrl_dir = hd.ctrl_dir;
             h->ctrl_u = hd.ctrl_u;
             h->ctrl_eq = hd.ctrl_eq;
+            h->ctrl_most = std::max(hd.ctrl_forcing, hd.ctrl_eq);
             h->calls_on_device = false;
         }
         if (!st) {
@@ -2064,6 +1867,7 @@ extern "C" lgca_status lgca_controller_set(lgca_lattice* h, int dir, float u, in
     h->ctrl_dir = dir;
     h->ctrl_u = u;
     h->ctrl_eq = equilibrium_forcing;
+    h->ctrl_most = std::max(forcing, equilibrium_forcing);
     return LGCA_OK;
 }
 
@@ -2085,16 +1889,12 @@ extern "C" lgca_status lgca_controller_tick(lgca_lattice* h, uint64_t steps)
                        (long long)h->ctrl_eq, unit_y);
     HIPCHK(h, hipGetLastError());
     // count-mode force with the decided amount
-    const CountForceArgs a = count_force_args(h, h->ctrl_dir);
-    switch (h->kind) {
-    case kHPP: hipLaunchKernelGGL(controlled_force_kernel<kHPP>, dim3(1), dim3(kForceThreads), 0, h->stream, a, h->ctrl); break;
-    case kFHP1: hipLaunchKernelGGL(controlled_force_kernel<kFHP1>, dim3(1), dim3(kForceThreads), 0, h->stream, a, h->ctrl); break;
-    default: hipLaunchKernelGGL(controlled_force_kernel<kFHP2>, dim3(1), dim3(kForceThreads), 0, h->stream, a, h->ctrl); break;
-    }
-    HIPCHK(h, hipGetLastError());
-    // the steps, then the snapshot the next tick decides on
-    lgca_status st = step_locked(h, steps);
+    CountForceArgs a{};
+    a.ctrl = h->ctrl;
+    lgca_status st = queue_count_force(h, a, h->ctrl_dir, h->ctrl_most);
     if (st) return st;
+    // the steps, then the snapshot the next tick decides on
+    if ((st = step_locked(h, steps))) return st;
     HIPCHK(h, hipMemcpyAsync(h->snap, h->state[h->cur], h->state_words * 4, hipMemcpyDeviceToDevice,
                              h->stream));
     return LGCA_OK;

@@ -275,4 +275,37 @@ hipError_t launch_mean_velocity(int kind, const uint32_t* planes, const uint32_t
                                 const Geometry& g, long long* acc3, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 
+// Device-resident state of the viewers' forcing controller.
+struct Controller {
+    long long acc[3];   // mean-velocity sums of the snapshot: x, y (units of 1/840), FLUID cells
+    long long forcing;  // the controller's current forcing amount
+    long long amount;   // this tick: amount to apply, or -1
+    long long reverted; // particles reverted by the last applied force
+    uint32_t calls;     // count-mode force call counter (hash stream 3)
+    float v[2];         // mean velocity the last decision saw
+};
+
+// Count-mode body force (lgca_force.hip).
+struct CountForceArgs {
+    uint32_t* planes;
+    const uint32_t* mask;
+    Geometry g;
+    uint32_t key0, key1;
+    int dir;                          // 1 x, 2 y
+    uint64_t cells_magic, row_magic;  // floor((2^64 - 1) / n) of the cell count and of dim_x
+    // the call's number, amount and where its reverted count goes; with a
+    // controller, its own (amount -1: nothing is done and no call counted)
+    uint32_t call;
+    long long amount;
+    long long* result;
+    Controller* ctrl;
+    uint32_t tries;                   // tries listed ahead (0: none), and their workspace
+    void* ws;
+};
+// Tries to list ahead for a lattice of n cells and amounts up to `most`, and
+// the bytes their workspace takes.
+uint32_t count_force_tries(uint64_t n, int64_t most);
+size_t count_force_bytes(uint32_t tries);
+hipError_t launch_count_force(int kind, const CountForceArgs& a, hipStream_t s);
+
 }  // namespace lgca
