@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void setup_kernel(const JobInstall* __restrict
         const uint32_t fluid = valid & ~ns;
         for (uint32_t d = 0; d < g.Q; ++d) {
             const size_t at = ((size_t)y * g.Q + d) * g.P + w;
-            r.job.buf0[at] = fluid ? (fill_word(w, y, d, g.dim_x, r.job.a.key0, r.job.a.key1, r.fill_thr) & fluid) : 0u;
+            r.job.buf0[at] = fluid ? (fill_word(w, y, d, r.job.a.key0, r.job.a.key1, r.fill_thr) & fluid) : 0u;
             r.job.buf1[at] = 0u;
         }
     }

@@ -230,21 +230,20 @@ __host__ __device__ __forceinline__ void apply_force(T s[7], T f, int dir)
 }
 
 // Initial fill of plane d of word w of row y (hash stream 2): bit b is set
-// when philox({x >> 2, y, d, 2})[x & 3] < thr for x = 32w + b < dim_x.
-__device__ __forceinline__ uint32_t fill_word(uint32_t w, uint32_t y, uint32_t d, uint32_t dim_x,
-                                              uint32_t key0, uint32_t key1, uint64_t thr)
+// when philox({x >> 2, y, d, 2})[x & 3] < thr for x = 32w + b, also past the end
+// of the row: the caller masks.
+__device__ __forceinline__ uint32_t fill_word(uint32_t w, uint32_t y, uint32_t d, uint32_t key0, uint32_t key1,
+                                              uint64_t thr)
 {
+    const uint32_t t = (uint32_t)thr, all = (uint32_t)(thr >> 32);  // thr = 2^32 fills every cell
     uint32_t word = 0;
+#pragma unroll
     for (uint32_t gi = 0; gi < 8; ++gi) {
-        const uint32_t x = 32 * w + 4 * gi;
-        if (x >= dim_x) break;
-        const U4 r = philox4x32_10(x >> 2, y, d, 2u, key0, key1);
-        word |= (uint32_t)((uint64_t)r.x < thr) << (4 * gi + 0);
-        word |= (uint32_t)((uint64_t)r.y < thr) << (4 * gi + 1);
-        word |= (uint32_t)((uint64_t)r.z < thr) << (4 * gi + 2);
-        word |= (uint32_t)((uint64_t)r.w < thr) << (4 * gi + 3);
+        const U4 r = philox4x32_10(8 * w + gi, y, d, 2u, key0, key1);
+        word |= ((uint32_t)(r.x < t) | (uint32_t)(r.y < t) << 1 | (uint32_t)(r.z < t) << 2 | (uint32_t)(r.w < t) << 3)
+                << (4 * gi);
     }
-    return word;
+    return all ? ~0u : word;
 }
 
 // Per-cell force decisions of word w of row y at one step of the four-step

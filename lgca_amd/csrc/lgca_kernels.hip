@@ -236,61 +236,193 @@ hipError_t launch_force_draw(const ForceDrawArgs& a, hipStream_t s)
 }
 
 // ------------------------------------------------------------------ codec
+// One byte per cell to and from planes.  Bytes and planes cross memory once
+// each, which is the bound; a lane therefore moves 16 bytes at a time.  A row
+// starts at any byte (y * dim_x): loads are unaligned, as global memory takes
+// them on this target, stores are aligned to the memory, and only the cells at a
+// row's ends are moved byte by byte.  4100 x 2050, one byte at a time -> so:
+// unpack 12.5 -> 8.0 us (6000 x 3000 23 -> 8.9), cell types 24 -> 5.4 us; pack of 8192 x 4096 71 -> 14 us.
+// Workgroups are qx lanes wide (row_lanes) by 256 / qx rows.
 
-__global__ __launch_bounds__(256) void pack_kernel(const uint8_t* __restrict__ st,
-                                                   uint32_t* __restrict__ planes, Geometry g,
-                                                   uint32_t* err)
+constexpr uint32_t kCodecCells = 16;
+
+// Lanes along x for rows of n items: as many, up to a wave, as leave at most
+// an eighth of the lanes without work, and at least 8.
+static uint32_t row_lanes(uint32_t n)
 {
-    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t y = blockIdx.y;
-    if (w >= g.P) return;
-    uint32_t acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t bad = 0;
+    uint32_t qx = 64;
+    while (qx > 8 && div_up(n, qx) * qx > n + n / 8) qx >>= 1;
+    return qx;
+}
+
+static dim3 row_grid(const Geometry& g, uint32_t n, uint32_t qx) { return dim3(div_up(n, qx), div_up(g.dim_y, 256u / qx)); }
+
+struct Bytes16 {
+    uint32_t v[4];
+};
+
+__device__ __forceinline__ Bytes16 load_bytes16(const uint8_t* p)
+{
+    Bytes16 r;
+    __builtin_memcpy(&r, p, 16);
+    return r;
+}
+
+// Bit d of 16 bytes, the byte of cell 0 first.
+__device__ __forceinline__ uint32_t gather_bits(const Bytes16& c, int d)
+{
+    const uint32_t m = 0x01010101u;
+    const uint32_t lo = __builtin_amdgcn_udot4((c.v[1] >> d) & m, 0x80402010u,
+                                               __builtin_amdgcn_udot4((c.v[0] >> d) & m, 0x08040201u, 0u, false), false);
+    const uint32_t hi = __builtin_amdgcn_udot4((c.v[3] >> d) & m, 0x80402010u,
+                                               __builtin_amdgcn_udot4((c.v[2] >> d) & m, 0x08040201u, 0u, false), false);
+    return lo | (hi << 8);
+}
+
+// Transpose of an 8 x 8 bit matrix, row r in byte r of hi:lo (the three swaps of
+// Hacker's Delight, section 7-3).
+__device__ __forceinline__ void transpose8(uint32_t& lo, uint32_t& hi)
+{
+    uint32_t t = (lo ^ (lo >> 7)) & 0x00AA00AAu, u = (hi ^ (hi >> 7)) & 0x00AA00AAu;
+    lo ^= t ^ (t << 7);
+    hi ^= u ^ (u << 7);
+    t = (lo ^ (lo >> 14)) & 0x0000CCCCu;
+    u = (hi ^ (hi >> 14)) & 0x0000CCCCu;
+    lo ^= t ^ (t << 14);
+    hi ^= u ^ (u << 14);
+    t = (lo ^ (hi << 4)) & 0xF0F0F0F0u;
+    lo ^= t;
+    hi ^= t >> 4;
+}
+
+template <int Q>
+__global__ __launch_bounds__(256) void pack_kernel(const uint8_t* __restrict__ st, uint32_t* __restrict__ planes,
+                                                   Geometry g, uint32_t* err)
+{
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t y = blockIdx.y * blockDim.y + threadIdx.y;
+    if (w >= g.P || y >= g.dim_y) return;
+    uint32_t acc[Q] = {}, bad = 0;
     const uint8_t* row = st + (size_t)y * g.dim_x;
-    for (uint32_t b = 0; b < 32; ++b) {
-        const uint32_t x = 32 * w + b;
-        if (x >= g.dim_x) break;
-        const uint32_t v = row[x];
-        bad |= v >> g.Q;
 #pragma unroll
-        for (int d = 0; d < 8; ++d) acc[d] |= ((v >> d) & 1u) << b;
+    for (uint32_t half = 0; half < 2; ++half) {
+        const uint32_t x = 32 * w + kCodecCells * half;
+        Bytes16 c = {};
+        if (x + kCodecCells <= g.dim_x) c = load_bytes16(row + x);
+        else
+            for (uint32_t b = 0; x + b < g.dim_x; ++b) {
+                const uint32_t v = (uint32_t)row[x + b] << (8 * (b & 3u));
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) c.v[k] |= b >> 2 == k ? v : 0u;
+            }
+        bad |= (c.v[0] | c.v[1] | c.v[2] | c.v[3]) & ((0xFFu << Q & 0xFFu) * 0x01010101u);
+#pragma unroll
+        for (int d = 0; d < Q; ++d) acc[d] |= gather_bits(c, d) << (16 * half);
     }
-    for (uint32_t d = 0; d < g.Q; ++d) planes[((size_t)y * g.Q + d) * g.P + w] = acc[d];
+#pragma unroll
+    for (int d = 0; d < Q; ++d) planes[((size_t)y * Q + d) * g.P + w] = acc[d];
     if (bad) atomicOr(err, 1u);
 }
 
 hipError_t launch_pack(const uint8_t* state, uint32_t* planes, const Geometry& g, uint32_t* err,
                        hipStream_t s)
 {
-    hipLaunchKernelGGL(pack_kernel, dim3(div_up(g.P, 256), g.dim_y), dim3(256), 0, s, state,
-                       planes, g, err);
+    const uint32_t qx = row_lanes(g.P);
+    const dim3 grid = row_grid(g, g.P, qx), block(qx, 256u / qx);
+    switch (g.Q) {
+    case 4: hipLaunchKernelGGL(pack_kernel<4>, grid, block, 0, s, state, planes, g, err); break;
+    case 6: hipLaunchKernelGGL(pack_kernel<6>, grid, block, 0, s, state, planes, g, err); break;
+    default: hipLaunchKernelGGL(pack_kernel<7>, grid, block, 0, s, state, planes, g, err); break;
+    }
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(256) void unpack_kernel(const uint32_t* __restrict__ planes,
-                                                     uint8_t* __restrict__ st, Geometry g)
+// Q planes per lattice row (a state's, or the two of a type mask) to bytes; null
+// planes are empty.  A lane writes 16 bytes that start at a multiple of 16 in
+// memory (at cells x..x + 15, from up to two words of a plane) in each of
+// kUnpackRows rows, all of whose words are in flight together.  Neighbouring
+// lanes, through the workgroup and on to the next one, take neighbouring
+// chunks: narrow workgroups over many rows read each 128-byte line of a plane
+// several times.
+constexpr uint32_t kUnpackRows = 4;
+
+template <int Q>
+__global__ __launch_bounds__(256) void unpack_kernel(const uint32_t* __restrict__ planes, uint8_t* __restrict__ st,
+                                                     Geometry g, uint32_t chunks, uint32_t slab)
 {
-    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t y = blockIdx.y;
-    if (w >= g.W) return;
-    uint32_t pl[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t d = 0; d < g.Q; ++d) pl[d] = planes[((size_t)y * g.Q + d) * g.P + w];
-    uint8_t* row = st + (size_t)y * g.dim_x;
-    for (uint32_t b = 0; b < 32; ++b) {
-        const uint32_t x = 32 * w + b;
-        if (x >= g.dim_x) break;
-        uint32_t v = 0;
+    // blockIdx.y picks a slab of row groups
+    const uint32_t id = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t group = id / chunks, i = id - group * chunks;
+    const uint32_t y0 = (blockIdx.y * slab + group) * kUnpackRows;
+    if (group >= slab || y0 >= g.dim_y) return;
+    uint32_t w[kUnpackRows][Q] = {}, n[kUnpackRows][Q] = {};
+    int32_t x[kUnpackRows];  // the lattice is narrower than 2^30 cells
 #pragma unroll
-        for (int d = 0; d < 8; ++d) v |= ((pl[d] >> b) & 1u) << d;
-        row[x] = (uint8_t)v;
+    for (uint32_t k = 0; k < kUnpackRows; ++k)
+        x[k] = (int32_t)(kCodecCells * i) - (int32_t)((uintptr_t)(st + (size_t)min(y0 + k, g.dim_y - 1) * g.dim_x) & 15u);
+    if (planes) {
+#pragma unroll
+        for (uint32_t k = 0; k < kUnpackRows; ++k) {
+            const uint32_t at = min((uint32_t)max(x[k], 0) >> 5, g.W - 1);
+            const uint32_t up = min((uint32_t)(x[k] + (int32_t)kCodecCells - 1) >> 5, g.W - 1);
+            const uint32_t* row = planes + (size_t)min(y0 + k, g.dim_y - 1) * Q * g.P;
+#pragma unroll
+            for (int d = 0; d < Q; ++d, row += g.P) {
+                w[k][d] = row[at];
+                n[k][d] = row[up];
+            }
+        }
     }
+#pragma unroll
+    for (uint32_t k = 0; k < kUnpackRows; ++k) {
+        const uint32_t y = y0 + k;
+        if (y >= g.dim_y || x[k] >= (int32_t)g.dim_x) continue;
+        // sixteen cells of each plane in the low half; a chunk that starts
+        // before the row has its first cells at the top of it
+        uint32_t pl[8] = {};
+#pragma unroll
+        for (int d = 0; d < Q; ++d)
+            pl[d] = x[k] < 0 ? w[k][d] << (uint32_t)-x[k] : __builtin_amdgcn_alignbit(n[k][d], w[k][d], (uint32_t)x[k]);
+        uint32_t c[4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            // byte h of every plane
+            const uint32_t two = h ? 0x0c0c0501u : 0x0c0c0400u;
+            c[2 * h] = __builtin_amdgcn_perm(pl[1], pl[0], two) | (__builtin_amdgcn_perm(pl[3], pl[2], two) << 16);
+            c[2 * h + 1] = __builtin_amdgcn_perm(pl[5], pl[4], two) | (__builtin_amdgcn_perm(pl[7], pl[6], two) << 16);
+            transpose8(c[2 * h], c[2 * h + 1]);
+        }
+        uint8_t* out = st + (size_t)y * g.dim_x;
+        if (x[k] >= 0 && x[k] + (int32_t)kCodecCells <= (int32_t)g.dim_x) {
+            *(u32x4*)(out + x[k]) = u32x4{c[0], c[1], c[2], c[3]};
+        } else {
+            const int32_t first = max(-x[k], 0), end = min((int32_t)kCodecCells, (int32_t)g.dim_x - x[k]);
+#pragma unroll 1
+            for (int32_t b = first; b < end; ++b) {
+                const uint32_t v = b < 8 ? (b < 4 ? c[0] : c[1]) : (b < 12 ? c[2] : c[3]);
+                out[x[k] + b] = (uint8_t)(v >> (8 * (b & 3)));
+            }
+        }
+    }
+}
+
+template <int Q>
+static hipError_t unpack_planes(const uint32_t* planes, uint8_t* out, const Geometry& g, hipStream_t s)
+{
+    const uint32_t chunks = div_up(g.dim_x + kCodecCells - 1, kCodecCells), groups = div_up(g.dim_y, kUnpackRows);
+    const uint32_t slab = std::min(groups, std::max(1u, (1u << 30) / chunks));
+    hipLaunchKernelGGL(unpack_kernel<Q>, dim3(div_up((uint64_t)chunks * slab, 256), div_up(groups, slab)), dim3(256), 0,
+                       s, planes, out, g, chunks, slab);
+    return hipGetLastError();
 }
 
 hipError_t launch_unpack(const uint32_t* planes, uint8_t* state, const Geometry& g, hipStream_t s)
 {
-    hipLaunchKernelGGL(unpack_kernel, dim3(div_up(g.W, 256), g.dim_y), dim3(256), 0, s, planes,
-                       state, g);
-    return hipGetLastError();
+    switch (g.Q) {
+    case 4: return unpack_planes<4>(planes, state, g, s);
+    case 6: return unpack_planes<6>(planes, state, g, s);
+    default: return unpack_planes<7>(planes, state, g, s);
+    }
 }
 
 // ------------------------------------------------------------- cell types
@@ -300,24 +432,41 @@ __global__ __launch_bounds__(256) void types_kernel(const uint8_t* __restrict__ 
                                                     int32_t* __restrict__ row_range, Geometry g,
                                                     uint32_t* err)
 {
-    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t y = blockIdx.y;
-    if (w >= g.P) return;
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t y = blockIdx.y * blockDim.y + threadIdx.y;
+    if (w >= g.P || y >= g.dim_y) return;
     uint32_t ns = 0, sl = 0, bad = 0;
     const uint8_t* row = types + (size_t)y * g.dim_x;
-    for (uint32_t b = 0; b < 32; ++b) {
-        const uint32_t x = 32 * w + b;
-        if (x >= g.dim_x) break;
-        const uint32_t t = row[x];
-        ns |= (uint32_t)(t == 1) << b;
-        sl |= (uint32_t)(t == 2) << b;
-        bad |= t > 2;
+#pragma unroll
+    for (uint32_t half = 0; half < 2; ++half) {
+        const uint32_t x = 32 * w + kCodecCells * half;
+        if (x + kCodecCells <= g.dim_x) {
+            const Bytes16 c = load_bytes16(row + x);
+            const uint32_t any = c.v[0] | c.v[1] | c.v[2] | c.v[3];
+            if (!any) continue;  // FLUID, as nearly all cells are
+            const uint32_t t1 = gather_bits(c, 0), t2 = gather_bits(c, 1);
+            if (!(any & 0xFCFCFCFCu) && !(t1 & t2)) {
+                ns |= t1 << (16 * half);
+                sl |= t2 << (16 * half);
+                continue;
+            }
+        }
+        for (uint32_t b = 0; b < kCodecCells && x + b < g.dim_x; ++b) {
+            const uint32_t t = row[x + b];
+            ns |= (uint32_t)(t == 1) << (16 * half + b);
+            sl |= (uint32_t)(t == 2) << (16 * half + b);
+            bad |= t > 2;
+        }
     }
     mask[((size_t)y * 2 + 0) * g.P + w] = ns;
     mask[((size_t)y * 2 + 1) * g.P + w] = sl;
     if (ns | sl) {
-        atomicMin(row_range + y, (int32_t)w);
-        atomicMax(row_range + g.dim_y + y, (int32_t)w + 1);
+        // one of a run of words with solid cells speaks for it at each end
+        const unsigned long long some = __ballot(true);
+        const uint32_t lane = (threadIdx.y * blockDim.x + threadIdx.x) & 63u, at = threadIdx.x & 63u;
+        const bool before = at && ((some >> (lane - 1u)) & 1ull), after = at + 1u < blockDim.x && lane < 63u && ((some >> (lane + 1u)) & 1ull);
+        if (!before) atomicMin(row_range + y, (int32_t)w);
+        if (!after) atomicMax(row_range + g.dim_y + y, (int32_t)w + 1);
     }
     if (bad) atomicOr(err, 1u);
 }
@@ -325,48 +474,32 @@ __global__ __launch_bounds__(256) void types_kernel(const uint8_t* __restrict__ 
 hipError_t launch_types(const uint8_t* types, uint32_t* mask, int32_t* row_range,
                         const Geometry& g, uint32_t* err, hipStream_t s)
 {
-    hipLaunchKernelGGL(types_kernel, dim3(div_up(g.P, 256), g.dim_y), dim3(256), 0, s, types,
-                       mask, row_range, g, err);
+    const uint32_t qx = row_lanes(g.P);
+    hipLaunchKernelGGL(types_kernel, row_grid(g, g.P, qx), dim3(qx, 256u / qx), 0, s, types, mask, row_range, g, err);
     return hipGetLastError();
-}
-
-__global__ __launch_bounds__(256) void types_unpack_kernel(const uint32_t* __restrict__ mask,
-                                                           uint8_t* __restrict__ types, Geometry g)
-{
-    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t y = blockIdx.y;
-    if (w >= g.W) return;
-    const uint32_t ns = mask ? mask[((size_t)y * 2 + 0) * g.P + w] : 0u;
-    const uint32_t sl = mask ? mask[((size_t)y * 2 + 1) * g.P + w] : 0u;
-    uint8_t* row = types + (size_t)y * g.dim_x;
-    for (uint32_t b = 0; b < 32; ++b) {
-        const uint32_t x = 32 * w + b;
-        if (x >= g.dim_x) break;
-        row[x] = (uint8_t)(((ns >> b) & 1u) | (((sl >> b) & 1u) << 1));
-    }
 }
 
 hipError_t launch_types_unpack(const uint32_t* mask, uint8_t* types, const Geometry& g,
                                hipStream_t s)
 {
-    hipLaunchKernelGGL(types_unpack_kernel, dim3(div_up(g.W, 256), g.dim_y), dim3(256), 0, s,
-                       mask, types, g);
-    return hipGetLastError();
+    return unpack_planes<2>(mask, types, g, s);
 }
 
 // ------------------------------------------------------------ hash fill
 // init_random (src/lattice.cpp:198-217) with the draw of cell (x, y),
 // direction d = philox({x>>2, y, d, 2})[x & 3] < thr, on FLUID cells only.
+// Bound by the hash, one call per four bits: 4100 x 2050, 38 -> 31 us with the
+// eight calls of a word in flight together and 32-bit comparisons.
 
 __global__ __launch_bounds__(256) void init_fill_kernel(uint32_t* __restrict__ planes,
                                                         const uint32_t* __restrict__ mask,
                                                         const uint8_t* __restrict__ region,
                                                         Geometry g, uint32_t key0, uint32_t key1,
-                                                        uint64_t thr)
+                                                        uint64_t thr, uint32_t planes_each)
 {
-    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t y = blockIdx.y;
-    if (w >= g.W) return;
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t y = blockIdx.y * blockDim.y + threadIdx.y;
+    if (w >= g.W || y >= g.dim_y) return;
     uint32_t fluid = valid_mask(g, w);
     if (mask)
         fluid &= ~(mask[((size_t)y * 2 + 0) * g.P + w] | mask[((size_t)y * 2 + 1) * g.P + w]);
@@ -379,8 +512,8 @@ __global__ __launch_bounds__(256) void init_fill_kernel(uint32_t* __restrict__ p
         }
         fluid &= sel;
     }
-    for (uint32_t d = 0; d < g.Q; ++d) {
-        const uint32_t word = fill_word(w, y, d, g.dim_x, key0, key1, thr);
+    for (uint32_t d = blockIdx.z * planes_each; d < min(g.Q, (blockIdx.z + 1) * planes_each); ++d) {
+        const uint32_t word = fill_word(w, y, d, key0, key1, thr);
         uint32_t* p = planes + ((size_t)y * g.Q + d) * g.P + w;
         *p = (word & fluid) | (*p & ~fluid);
     }
@@ -390,8 +523,16 @@ hipError_t launch_init_fill(uint32_t* planes, const uint32_t* mask, const uint8_
                             const Geometry& g, uint32_t key0, uint32_t key1, uint64_t thr,
                             hipStream_t s)
 {
-    hipLaunchKernelGGL(init_fill_kernel, dim3(div_up(g.W, 256), g.dim_y), dim3(256), 0, s, planes,
-                       mask, region, g, key0, key1, thr);
+    const uint32_t qx = row_lanes(g.W);
+    dim3 grid = row_grid(g, g.W, qx);
+    // A lane fills one plane's word while the lattice has few words, so that the
+    // last workgroups do not run alone (4100 x 2050: 31 us, 34 with a lane per
+    // word), and all planes' words above, reading the masks once (32768 x 8192:
+    // 650 us, 732 with a lane per plane).
+    const bool split = (uint64_t)grid.x * grid.y < 4096;
+    if (split) grid.z = g.Q;
+    hipLaunchKernelGGL(init_fill_kernel, grid, dim3(qx, 256u / qx), 0, s, planes, mask, region, g, key0, key1, thr,
+                       split ? 1u : g.Q);
     return hipGetLastError();
 }
 
@@ -403,12 +544,8 @@ hipError_t launch_init_fill(uint32_t* planes, const uint32_t* mask, const uint8_
 __device__ constexpr float kSin60 = 0.866025388240814208984375f;  // (float)sin(pi/3)
 
 template <int KIND>
-__device__ __forceinline__ void cell_values(const uint32_t* pl, uint32_t b, int& rho, float& mx,
-                                            float& my)
+__device__ __forceinline__ void cell_values(const uint32_t* s, int& rho, float& mx, float& my)
 {
-    uint32_t s[7];
-#pragma unroll
-    for (int d = 0; d < num_dir_of_kind(KIND); ++d) s[d] = (pl[d] >> b) & 1u;
     if (KIND == kHPP) {
         rho = (int)(s[0] + s[1] + s[2] + s[3]);
         mx = (float)((int)s[0] - (int)s[2]);
@@ -423,34 +560,50 @@ __device__ __forceinline__ void cell_values(const uint32_t* pl, uint32_t b, int&
     }
 }
 
+// A wave owns kFieldCells cells of a row, lane l the cells l and l + 64: the
+// planes' words are the same for the whole wave, so they are scalar loads whose
+// 64 bits select a lane's value, and each store covers 64 neighbouring cells.
+// Bound by the 12 bytes a cell that it writes: 4400 x 2200, 109 us with a lane
+// per word (stores 128 and 256 bytes apart), 21 us so.
+constexpr uint32_t kFieldCells = 128;
+
 template <int KIND>
 __global__ __launch_bounds__(256) void cell_fields_kernel(const uint32_t* __restrict__ planes,
                                                           Geometry g, float* __restrict__ dens,
                                                           float* __restrict__ mom)
 {
     constexpr int Q = num_dir_of_kind(KIND);
-    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t y = blockIdx.y;
-    if (w >= g.W) return;
-    uint32_t pl[7];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t x0 = kFieldCells * (4 * blockIdx.x + wave), y = blockIdx.y;
+    if (x0 >= g.dim_x) return;
+    uint64_t pl[Q][2];  // four words of every plane: the pitch is a multiple of four words
 #pragma unroll
-    for (int d = 0; d < Q; ++d) pl[d] = planes[((size_t)y * Q + d) * g.P + w];
-    for (uint32_t b = 0; b < 32; ++b) {
-        const uint32_t x = 32 * w + b;
-        if (x >= g.dim_x) break;
+    for (int d = 0; d < Q; ++d) {
+        const u32x4 v = ldq(planes + ((size_t)y * Q + d) * g.P + (x0 >> 5));
+        pl[d][0] = v.x | (uint64_t)v.y << 32;
+        pl[d][1] = v.z | (uint64_t)v.w << 32;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+        uint32_t s[Q];
+#pragma unroll
+        for (int d = 0; d < Q; ++d) s[d] = __builtin_amdgcn_inverse_ballot_w64(pl[d][k]) ? 1u : 0u;
         int rho;
         float mx, my;
-        cell_values<KIND>(pl, b, rho, mx, my);
+        cell_values<KIND>(s, rho, mx, my);
+        const uint32_t x = x0 + 64 * k + lane;
+        if (x >= g.dim_x) return;
         const size_t cell = (size_t)y * g.dim_x + x;
         if (dens) dens[cell] = (float)rho;
-        if (mom) { mom[2 * cell] = mx; mom[2 * cell + 1] = my; }
+        if (mom) ((float2*)mom)[cell] = make_float2(mx, my);
     }
 }
 
 hipError_t launch_cell_fields(int kind, const uint32_t* planes, const Geometry& g, float* density,
                               float* momentum, hipStream_t s)
 {
-    const dim3 grid(div_up(g.W, 256), g.dim_y);
+    const dim3 grid(div_up(g.dim_x, 4 * kFieldCells), g.dim_y);
     switch (kind) {
     case kHPP: hipLaunchKernelGGL(cell_fields_kernel<kHPP>, grid, dim3(256), 0, s, planes, g, density, momentum); break;
     case kFHP1: hipLaunchKernelGGL(cell_fields_kernel<kFHP1>, grid, dim3(256), 0, s, planes, g, density, momentum); break;
@@ -632,7 +785,10 @@ __global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __rest
     auto visit = [&](uint32_t x, uint32_t y) {
         int rho;
         float mx, my;
-        cell_values<KIND>(pl, x & 31u, rho, mx, my);
+        uint32_t b[7];
+#pragma unroll
+        for (int d = 0; d < Q; ++d) b[d] = (pl[d] >> (x & 31u)) & 1u;
+        cell_values<KIND>(b, rho, mx, my);
         sd += (float)rho;
         sx += mx;
         sy += my;
