@@ -7,6 +7,7 @@
 #include "lgca.h"
 
 #include "lgca_dev.hpp"
+#include "lgca_hostcopy.hpp"
 #include "lgca_kernels.hpp"
 
 #include <algorithm>
@@ -126,6 +127,7 @@ struct lgca_lattice {
     void* force_ws = nullptr;       // count-mode force: listed tries (count_force_bytes)
     size_t force_ws_bytes = 0;
     bool calls_on_device = false;   // the count-mode call counter lives in ctrl
+    HostCopier copier;              // large results to the host
     std::string err;
     std::mutex mu;
 };
@@ -338,6 +340,7 @@ extern "C" lgca_status lgca_destroy(lgca_lattice* h)
         if (h->pipe_exch) (void)hipFree(h->pipe_exch);
         if (h->pipe_ctr) (void)hipFree(h->pipe_ctr);
         for (hipEvent_t ev : h->trial_ev) (void)hipEventDestroy(ev);
+        h->copier.release();
         if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
     }
     delete h;
@@ -489,8 +492,8 @@ extern "C" lgca_status lgca_get_cell_types(lgca_lattice* h, uint8_t* host_types)
     lgca_status st = ensure_bytes(h);
     if (st) return st;
     HIPCHK(h, launch_types_unpack(h->mask, h->bytes, h->g, h->stream));
-    HIPCHK(h, hipMemcpyAsync(host_types, h->bytes, n, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const HostCopy copy{host_types, h->bytes, n};
+    HIPCHK(h, h->copier.run(&copy, 1, h->stream));
     return LGCA_OK;
 }
 
@@ -541,8 +544,8 @@ static lgca_status download_state(lgca_lattice* h, uint8_t* dst, hipMemcpyKind k
     lgca_status st = ensure_bytes(h);
     if (st) return st;
     HIPCHK(h, launch_unpack(h->state[h->cur], h->bytes, h->g, h->stream));
-    HIPCHK(h, hipMemcpyAsync(dst, h->bytes, n, kind, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const HostCopy copy{dst, h->bytes, n};
+    HIPCHK(h, h->copier.run(&copy, 1, h->stream));
     return check_pipe(h);
 }
 
@@ -1555,25 +1558,24 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
     DeviceGuard dg(h->device);
     const size_t n = (size_t)h->dim_x * h->dim_y;
     const size_t nc = (size_t)(h->dim_x / (2 * h->r)) * (h->dim_y / (2 * h->r));
+    HostCopy copies[4];
+    int n_copies = 0;
     if (cell_density || cell_momentum) {
         if (cell_density && !h->cell_density) HIPCHK(h, dalloc(&h->cell_density, n * 4));
         if (cell_momentum && !h->cell_momentum) HIPCHK(h, dalloc(&h->cell_momentum, n * 8));
-        HIPCHK(h, launch_cell_fields(h->kind, h->snap, h->g, cell_density ? h->cell_density : nullptr,
-                                     cell_momentum ? h->cell_momentum : nullptr, h->stream));
-        if (cell_density)
-            HIPCHK(h, hipMemcpyAsync(cell_density, h->cell_density, n * 4, hipMemcpyDeviceToHost, h->stream));
-        if (cell_momentum)
-            HIPCHK(h, hipMemcpyAsync(cell_momentum, h->cell_momentum, n * 8, hipMemcpyDeviceToHost, h->stream));
     }
     if (mean_density || mean_momentum) {
         lgca_status st = run_coarse(h);
         if (st) return st;
-        if (mean_density)
-            HIPCHK(h, hipMemcpyAsync(mean_density, h->mean_density, nc * 4, hipMemcpyDeviceToHost, h->stream));
-        if (mean_momentum)
-            HIPCHK(h, hipMemcpyAsync(mean_momentum, h->mean_momentum, nc * 8, hipMemcpyDeviceToHost, h->stream));
     }
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (cell_density || cell_momentum)
+        HIPCHK(h, launch_cell_fields(h->kind, h->snap, h->g, cell_density ? h->cell_density : nullptr,
+                                     cell_momentum ? h->cell_momentum : nullptr, h->stream));
+    if (cell_density) copies[n_copies++] = {cell_density, h->cell_density, n * 4};
+    if (cell_momentum) copies[n_copies++] = {cell_momentum, h->cell_momentum, n * 8};
+    if (mean_density) copies[n_copies++] = {mean_density, h->mean_density, nc * 4};
+    if (mean_momentum) copies[n_copies++] = {mean_momentum, h->mean_momentum, nc * 8};
+    HIPCHK(h, h->copier.run(copies, n_copies, h->stream));
     return LGCA_OK;
 }
 
@@ -1698,11 +1700,10 @@ extern "C" lgca_status lgca_save_checkpoint(lgca_lattice* h, const char* path)
     lgca_status st = ensure_bytes(h);
     if (st) return st;
     HIPCHK(h, launch_types_unpack(h->mask, h->bytes, h->g, h->stream));
-    HIPCHK(h, hipMemcpyAsync(types, h->bytes, n, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const HostCopy types_copy{types, h->bytes, n}, snap_copy{snap, h->bytes, n};
+    HIPCHK(h, h->copier.run(&types_copy, 1, h->stream));
     HIPCHK(h, launch_unpack(h->snap, h->bytes, h->g, h->stream));
-    HIPCHK(h, hipMemcpyAsync(snap, h->bytes, n, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    HIPCHK(h, h->copier.run(&snap_copy, 1, h->stream));
     if ((st = download_state(h, state, hipMemcpyDeviceToHost))) return st;
     CheckpointHeader hd{};
     std::memcpy(hd.magic, kCheckpointMagic, 8);

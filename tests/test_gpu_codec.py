@@ -88,3 +88,43 @@ def test_types_fill_and_fields(model, dx, dy):
     assert np.array_equal(lat.cell_density(), density)
     assert np.array_equal(lat.cell_momentum(), momentum.reshape(-1))
     lat.close()
+
+
+@pytest.mark.parametrize("dx,dy", [(1200, 1024), (2049, 3002), (4096, 2048)])
+def test_large_results_arrive_whole(dx, dy):
+    """Results on both sides of the size from which several threads copy them,
+    with a ragged last chunk, into ordinary and into pinned memory, twice into
+    the same arrays, and from two lattices on two threads at once."""
+    import threading
+    lats = [make(2, dx, dy), make(0, dx, dy)]
+    rng = np.random.default_rng(dx)
+    n = dx * dy
+    states = [rng.integers(0, 1 << Q[m], n, dtype=np.uint8) for m in (2, 0)]
+    types = (rng.random(n) < 0.1).astype(np.uint8)
+    bad = []
+
+    def check(lat, state, model):
+        from lgca_amd import _capi as capi
+        for _ in range(2):
+            lat.set_cell_types(types)
+            lat.set_state_u8(state)
+            lat.copy_data_to_output_buffer()
+            lat.post_process()
+            density, momentum = orc.cell_post_process(model, dx, dy, state)
+            pinned = torch.empty(n, dtype=torch.uint8).pin_memory()
+            capi.check(capi.lib().lgca_get_state_u8(lat.handle, pinned.data_ptr()), lat.handle)
+            for name, got, want in (("state", lat.get_state_u8(), state), ("pinned", pinned.numpy(), state),
+                                    ("types", lat.get_cell_types(), types), ("density", lat.cell_density(), density),
+                                    ("momentum", lat.cell_momentum(), momentum.reshape(-1))):
+                if not np.array_equal(got, want):
+                    bad.append((model, name))
+            state = state[::-1].copy()
+
+    threads = [threading.Thread(target=check, args=a) for a in zip(lats, states, (2, 0))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for lat in lats:
+        lat.close()
