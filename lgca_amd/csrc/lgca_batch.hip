@@ -817,9 +817,9 @@ uint32_t tile_rows_for(uint64_t wave_rows_total, uint32_t waves)
     return (uint32_t)th;
 }
 
-// Blocks of a job's k-step round: rows per block and blocks.
+// Blocks of a job's k-step round: rows per block, row tiles, blocks.
 struct JobBlocks {
-    uint32_t th, tiles, strips;
+    uint32_t th, tiles, blocks;
 };
 JobBlocks job_blocks(const Geometry& g, const Candidate& c, int k)
 {
@@ -831,7 +831,7 @@ JobBlocks job_blocks(const Geometry& g, const Candidate& c, int k)
     b.th = (g.dim_y + b.tiles - 1) / b.tiles;
     b.th += b.th & 1u;
     b.tiles = (g.dim_y + b.th - 1) / b.th;
-    b.strips = seg ? 1 : tile_strips(g, k);
+    b.blocks = (uint32_t)block_count(g, k, b.tiles);
     return b;
 }
 
@@ -856,7 +856,7 @@ float mix_round_us(const lgca_batch* b, const Candidate& c)
             bw += w;
             bl += 0.08f + std::max(w, chain);
         }
-        const float blocks = (float)n.tiles * (float)n.strips;
+        const float blocks = (float)n.blocks;
         work += blocks * bw;
         wait += blocks * (bl - bw + 1.5f);
         most = std::max(most, bl);
@@ -946,12 +946,22 @@ void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th, const C
             const uint64_t key = g.nb != 32 ? 1u : 0u;
             std::vector<WorkItem>& vh = cls[key];
             std::vector<WorkItem>& vl = light[key];
-            const uint32_t bits = block_shape_bits(n.th, halo, (uint32_t)k, seg);
-            for (uint32_t t = 0; t < n.tiles; ++t) {
-                const int64_t y0 = (int64_t)t * n.th, rows = std::min<int64_t>(n.th, g.dim_y - y0);
-                std::vector<WorkItem>& v = rows_heavy(j, y0 - k, y0 + rows + k) ? vh : vl;
-                for (uint32_t st = 0; st < n.strips; ++st)
-                    v.push_back(WorkItem{(uint32_t)j->slot, st, t, bits, n.tiles * n.strips});
+            const BlockLanes lanes = block_lanes(g, k);
+            const uint32_t bits = block_shape_bits(n.th, halo, (uint32_t)k, lanes);
+            const uint32_t per_tile = lanes == kLanesPacked ? 1u : n.blocks / n.tiles;
+            const uint64_t span = g.W + 2 * halo, stride = 64 - 2 * halo;
+            for (uint32_t i = 0; i < n.blocks; ++i) {
+                // the row tiles of block i
+                uint64_t t0 = i / per_tile, t1 = t0;
+                if (lanes == kLanesPacked) {
+                    t0 = (i * stride) / span;
+                    t1 = std::min<uint64_t>(n.tiles - 1, (i * stride + stride - 1) / span);
+                }
+                const int64_t y0 = (int64_t)t0 * n.th, y1 = std::min<int64_t>((int64_t)(t1 + 1) * n.th, g.dim_y);
+                std::vector<WorkItem>& v = rows_heavy(j, y0 - k, y1 + k) ? vh : vl;
+                const WorkItem item = lanes == kLanesPacked ? WorkItem{(uint32_t)j->slot, i, 0u, bits, n.blocks}
+                                                            : WorkItem{(uint32_t)j->slot, i % per_tile, (uint32_t)t0, bits, n.blocks};
+                v.push_back(item);
             }
             continue;
         }

@@ -11,8 +11,8 @@
 // one barrier per step.  The state crosses HBM once per pass.  Each lattice's
 // best walk against its best blocks, us per step: 256 x 256 HPP 0.78 -> 0.24,
 // 1001 x 754 FHP-I slip box 3.06 -> 0.82, 2048 x 512 FHP-II pipe 3.05 -> 1.13,
-// 4400 x 2200 FHP-III cylinder 5.2 -> 2.4, 6000 x 3000 FHP-II forced channel
-// 8.0 -> 5.4 (2.0 of it the force draws).
+// 4400 x 2200 FHP-III cylinder 5.2 -> 2.0, 6000 x 3000 FHP-II forced channel
+// 8.0 -> 4.3 (1.2 of it the force draws).
 //
 // What bounds it: on the small ones the launch and the first loads (3 us a
 // pass) and each step's chain of dependent instructions through one barrier;
@@ -24,7 +24,13 @@
 // compile time).  The rows that the stored ones still depend on shrink by one on
 // either side per step; waves with none of them left only keep the barrier.
 // x-halo: as in lgca_tile.hpp (strips of 64 words with `halo` words either
-// side that are not stored; whole rows in segment mode).
+// side that are not stored; whole rows in segment mode), or packed: the row
+// tiles' words, `halo` either side of each tile's row included, form one
+// sequence, and a wave takes 64 of it, so that the end of one tile's rows
+// shares a wave with the start of the next one's.  Neighbours in the sequence
+// are neighbours in the row except at the halos' outer ends, where strips have
+// the same garbage.  A 188-word row takes 3.06 waves so, and 4 strips: 6000 x
+// 3000 FHP-II 3.2 -> 2.5 us a step, 4400 x 2200 (138 words) 2.4 -> 2.0.
 //
 // Chirality: a row's Philox call serves its word for a group of four steps;
 // the words wait in LDS (read once a step), which costs no registers and no
@@ -34,6 +40,9 @@
 #include "lgca_tile.hpp"
 
 namespace lgca {
+
+// A further segment mode, of blocks only: packed strips.
+constexpr int kPacked = 3;
 
 // The shifts of lgca_tile.hpp for words whose bits past the row's end may hold
 // anything (they are cleared once, before the store): the last word takes its
@@ -48,8 +57,9 @@ __device__ __forceinline__ uint32_t block_shift_p1(uint32_t v, const LaneCtx& c,
     return bit3<kMux>(last_bit, R << (c.nb - 1u), o);
 }
 
-// One workgroup's block: strip `strip` of row tile `tile`, k steps with hk halo
-// rows.  FEAT: 0 no solids and no forcing on the lattice, 1 either.  Every
+// One workgroup's block: strip `strip` of row tile `tile` (packed: `strip`
+// counts the waves' shares of the sequence, and `tile` is unused), k steps with
+// hk halo rows.  FEAT: 0 no solids and no forcing on the lattice, 1 either.  Every
 // wave of the workgroup makes k + 1 barriers.
 template <int KIND, int M, bool RAGGED, int SEG, int FEAT>
 __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32_t hk, uint32_t strip, uint32_t tile,
@@ -57,18 +67,31 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
 {
     constexpr int Q = num_dir_of_kind(KIND);
     constexpr uint32_t NX = KIND == kHPP ? 1 : 2;  // planes exchanged per direction
+    constexpr bool kRows = SEG != kStrips;                    // rows differ from lane to lane
+    constexpr bool kStacked = kRows && SEG != kPacked;        // segments hold one above the other
+    constexpr int SHIFT = SEG == kPacked ? kStrips : SEG;     // where neighbouring words are
     const Geometry& g = a.g;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwave = blockDim.x >> 6;
-    const uint32_t y0 = tile * a.th, rows = min(a.th, g.dim_y - y0);
+    uint32_t y0 = tile * a.th, rows = min(a.th, g.dim_y - y0);  // packed: this lane's
 
     // this lane's word and the group of M rows it works on
-    const uint32_t S = SEG ? 64u / g.W : 1u;
+    const uint32_t S = kStacked ? 64u / g.W : 1u;
     uint32_t group = wave;
     int wabs;
     bool writer;
     LaneCtx c;
-    if (SEG) {
+    if (SEG == kPacked) {
+        const uint32_t stride = 64u - 2u * a.halo, span = g.W + 2u * a.halo;
+        const uint32_t total = (g.dim_y + a.th - 1) / a.th * span;
+        const int f = (int)(strip * stride) - (int)a.halo + (int)lane;
+        const uint32_t at = (uint32_t)min(max(f, 0), (int)total - 1), t = at / span;
+        y0 = t * a.th;
+        rows = min(a.th, g.dim_y - y0);
+        wabs = (int)(at - t * span) - (int)a.halo;
+        writer = lane >= a.halo && lane < 64u - a.halo && f < (int)total && wabs >= 0 && wabs < (int)g.W;
+        c.lsrc = c.rsrc = 0;
+    } else if (SEG) {
         const uint32_t seg = lane / g.W, base = seg * g.W;
         group = wave * S + min(seg, S - 1u);
         wabs = (int)(lane - base);
@@ -100,13 +123,14 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
         else if (r >= dy) r -= dy;
         if (r < 0 || r >= dy) r = (r % dy + dy) % dy;  // (blocks taller than the lattice)
         j[m] = (uint32_t)r;
-        if (!SEG) j[m] = __builtin_amdgcn_readfirstlane(j[m]);
+        if (!kRows) j[m] = __builtin_amdgcn_readfirstlane(j[m]);
     }
     // The stored rows depend on rows [hk - left, hk + rows + left) of the block
     // with `left` steps to go: the wave works on its rows [wave_lo, wave_hi)
     // for the pass's first `act` steps.
     const int wave_lo = (int)(wave * S * M), wave_hi = wave_lo + (int)(S * M);
-    const int idle = max(0, max(wave_lo - (int)(hk + rows) + 1, (int)hk - wave_hi + 1));
+    const uint32_t most = SEG == kPacked ? a.th : rows;
+    const int idle = max(0, max(wave_lo - (int)(hk + most) + 1, (int)hk - wave_hi + 1));
     const int act = (int)k - idle;
     const bool work = act >= 0;  // (at 0 its initial planes are still read)
 
@@ -123,12 +147,12 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
     // row's; in segment mode rows differ per lane.
     const uint32_t fplane_b = (a.fy1 - a.fy0) * a.fwn * 4u;
     const bool fcol = c.w >= a.fw0 && c.w < a.fw0 + a.fwn;
-    uint32_t foff[SEG ? M : 1];
-    if (!SEG) foff[0] = fcol ? (c.w - a.fw0) * 4u : kOutside;
+    uint32_t foff[kRows ? M : 1];
+    if (!kRows) foff[0] = fcol ? (c.w - a.fw0) * 4u : kOutside;
     auto frow = [&](int m) { return j[m] >= a.fy0 && j[m] < a.fy1; };
     auto load_force = [&](int m, uint32_t step) {
-        const uint32_t off = SEG ? foff[SEG ? m : 0] : (frow(m) ? foff[0] : kOutside);
-        const uint32_t row = !SEG && frow(m) ? (j[m] - a.fy0) * a.fwn * 4u : 0u;
+        const uint32_t off = kRows ? foff[kRows ? m : 0] : (frow(m) ? foff[0] : kOutside);
+        const uint32_t row = !kRows && frow(m) ? (j[m] - a.fy0) * a.fwn * 4u : 0u;
         return bload(make_rsrc(a.fdec, k * fplane_b), off, step * fplane_b + row);
     };
     if (work) {
@@ -136,14 +160,14 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
         for (int m = 0; m < M; ++m)
 #pragma unroll
             for (int d = 0; d < Q; ++d)
-                s[m][d] = SEG ? bload(make_rsrc(a.src, g.dim_y * row_b), j[m] * row_b + c.wb, (uint32_t)d * plane_b)
+                s[m][d] = kRows ? bload(make_rsrc(a.src, g.dim_y * row_b), j[m] * row_b + c.wb, (uint32_t)d * plane_b)
                               : bload(make_rsrc(a.src + (size_t)j[m] * Q * g.P, row_b), c.wb, (uint32_t)d * plane_b);
         if (FEAT) {
             if (a.fdec) {
                 bool any = false;
 #pragma unroll
                 for (int m = 0; m < M; ++m) {
-                    if (SEG) foff[SEG ? m : 0] = fcol && frow(m) ? ((j[m] - a.fy0) * a.fwn + (c.w - a.fw0)) * 4u : kOutside;
+                    if (kRows) foff[kRows ? m : 0] = fcol && frow(m) ? ((j[m] - a.fy0) * a.fwn + (c.w - a.fw0)) * 4u : kOutside;
                     any |= fcol && frow(m);
                 }
                 forced = __builtin_amdgcn_ballot_w64(any) != 0;
@@ -157,9 +181,9 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
                 const uint32_t mrow_b = 2u * plane_b;
 #pragma unroll
                 for (int m = 0; m < M; ++m) {
-                    const uint32_t* row = a.mask + (SEG ? (size_t)0 : (size_t)j[m] * 2 * g.P);
-                    const __amdgpu_buffer_rsrc_t r = make_rsrc(row, SEG ? g.dim_y * mrow_b : mrow_b);
-                    const uint32_t off = (SEG ? j[m] * mrow_b : 0u) + c.wb;
+                    const uint32_t* row = a.mask + (kRows ? (size_t)0 : (size_t)j[m] * 2 * g.P);
+                    const __amdgpu_buffer_rsrc_t r = make_rsrc(row, kRows ? g.dim_y * mrow_b : mrow_b);
+                    const uint32_t off = (kRows ? j[m] * mrow_b : 0u) + c.wb;
                     ns[m] = bload(r, off, 0);
                     sl[m] = bload(r, off, plane_b);
                 }
@@ -184,7 +208,7 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
     // (those rows are not needed)
     uint32_t above = wave > 0 ? wave - 1u : 0u, below = wave + 1u < nwave ? wave + 1u : wave;
     uint32_t alane = lane, blane = lane;
-    if (SEG) {
+    if (kStacked) {
         const uint32_t seg = min(lane / g.W, S - 1u);
         if (seg > 0) { above = wave; alane = lane - g.W; }
         else alane = lane + (S - 1u) * g.W;
@@ -233,28 +257,28 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
         for (int m = 0; m < M; ++m) {
             uint32_t in[7], st[7];
             if (KIND == kHPP) {
-                in[0] = shift_m1<RAGGED, SEG>(s[m][0], c);
+                in[0] = shift_m1<RAGGED, SHIFT>(s[m][0], c);
                 in[1] = p1;
-                in[2] = block_shift_p1<RAGGED, SEG>(s[m][2], c, last_bit);
+                in[2] = block_shift_p1<RAGGED, SHIFT>(s[m][2], c, last_bit);
                 in[3] = m + 1 < M ? s[m + 1 < M ? m + 1 : 0][3] : n4;
                 p1 = s[m][1];
             } else {
                 const uint32_t r4 = m + 1 < M ? s[m + 1 < M ? m + 1 : 0][4] : n4;
                 const uint32_t r5 = m + 1 < M ? s[m + 1 < M ? m + 1 : 0][5] : n5;
-                in[0] = shift_m1<RAGGED, SEG>(s[m][0], c);
-                in[3] = block_shift_p1<RAGGED, SEG>(s[m][3], c, last_bit);
+                in[0] = shift_m1<RAGGED, SHIFT>(s[m][0], c);
+                in[3] = block_shift_p1<RAGGED, SHIFT>(s[m][3], c, last_bit);
                 if (Q == 7) in[6] = s[m][Q - 1];
                 auto odd_row = [&] {
                     in[1] = p1;
-                    in[2] = block_shift_p1<RAGGED, SEG>(p2, c, last_bit);
-                    in[4] = block_shift_p1<RAGGED, SEG>(r4, c, last_bit);
+                    in[2] = block_shift_p1<RAGGED, SHIFT>(p2, c, last_bit);
+                    in[4] = block_shift_p1<RAGGED, SHIFT>(r4, c, last_bit);
                     in[5] = r5;
                 };
                 auto even_row = [&] {
-                    in[1] = shift_m1<RAGGED, SEG>(p1, c);
+                    in[1] = shift_m1<RAGGED, SHIFT>(p1, c);
                     in[2] = p2;
                     in[4] = r4;
-                    in[5] = shift_m1<RAGGED, SEG>(r5, c);
+                    in[5] = shift_m1<RAGGED, SHIFT>(r5, c);
                 };
                 if (M % 2 == 0) {  // blocks start on even rows
                     if (m & 1) odd_row();
@@ -335,11 +359,11 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
         for (int m = 0; m < M; ++m) {
             const uint32_t l = group * M + m;
             const bool wr = writer && l >= hk && l < hk + rows;
-            if (!SEG && !(l >= hk && l < hk + rows)) continue;  // wave-uniform
+            if (!kStacked && !(l >= hk && l < hk + most)) continue;  // wave-uniform
 #pragma unroll
             for (int d = 0; d < Q; ++d) {
                 if (RAGGED) s[m][d] &= c.vmask;
-                if (SEG) bstore(s[m][d], make_rsrc(a.dst, g.dim_y * row_b), wr ? j[m] * row_b + c.wb : kOutside, (uint32_t)d * plane_b);
+                if (kRows) bstore(s[m][d], make_rsrc(a.dst, g.dim_y * row_b), wr ? j[m] * row_b + c.wb : kOutside, (uint32_t)d * plane_b);
                 else bstore(s[m][d], make_rsrc(a.dst + (size_t)j[m] * Q * g.P, row_b), wr ? c.wb : kOutside, (uint32_t)d * plane_b);
             }
         }
@@ -386,21 +410,24 @@ void block_batch_kernel(const BatchJob* __restrict__ jobs, BatchState* state, co
     TileArgs a = jobs[it.job].a;
     a.t0 = bs.step;
     a.th = it.shape & 0xFFFFu;
-    a.halo = (it.shape >> 16) & 0xFFu;
+    a.halo = (it.shape >> 16) & 0x7Fu;
     a.src = bs.cur ? jobs[it.job].buf1 : jobs[it.job].buf0;
     a.dst = bs.cur ? jobs[it.job].buf0 : jobs[it.job].buf1;
     if (a.fdec) a.fdec += (size_t)(bs.step - bs.fdec_step0) * a.fdec_stride;
     const uint32_t k = (it.shape >> 24) & 0x7Fu, hk = block_halo(M, k);
-    const bool seg = (it.shape >> 31) != 0;
+    const bool seg = (it.shape >> 31) != 0, packed = ((it.shape >> 23) & 1u) != 0;
     const uint32_t Q = __builtin_amdgcn_readfirstlane(a.g.Q);
     if (Q == 4) {
         if (seg) block_body<kHPP, M, RAGGED, kSegments, 1>(a, k, hk, it.strip, it.tile, block_lds);
+        else if (packed) block_body<kHPP, M, RAGGED, kPacked, 1>(a, k, hk, it.strip, it.tile, block_lds);
         else block_body<kHPP, M, RAGGED, kStrips, 1>(a, k, hk, it.strip, it.tile, block_lds);
     } else if (Q == 6) {
         if (seg) block_body<kFHP1, M, RAGGED, kSegments, 1>(a, k, hk, it.strip, it.tile, block_lds);
+        else if (packed) block_body<kFHP1, M, RAGGED, kPacked, 1>(a, k, hk, it.strip, it.tile, block_lds);
         else block_body<kFHP1, M, RAGGED, kStrips, 1>(a, k, hk, it.strip, it.tile, block_lds);
     } else {
         if (seg) block_body<kFHP2, M, RAGGED, kSegments, 1>(a, k, hk, it.strip, it.tile, block_lds);
+        else if (packed) block_body<kFHP2, M, RAGGED, kPacked, 1>(a, k, hk, it.strip, it.tile, block_lds);
         else block_body<kFHP2, M, RAGGED, kStrips, 1>(a, k, hk, it.strip, it.tile, block_lds);
     }
     // The job's last workgroup of the round advances it.  Every wave of every
@@ -428,10 +455,12 @@ hipError_t launch_block_km(const BlockArgs& b, uint32_t waves, uint32_t blocks, 
         else hipLaunchKernelGGL((block_kernel<KIND, M, RG, SG, 0>), grid, block, lds, s, b);             \
     } while (0)
     if (ragged) {
-        if (seg) LGCA_BLOCK_LAUNCH(true, kSegments);
+        if (seg == kPacked) LGCA_BLOCK_LAUNCH(true, kPacked);
+        else if (seg) LGCA_BLOCK_LAUNCH(true, kSegments);
         else LGCA_BLOCK_LAUNCH(true, kStrips);
     } else {
-        if (seg == kWholeRow) LGCA_BLOCK_LAUNCH(false, kWholeRow);
+        if (seg == kPacked) LGCA_BLOCK_LAUNCH(false, kPacked);
+        else if (seg == kWholeRow) LGCA_BLOCK_LAUNCH(false, kWholeRow);
         else if (seg) LGCA_BLOCK_LAUNCH(false, kSegments);
         else LGCA_BLOCK_LAUNCH(false, kStrips);
     }

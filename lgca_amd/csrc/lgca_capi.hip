@@ -1086,7 +1086,9 @@ static hipError_t launch_block_pass(lgca_lattice* h, uint32_t k, const BlockShap
     b.a.t0 = t0;
     b.k = k;
     b.hk = block_halo(s.m, k);
-    b.nstrips = tile_segments(h->g, (int)k) ? 1 : tile_strips(h->g, (int)k);
+    const uint32_t tiles = (h->dim_y + s.th - 1) / s.th;
+    const uint64_t blocks = block_count(h->g, (int)k, tiles);
+    b.nstrips = (uint32_t)(block_lanes(h->g, (int)k) == kLanesPacked ? blocks : blocks / tiles);
     return launch_block(h->kind, s, b, h->stream);
 }
 

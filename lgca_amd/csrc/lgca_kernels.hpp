@@ -148,8 +148,14 @@ struct BlockArgs {
     TileArgs a;        // a.th: rows a block stores (even)
     uint32_t k;        // steps of the pass
     uint32_t hk;       // halo rows either side, >= k, even unless m is 1
-    uint32_t nstrips;  // x-strips (1 in segment mode)
+    uint32_t nstrips;  // x-strips (1 in segment mode; packed: all the pass's blocks)
 };
+// How the row tiles of a block pass share out the lanes (segment modes of
+// lgca_tile.hpp and lgca_block.hpp): whole rows, strips, or packed strips.
+enum BlockLanes { kLanesRows, kLanesStrips, kLanesPacked };
+BlockLanes block_lanes(const Geometry& g, int k);
+// Workgroups of a pass over `tiles` row tiles.
+uint64_t block_count(const Geometry& g, int k, uint32_t tiles);
 // Shape of a pass: m rows per wave and segment, `waves` waves per workgroup, th
 // stored rows per block.
 struct BlockShape {
@@ -206,9 +212,9 @@ hipError_t launch_block_batch(uint32_t m, uint32_t waves, bool ragged, const Bat
 template <int M>
 hipError_t launch_block_batch_m(const BatchJob* jobs, BatchState* state, const WorkItem* items, uint32_t n_items,
                                 uint32_t n_heavy, uint32_t waves, bool ragged, hipStream_t s);
-inline uint32_t block_shape_bits(uint32_t th, uint32_t halo, uint32_t k, bool seg)
+inline uint32_t block_shape_bits(uint32_t th, uint32_t halo, uint32_t k, BlockLanes lanes)
 {
-    return th | (halo << 16) | (k << 24) | (seg ? 1u << 31 : 0u);
+    return th | (halo << 16) | (lanes == kLanesPacked ? 1u << 23 : 0u) | (k << 24) | (lanes == kLanesRows ? 1u << 31 : 0u);
 }
 hipError_t launch_tile_batch(int k, bool ragged, const BatchJob* jobs, BatchState* state,
                              const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s);

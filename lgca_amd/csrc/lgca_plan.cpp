@@ -204,17 +204,40 @@ uint32_t block_lds_bytes(int kind, uint32_t m, uint32_t waves)
     return waves * 64u * 4u * (kind == 0 ? 4u : 8u + 4u * m);
 }
 
-// Lattices whose walks the fixed rule gives 2-row tiles, about 25 wave-rows (64
-// words of a row) per SIMD.  FHP-II on
-// torus lattices, us per step in blocks / walked: 2048 x 1024 1.02 / 2.06,
-// 4400 x 2200 1.93 / 3.90, 8192 x 4096 (20,480 wave-rows) 4.05 / 4.93, 16384 x
-// 4096 (36,864) 6.85 / 6.82, 32768 x 8192 22 / 19: the larger ones fill the
-// GPU with walks, which read and compute fewer halo rows.
+// Packed strips where rows of more than half a wave leave lanes of their
+// strips idle: their rows differ per lane, which costs three instructions a
+// Philox call, so from 3 % fewer waves on.  (Their row offsets are lane
+// offsets, below 2 GiB.)  Shorter rows stack 64 / W segments, whose blocks are
+// that much taller.
+BlockLanes block_lanes(const Geometry& g, int k)
+{
+    if (tile_segments(g, k)) return kLanesRows;
+    const uint64_t h = tile_halo(g, k), span = g.W + 2 * h, stride = 64 - 2 * h;
+    const bool fits = (uint64_t)g.dim_y * g.Q * g.P * 4 < ((uint64_t)1 << 31);
+    return fits && g.W > 32 && span * 100 <= 97 * stride * tile_strips(g, k) ? kLanesPacked : kLanesStrips;
+}
+
+uint64_t block_count(const Geometry& g, int k, uint32_t tiles)
+{
+    switch (block_lanes(g, k)) {
+    case kLanesRows: return tiles;
+    case kLanesStrips: return (uint64_t)tiles * tile_strips(g, k);
+    default: break;
+    }
+    const uint64_t h = tile_halo(g, k), stride = 64 - 2 * h;
+    return ((uint64_t)tiles * (g.W + 2 * h) + stride - 1) / stride;
+}
+
+// Lattices of up to 32 wave-rows (64 words of a row, packed as the blocks have
+// them) per SIMD.  us per step in blocks / walked, FHP-II: 4400 x 2200 1.9 /
+// 3.9, 8192 x 4096 (17,045 wave-rows) 3.6 / 5.3, 12000 x 4000 (24,323) 5.6 /
+// 6.3, 16384 x 4096 (33,957) 6.6 / 6.9, 32768 x 2048 (33,891) 6.8 / 6.6, 16384 x
+// 8192 (67,914) 12.6 / 10.5: the larger ones fill the GPU with walks, which
+// read and compute fewer halo rows.
 bool block_lattice(const Geometry& g)
 {
-    const bool seg = tile_segments(g, 8);
-    const uint64_t wave_rows = seg ? (uint64_t)g.dim_y / (64 / g.W) : (uint64_t)g.dim_y * tile_strips(g, 8);
-    return wave_rows < 3 * 8704;
+    const uint64_t wave_rows = tile_segments(g, 8) ? (uint64_t)g.dim_y / (64 / g.W) : block_count(g, 8, g.dim_y);
+    return wave_rows < 32768;
 }
 
 std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k)
@@ -246,7 +269,7 @@ float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32
     const bool seg = tile_segments(g, (int)k);
     const uint32_t S = seg ? 64 / g.W : 1, held = s.m * s.waves * S, hk = block_halo(s.m, k);
     if (!k || !s.th || held < s.th + 2 * hk || (!seg && k > 32)) return -1.0f;
-    const uint64_t blocks = (uint64_t)((g.dim_y + s.th - 1) / s.th) * (seg ? 1 : tile_strips(g, (int)k));
+    const uint64_t blocks = block_count(g, (int)k, (g.dim_y + s.th - 1) / s.th);
     // workgroups a CU holds: 128 registers allow 16 waves, half of them 32
     const uint32_t waves_cu = feat && s.m > 2 ? 16 : 32;
     const uint32_t fit = std::max(1u, std::min(waves_cu / s.waves, 160u * 1024u / block_lds_bytes(kind, s.m, s.waves)));

@@ -74,10 +74,10 @@ hipError_t launch_block(int kind, const BlockShape& sh, const BlockArgs& b, hipS
         return hipErrorInvalidValue;
     if (!seg && (b.a.halo < tile_halo(g, (int)b.k) || b.a.halo > 16 || b.k > 32)) return hipErrorInvalidValue;
     if (b.a.fdec && (uint64_t)b.k * b.a.fdec_stride * 4u >= ((uint64_t)1 << 31)) return hipErrorInvalidValue;
-    const uint64_t blocks = (uint64_t)((g.dim_y + b.a.th - 1) / b.a.th) * b.nstrips;
-    if (blocks >= ((uint64_t)1 << 31)) return hipErrorInvalidValue;
+    const uint64_t blocks = block_count(g, (int)b.k, (g.dim_y + b.a.th - 1) / b.a.th);
+    if (blocks >= ((uint64_t)1 << 31) || blocks % b.nstrips) return hipErrorInvalidValue;
     const bool ragged = g.nb != 32;
-    const int seg_mode = !seg ? 0 : (g.W == 64 && !ragged) ? 2 : 1;
+    const int seg_mode = block_lanes(g, (int)b.k) == kLanesPacked ? 3 : !seg ? 0 : (g.W == 64 && !ragged) ? 2 : 1;
 #define LGCA_BLOCK_CASE(KD, MM) \
     if (kind == KD && m == MM) return launch_block_km<KD, MM>(b, waves, (uint32_t)blocks, ragged, seg_mode, s);
     LGCA_BLOCK_CASE(kHPP, 1) LGCA_BLOCK_CASE(kHPP, 2) LGCA_BLOCK_CASE(kHPP, 4)

@@ -122,3 +122,18 @@ def test_batch_blocks_match_the_oracle():
         assert b.stats()["wave_target"] <= 16  # waves per workgroup: the rounds ran in blocks
         for i, w in zip(ids, want):
             np.testing.assert_array_equal(b.result(i)[0], w)
+
+
+# rows that share waves with the next row tile's: widths whose rows end within,
+# at and past a wave's words, short last words with one and two halo words,
+# heights whose last tile is short or the only one, every kind of cell and
+# force, and lattices large enough for each number of rows per wave
+@pytest.mark.parametrize("case", [
+    (2, 1100, 130, "slip", dict(dir="y", p=0.05)), (1, 1056, 64, None, None), (0, 1057, 63, "mixed", dict(dir="x", p=0.1)),
+    (2, 1969, 200, "pipe", dict(dir="x", p=0.1)), (3, 2050, 46, "mixed", dict(dir="x", p=0.2)),
+    (1, 4017, 500, "cylinder", dict(dir="x", p=0.05, x0=0, x1=64)), (2, 4400, 740, "pipe", dict(dir="x", p=0.01)),
+    (0, 2700, 1001, "slip", None), (2, 6000, 1500, "cylinder", dict(dir="x", p=0.01)), (1, 4400, 2200, None, None),
+    (3, 2177, 2, "pipe", None), (2, 6000, 3000, "pipe", dict(dir="y", p=0.01))], ids=lambda c: f"m{c[0]}_{c[1]}x{c[2]}")
+@pytest.mark.parametrize("tune", [False, True])
+def test_rows_packed_into_waves(case, tune):
+    check(*case, calls=(1, 3, 26), step0=2, tune=tune)
