@@ -44,19 +44,6 @@ namespace lgca {
 // A further segment mode, of blocks only: packed strips.
 constexpr int kPacked = 3;
 
-// The shifts of lgca_tile.hpp for words whose bits past the row's end may hold
-// anything (they are cleared once, before the store): the last word takes its
-// cell nb - 1 from the first word's cell 0 by a bit select.  last_bit: bit
-// nb - 1 on the lane holding word W - 1, else 0.
-template <bool RAGGED, int SEG>
-__device__ __forceinline__ uint32_t block_shift_p1(uint32_t v, const LaneCtx& c, uint32_t last_bit)
-{
-    const uint32_t R = right_word<SEG>(v, c);
-    const uint32_t o = __builtin_amdgcn_alignbit(R, v, 1);
-    if (!RAGGED) return o;
-    return bit3<kMux>(last_bit, R << (c.nb - 1u), o);
-}
-
 // One workgroup's block: strip `strip` of row tile `tile` (packed: `strip`
 // counts the waves' shares of the sequence, and `tile` is unused), k steps with
 // hk halo rows.  FEAT: 0 no solids and no forcing on the lattice, 1 either.  Every
@@ -108,9 +95,9 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
     c.wb = 4u * c.w;
     c.nb = g.nb;
     c.first_shl = c.w == 0 ? 32u - g.nb : 0u;
-    c.last = c.w + 1 == g.W;
-    c.vmask = (c.last && g.nb < 32) ? ((1u << g.nb) - 1u) : 0xFFFFFFFFu;
-    const uint32_t last_bit = c.last ? 1u << (g.nb - 1u) : 0u;
+    const uint32_t last_bit = c.w + 1 == g.W ? 1u << (g.nb - 1u) : 0u;
+    c.last_bit = last_bit;
+    c.vmask = (last_bit && g.nb < 32) ? ((1u << g.nb) - 1u) : 0xFFFFFFFFu;
     const uint32_t edge = (c.w == 0 ? 1u : 0u) | last_bit;  // this lane's cells on the east / west columns
 
     // rows of the lattice behind the lane's M rows
@@ -259,19 +246,19 @@ __device__ __forceinline__ void block_body(const TileArgs& a, uint32_t k, uint32
             if (KIND == kHPP) {
                 in[0] = shift_m1<RAGGED, SHIFT>(s[m][0], c);
                 in[1] = p1;
-                in[2] = block_shift_p1<RAGGED, SHIFT>(s[m][2], c, last_bit);
+                in[2] = shift_p1<RAGGED, SHIFT>(s[m][2], c);
                 in[3] = m + 1 < M ? s[m + 1 < M ? m + 1 : 0][3] : n4;
                 p1 = s[m][1];
             } else {
                 const uint32_t r4 = m + 1 < M ? s[m + 1 < M ? m + 1 : 0][4] : n4;
                 const uint32_t r5 = m + 1 < M ? s[m + 1 < M ? m + 1 : 0][5] : n5;
                 in[0] = shift_m1<RAGGED, SHIFT>(s[m][0], c);
-                in[3] = block_shift_p1<RAGGED, SHIFT>(s[m][3], c, last_bit);
+                in[3] = shift_p1<RAGGED, SHIFT>(s[m][3], c);
                 if (Q == 7) in[6] = s[m][Q - 1];
                 auto odd_row = [&] {
                     in[1] = p1;
-                    in[2] = block_shift_p1<RAGGED, SHIFT>(p2, c, last_bit);
-                    in[4] = block_shift_p1<RAGGED, SHIFT>(r4, c, last_bit);
+                    in[2] = shift_p1<RAGGED, SHIFT>(p2, c);
+                    in[4] = shift_p1<RAGGED, SHIFT>(r4, c);
                     in[5] = r5;
                 };
                 auto even_row = [&] {

@@ -54,7 +54,7 @@ struct LaneCtx {
     uint32_t w;          // word index of this lane (torus, 0..W-1)
     uint32_t wb;         // 4 * w, the lane's byte offset within a plane row
     uint32_t first_shl;  // 32 - nb on the lane holding word 0, else 0
-    bool last;           // lane holds word W-1
+    uint32_t last_bit;   // bit nb - 1 on the lane holding word W-1, else 0
     uint32_t nb;
     uint32_t vmask;      // valid bits of this lane's word
     uint32_t lsrc, rsrc; // segment mode: byte address of the lanes holding words w-1, w+1
@@ -144,6 +144,14 @@ __host__ __device__ constexpr int chir_src(int O, int s)
 }
 __host__ __device__ constexpr int chir_delay(int O, int s) { return s - chir_src(O, s); }
 
+// The bits past the row's end of a ragged row's last word may hold anything
+// (they are cleared once, before the store): the first word takes only cell
+// nb - 1 from it, and its own cell nb - 1 comes by a bit select.  Clearing
+// every level's planes and selecting by compares cost a quarter more
+// instructions; without, and with the plain and forced copies of the walk:
+// 30001 x 8000 FHP-III 22.2 -> 19.1 us a step, HPP 9.6 -> 5.7, 20001 x 6000
+// FHP-II forced pipe 26.9 -> 18.0.
+
 // out cell x = in cell x-1, cyclically over dim_x
 template <bool RAGGED, int SEG>
 __device__ __forceinline__ uint32_t shift_m1(uint32_t v, const LaneCtx& c)
@@ -159,7 +167,7 @@ __device__ __forceinline__ uint32_t shift_p1(uint32_t v, const LaneCtx& c)
     const uint32_t R = right_word<SEG>(v, c);
     const uint32_t o = __builtin_amdgcn_alignbit(R, v, 1);
     if (!RAGGED) return o;
-    return c.last ? ((v >> 1) | ((R & 1u) << (c.nb - 1u))) : o;
+    return bit3<kMux>(c.last_bit, R << (c.nb - 1u), o);
 }
 
 }  // namespace
@@ -240,11 +248,9 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, uint32_t strip, uin
     c.wb = 4u * c.w;
     c.nb = g.nb;
     c.first_shl = (c.w == 0) ? 32u - g.nb : 0u;
-    c.last = c.w + 1 == g.W;
-    c.vmask = (c.last && g.nb < 32) ? ((1u << g.nb) - 1u) : 0xFFFFFFFFu;
-    uint32_t edge = 0;  // cells of this lane on the east / west columns
-    if (c.w == 0) edge |= 1u;
-    if (c.last) edge |= 1u << (g.nb - 1u);
+    c.last_bit = c.w + 1 == g.W ? 1u << (g.nb - 1u) : 0u;
+    c.vmask = (c.last_bit && g.nb < 32) ? ((1u << g.nb) - 1u) : 0xFFFFFFFFu;
+    const uint32_t edge = (c.w == 0 ? 1u : 0u) | c.last_bit;  // this lane's cells on the east / west columns
 
     const uint32_t* src = a.src;
     uint32_t* dst = a.dst;
@@ -559,12 +565,25 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, uint32_t strip, uin
                 if (t_solids) {
                     const uint32_t ns = mns[s], sl = msl[s];
                     if (__builtin_amdgcn_ballot_w64((ns | sl) != 0) != 0) {
-                        // rows of NO_SLIP cells only (walls, obstacles) take
-                        // the one-select rule
-                        if (__builtin_amdgcn_ballot_w64(sl != 0) == 0)
-                            apply_no_slip<KIND, uint32_t>(st, in, ns);
-                        else
-                            apply_solids<KIND, uint32_t>(st, in, ns, sl, edge, j == 0 || j + 1 == g.dim_y);
+                        // one select for NO_SLIP cells (walls, obstacles)
+                        apply_no_slip<KIND, uint32_t>(st, in, ns);
+                        if (__builtin_amdgcn_ballot_w64(sl != 0) != 0) {
+                            // apply_solids as selects: SLIP cells on the east
+                            // and west columns mirror in y, the others in x on
+                            // the north and south rows, and pass through
+                            // elsewhere (32768 x 8000 slip box 36.3 -> 31.4 us
+                            // a step: the walls' columns are in every tile of
+                            // two strips)
+                            const uint32_t rim = sl & edge, inner = sl & ~edge;
+#pragma unroll
+                            for (int d = 0; d < Q; ++d) st[d] = bit3<kMux>(rim, in[miry_dir<KIND>(d)], st[d]);
+                            if (__builtin_amdgcn_ballot_w64(inner != 0) != 0) {
+                                const bool ns_row = j == 0 || j + 1 == g.dim_y;
+#pragma unroll
+                                for (int d = 0; d < Q; ++d)
+                                    st[d] = bit3<kMux>(inner, ns_row ? in[mirx_dir<KIND>(d)] : in[d], st[d]);
+                            }
+                        }
                     }
                     // fcur is zero outside the forced rows
                     if (t_force && (SEG || (j >= a.fy0 && j < a.fy1)))
@@ -576,7 +595,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, uint32_t strip, uin
                     apply_force<KIND, uint32_t>(st, fcur[s], a.force_dir);
                 }
 #pragma unroll
-                for (int d = 0; d < Q; ++d) out[d] = RAGGED ? (st[d] & c.vmask) : st[d];
+                for (int d = 0; d < Q; ++d) out[d] = st[d];
             }
             // slide the window of boundary s-1 (its newest row is cur)
             if (have_prev) {
@@ -596,7 +615,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, uint32_t strip, uin
                 if (s == K) {
                     const bool wr = writer && (!SEG || i - (uint32_t)(2 * K) < rows);
 #pragma unroll
-                    for (int d = 0; d < Q; ++d) store_plane(j, d, cur[d], wr);
+                    for (int d = 0; d < Q; ++d) store_plane(j, d, RAGGED ? (cur[d] & c.vmask) : cur[d], wr);
                 }
             }
         }
@@ -656,13 +675,12 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, uint32_t strip, uin
     // copy of the walk with that code left out (no tests, no branches).  Tiles
     // forced along x that hold no solids take a copy with the force applied
     // on every level and none of the solid tests (in the general walk they
-    // ran 1.75 times as long as a plain walk).  Rows with a short last word,
-    // and the multi-pass kernel, keep fewer copies: more would push those
-    // kernels past the register budget.
+    // ran 1.75 times as long as a plain walk).  The multi-pass kernel keeps
+    // fewer copies: more would push it past the register budget.
     using M0 = std::integral_constant<int, 0>;
     using M1 = std::integral_constant<int, 1>;
     using M2 = std::integral_constant<int, 2>;
-    const int mode = (RAGGED || tile_solids) ? 2 : !tile_force ? 0 : (a.force_dir == 1 && !PIPE) ? 1 : 2;
+    const int mode = tile_solids ? 2 : !tile_force ? 0 : (a.force_dir == 1 && !PIPE) ? 1 : 2;
     auto run = [&](auto up_tag) {
         if (mode == 2) walk(M2{}, up_tag);
         else if (mode == 1) walk(M1{}, up_tag);
