@@ -626,15 +626,18 @@ hipError_t launch_cell_fields(int kind, const uint32_t* planes, const Geometry& 
 // bound (2145 adds at r = 32).  So one wave of a workgroup does nothing else,
 // one chain per lane for 64 coarse cells, with the addends already in LDS in
 // the order it needs; the other kCoarseProducers waves read the planes, up
-// to 16 columns of a row at a time (a unit), turn them into addends and keep the
-// popcounts.  An 8192 x 4096 lattice at r = 32: 242 us with one thread per
-// coarse cell doing all of it, waiting out a memory latency per word; 52 us so
-// (4400 x 2200 at r = 20: 113 and 25 us; 1480 x 740 at r = 10: 36 and 9.9 us).
+// to kCoarseColumns columns of a row at a time (a unit), turn them into addends
+// and keep the popcounts.  An 8192 x 4096 lattice at r = 32: 242 us with one
+// thread per coarse cell doing all of it, waiting out a memory latency per
+// word, 52 us with units of 16 columns (twice the stages, whose barriers and
+// loads' latency count), 26 us so (4400 x 2200 at r = 20: 113, 25 and 15 us;
+// 1480 x 740 at r = 10: 36, 9.9 and 7.8 us).  The producers' arithmetic bounds
+// it: loads two stages ahead in place of one make no difference.
 constexpr uint32_t kCoarseExactRadius = 1023;
-constexpr uint32_t kCoarseProducers = 7;
+constexpr uint32_t kCoarseProducers = 7, kCoarseColumns = 36, kChainAhead = 4;
 
-// Addends of the y-momentum chain for the cells of one unit: bit j of the
-// four planes is cell j; out[j] = ky * sin(pi/3), ky = a1 + a2 - a4 - a5,
+// Addends of the y-momentum chain for the cells of one unit, zeros past its
+// end: bit j of the four planes is cell j; out[j] = ky * sin(pi/3), ky = a1 + a2 - a4 - a5,
 // exact.  The float's bits are put together from three planes: zero or not,
 // |ky| == 2 (exponent one up), sign.
 __device__ __forceinline__ void y_addends(uint32_t a1, uint32_t a2, uint32_t a4, uint32_t a5, uint32_t quads,
@@ -669,7 +672,7 @@ void coarse_kernel(const uint32_t* __restrict__ planes, Geometry g, uint32_t r, 
     // [2 stages][producer][chunk / 4 quads][64 coarse cells] addends
     extern __shared__ float4 addends[];
     __shared__ int sums[kCoarseProducers][3][64];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t cdx = g.dim_x / (2 * r), cdy = g.dim_y / (2 * r), nc = cdx * cdy;
     const uint32_t c = blockIdx.x * 64 + lane;
     const bool live = c < nc;
@@ -686,54 +689,79 @@ void coarse_kernel(const uint32_t* __restrict__ planes, Geometry g, uint32_t r, 
 
     int rho = 0, kx = 0, ky = 0;  // producers: density, x momentum in halves (HPP: ones), HPP y momentum
     float sy = 0.0f;              // wave 0: the chain
-    uint32_t lo[Q], hi[Q];        // producers: the unit's plane words, loaded a stage ahead
+    uint32_t word[3][Q];          // producers: the unit's plane words, loaded a stage ahead
     auto load_unit = [&](uint32_t u) {
         const uint32_t i = u % per_row, n = unit_cells(i);
         const uint32_t y = y0 + u / per_row + (i >= chunks ? 1u : 0u), x = i >= chunks ? 0u : x0 + i * chunk;
         const bool ok = live && u < units && y < g.dim_y;
         const uint32_t* p = planes + (size_t)y * Q * g.P + (x >> 5);
-        const bool two = ok && (x & 31u) + n > 32;
+        const bool two = ok && (x & 31u) + n > 32, three = ok && (x & 31u) + n > 64;
 #pragma unroll
         for (int d = 0; d < Q; ++d) {
-            lo[d] = ok ? p[(size_t)d * g.P] : 0u;
-            hi[d] = two ? p[(size_t)d * g.P + 1] : 0u;
+            word[0][d] = ok ? p[(size_t)d * g.P] : 0u;
+            word[1][d] = two ? p[(size_t)d * g.P + 1] : 0u;
+            word[2][d] = three ? p[(size_t)d * g.P + 2] : 0u;
         }
     };
     if (wave) load_unit(wave - 1);
+    else __builtin_amdgcn_s_setprio(3);  // every add of the chain waits for the last one
     for (uint32_t st = 0; st <= stages; ++st) {
         if (wave && st < stages) {
             const uint32_t u = st * kCoarseProducers + wave - 1, i = u % per_row, n = unit_cells(i);
             const uint32_t sh = i >= chunks ? 0u : (x0 + i * chunk) & 31u;
-            const uint32_t valid = n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u;
-            uint32_t a[Q];
+            // the unit's first 32 cells and the rest
+            const uint32_t valid = n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u, rest = n > 32 ? (1u << (n - 32u)) - 1u : 0u;
+            uint32_t a[Q], e[Q];
 #pragma unroll
-            for (int d = 0; d < Q; ++d) a[d] = __builtin_amdgcn_alignbit(hi[d], lo[d], sh) & valid;
+            for (int d = 0; d < Q; ++d) {
+                a[d] = __builtin_amdgcn_alignbit(word[1][d], word[0][d], sh) & valid;
+                e[d] = __builtin_amdgcn_alignbit(word[2][d], word[1][d], sh) & rest;
+            }
             if (st + 1 < stages) load_unit(u + kCoarseProducers);
+            auto count = [&](const uint32_t* v) {
 #pragma unroll
-            for (int d = 0; d < Q; ++d) rho += __popc(a[d]);
-            if (KIND == kHPP) {
-                kx += __popc(a[0]) - __popc(a[2]);
-                ky += __popc(a[1]) - __popc(a[3]);
-            } else {
-                kx += 2 * (__popc(a[0]) - __popc(a[3])) + __popc(a[1]) - __popc(a[2]) - __popc(a[4]) + __popc(a[5]);
-                y_addends(a[1], a[2], a[4], a[5], (n + 3) / 4,
-                          addends + ((st & 1u) * kCoarseProducers + wave - 1) * slot + lane);
+                for (int d = 0; d < Q; ++d) rho += __popc(v[d]);
+                if (KIND == kHPP) {
+                    kx += __popc(v[0]) - __popc(v[2]);
+                    ky += __popc(v[1]) - __popc(v[3]);
+                } else {
+                    kx += 2 * (__popc(v[0]) - __popc(v[3])) + __popc(v[1]) - __popc(v[2]) - __popc(v[4]) + __popc(v[5]);
+                }
+            };
+            count(a);
+            if (n > 32) count(e);
+            if (kChain) {
+                float4* out = addends + ((st & 1u) * kCoarseProducers + wave - 1) * slot + lane;
+                y_addends(a[1], a[2], a[4], a[5], min(chunk, 32u) / 4, out);
+                if (chunk > 32) y_addends(e[1], e[2], e[4], e[5], (chunk - 32) / 4, out + 8 * 64);
             }
         }
         if (kChain && !wave && st) {
-            for (uint32_t p = 0; p < kCoarseProducers; ++p) {
-                const uint32_t u = (st - 1) * kCoarseProducers + p;
-                if (u >= units) break;
-                const uint32_t quads = (unit_cells(u % per_row) + 3) / 4;
-                const float4* a = addends + (((st - 1) & 1u) * kCoarseProducers + p) * slot + lane;
-#pragma unroll 4
-                for (uint32_t k = 0; k < quads; ++k) {
-                    const float4 v = a[k * 64];
-                    sy += v.x;
-                    sy += v.y;
-                    sy += v.z;
-                    sy += v.w;
+            // the stage's addends are one stream: the next kChainAhead quads
+            // are on their way from LDS while the chain takes the last ones
+            const uint32_t quads = min(kCoarseProducers, units - (st - 1) * kCoarseProducers) * (chunk / 4);
+            const float4* a = addends + ((st - 1) & 1u) * kCoarseProducers * slot + lane;
+            float4 even[kChainAhead], odd[kChainAhead];
+            auto fetch = [&](float4 (&v)[kChainAhead], uint32_t q) {
+#pragma unroll
+                for (uint32_t k = 0; k < kChainAhead; ++k) v[k] = a[(q + k) * 64];
+            };
+            auto take = [&](const float4 (&v)[kChainAhead], uint32_t q) {
+#pragma unroll
+                for (uint32_t k = 0; k < kChainAhead; ++k) {
+                    if (q + k >= quads) return;
+                    sy += v[k].x;
+                    sy += v[k].y;
+                    sy += v[k].z;
+                    sy += v[k].w;
                 }
+            };
+            fetch(even, 0);
+            for (uint32_t q = 0; q < quads; q += 2 * kChainAhead) {
+                fetch(odd, q + kChainAhead);
+                take(even, q);
+                fetch(even, q + 2 * kChainAhead);
+                take(odd, q + kChainAhead);
             }
         }
         if (kChain) __syncthreads();
@@ -836,13 +864,14 @@ hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, ui
         }
         return hipGetLastError();
     }
-    // the r + 1 columns in units of at most 16, of about equal size, whole
-    // quads of addends: two stages of them take 56 KiB of LDS at most
-    const uint32_t chunks = (r + 1 + 15) / 16;
+    // the r + 1 columns in units of at most kCoarseColumns, of about equal size,
+    // whole quads of addends: two stages of them take 126 KiB of LDS at most
+    const uint32_t chunks = (r + kCoarseColumns) / kCoarseColumns;
     const uint32_t chunk = ((r + 1 + chunks - 1) / chunks + 3) & ~3u;
     const uint32_t used = (r + chunk) / chunk;  // chunks that hold a column
     const dim3 block(64 * (1 + kCoarseProducers));
-    const size_t lds = kind == kHPP ? 0 : (size_t)2 * kCoarseProducers * chunk * 64 * sizeof(float);
+    // (the chain reads up to three times kChainAhead quads past the last one)
+    const size_t lds = kind == kHPP ? 0 : (size_t)(2 * kCoarseProducers * chunk + 3 * 4 * kChainAhead) * 64 * sizeof(float);
     switch (kind) {
     case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
     case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;

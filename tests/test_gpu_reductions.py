@@ -62,3 +62,12 @@ def test_coarse_fields_bit_exact_at_unit_edges(model, dx, dy, r):
     np.testing.assert_array_equal(lat.mean_density().view(np.uint32), md.view(np.uint32))
     np.testing.assert_array_equal(lat.mean_momentum().view(np.uint32), mm.view(np.uint32))
     lat.close()
+
+
+# a row's columns in one unit of more than a word, in one of all its columns,
+# and in two and three units
+@pytest.mark.parametrize("model", [0, 1, 3])
+@pytest.mark.parametrize("dx,dy,r", [(620, 130, 31), (700, 140, 34), (1050, 144, 35), (72, 146, 36), (720, 150, 37),
+                                     (710, 284, 71), (1000, 300, 72), (880, 450, 109)])
+def test_coarse_fields_bit_exact_at_long_units(model, dx, dy, r):
+    test_coarse_fields_bit_exact_at_unit_edges(model, dx, dy, r)
