@@ -760,7 +760,7 @@ void finish(lgca_batch* b, Job* j)
     hipchk(hipEventRecord(j->last_ev, b->stream), "hipEventRecord");
     hipchk(hipStreamWaitEvent(b->post_stream, j->last_ev, 0), "hipStreamWaitEvent");
     hipchk(launch_coarse(p.kind, st, p.g, j->d.coarse_radius, (float*)(m + j->L.md), (float*)(m + j->L.mm),
-                         (float*)(m + j->L.vel), b->post_stream),
+                         (float*)(m + j->L.vel), nullptr, b->post_stream),
            "coarse");
     hipchk(launch_unpack(st, (uint8_t*)(m + j->L.bytes), p.g, b->post_stream), "unpack");
     j->done_ev = take_event(b);

@@ -56,6 +56,9 @@ struct PipeCache {
 // Counter words of a pipelined launch: the bands' ticket counters, the error
 // word, then one finished-pass count per work item (row tile x strip).
 constexpr uint32_t kPipeQueue = 0, kPipeError = kMaxBands, kPipeDone = 16;
+constexpr uint32_t kCounters = 16;
+constexpr size_t kPageCoarse = 256;              // offset of the coarse fields in a handle's page
+constexpr size_t kPageMost = (size_t)1 << 20;    // largest such fields
 // steps_per_pass value that lets the trial choose it
 constexpr int kAutoSteps = -1;
 }  // namespace lgca
@@ -96,6 +99,12 @@ struct lgca_lattice {
     float* velocity = nullptr;
     uint8_t* bytes = nullptr;       // N-byte staging for u8 state / types
     unsigned long long* counters = nullptr;  // 16 words: counters and flags
+    bool counters_used = false;     // they may hold something
+    // Pinned memory that kernels write small results to (null: copied instead):
+    // the counters, then the coarse fields (density, momentum) where they fit
+    char* page = nullptr;
+    char* page_dev = nullptr;       // the same, for kernels
+    bool page_coarse = false;       // the coarse fields have room in it
     uint64_t seed = 0, step = 0, force_calls = 0;
     int force_dir = LGCA_FORCE_NONE;
     uint64_t force_thr = 0;
@@ -204,17 +213,28 @@ lgca_status ensure_mask(lgca_lattice* h)
     return LGCA_OK;
 }
 
+// Counters to the host.  A kernel writes them to pinned memory and clears them
+// for the next call: the runtime's copy of a few bytes to ordinary memory and
+// the clearing launch before each use cost 13 us more.
 lgca_status read_counters(lgca_lattice* h, unsigned long long* out, int n)
 {
-    HIPCHK(h, hipMemcpyAsync(out, h->counters, n * sizeof(unsigned long long),
-                             hipMemcpyDeviceToHost, h->stream));
+    if (!h->page) {
+        HIPCHK(h, hipMemcpyAsync(out, h->counters, n * sizeof(unsigned long long),
+                                 hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        return LGCA_OK;
+    }
+    HIPCHK(h, launch_publish(h->counters, (unsigned long long*)h->page_dev, kCounters, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    std::memcpy(out, h->page, n * sizeof(unsigned long long));
+    h->counters_used = false;
     return LGCA_OK;
 }
 
 lgca_status clear_counters(lgca_lattice* h)
 {
-    HIPCHK(h, launch_fill_u32((uint32_t*)h->counters, 0u, 16, h->stream));
+    if (h->counters_used) HIPCHK(h, launch_fill_u32((uint32_t*)h->counters, 0u, 2 * kCounters, h->stream));
+    h->counters_used = true;
     return LGCA_OK;
 }
 
@@ -311,8 +331,22 @@ extern "C" lgca_status lgca_create(lgca_lattice** out, int model, uint32_t dim_x
     if ((e = dalloc(&h->state[0], sb)) != hipSuccess) return bail(hip_fail(h, e, "hipMalloc(state)"));
     if ((e = dalloc(&h->state[1], sb)) != hipSuccess) return bail(hip_fail(h, e, "hipMalloc(state)"));
     if ((e = dalloc(&h->snap, sb)) != hipSuccess) return bail(hip_fail(h, e, "hipMalloc(snapshot)"));
-    if ((e = dalloc(&h->counters, 16 * sizeof(unsigned long long))) != hipSuccess)
+    if ((e = dalloc(&h->counters, kCounters * sizeof(unsigned long long))) != hipSuccess)
         return bail(hip_fail(h, e, "hipMalloc(counters)"));
+    h->counters_used = true;
+    {
+        const size_t coarse = (size_t)(dim_x / (2 * coarse_radius)) * (dim_y / (2 * coarse_radius)) * 12;
+        h->page_coarse = coarse <= kPageMost;
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kPageCoarse + (h->page_coarse ? coarse : 0), hipHostMallocDefault) == hipSuccess) {
+            h->page = (char*)p;
+            if (hipHostGetDevicePointer((void**)&h->page_dev, p, 0) != hipSuccess) {
+                (void)hipHostFree(p);
+                h->page = nullptr;
+            }
+        }
+        if (!h->page) (void)hipGetLastError();
+    }
     const uint64_t nw = (uint64_t)h->state_words;
     if ((e = launch_fill_u32(h->state[0], 0u, nw, h->stream)) != hipSuccess ||
         (e = launch_fill_u32(h->state[1], 0u, nw, h->stream)) != hipSuccess ||
@@ -341,6 +375,7 @@ extern "C" lgca_status lgca_destroy(lgca_lattice* h)
         if (h->pipe_ctr) (void)hipFree(h->pipe_ctr);
         for (hipEvent_t ev : h->trial_ev) (void)hipEventDestroy(ev);
         h->copier.release();
+        if (h->page) (void)hipHostFree(h->page);
         if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
     }
     delete h;
@@ -1539,7 +1574,8 @@ extern "C" lgca_status lgca_snapshot(lgca_lattice* h)
     return LGCA_OK;
 }
 
-static lgca_status run_coarse(lgca_lattice* h)
+// `host`: also to these, density first, for kernels
+static lgca_status run_coarse(lgca_lattice* h, float* host = nullptr)
 {
     const size_t nc = (size_t)(h->dim_x / (2 * h->r)) * (h->dim_y / (2 * h->r));
     if (!h->mean_density) {
@@ -1548,7 +1584,7 @@ static lgca_status run_coarse(lgca_lattice* h)
         HIPCHK(h, dalloc(&h->velocity, nc * 8));
     }
     HIPCHK(h, launch_coarse(h->kind, h->snap, h->g, h->r, h->mean_density, h->mean_momentum,
-                            h->velocity, h->stream));
+                            h->velocity, host, h->stream));
     return LGCA_OK;
 }
 
@@ -1566,8 +1602,9 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
         if (cell_density && !h->cell_density) HIPCHK(h, dalloc(&h->cell_density, n * 4));
         if (cell_momentum && !h->cell_momentum) HIPCHK(h, dalloc(&h->cell_momentum, n * 8));
     }
-    if (mean_density || mean_momentum) {
-        lgca_status st = run_coarse(h);
+    const bool coarse = mean_density || mean_momentum, page = h->page && h->page_coarse;
+    if (coarse) {
+        lgca_status st = run_coarse(h, page ? (float*)(h->page_dev + kPageCoarse) : nullptr);
         if (st) return st;
     }
     if (cell_density || cell_momentum)
@@ -1575,9 +1612,14 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
                                      cell_momentum ? h->cell_momentum : nullptr, h->stream));
     if (cell_density) copies[n_copies++] = {cell_density, h->cell_density, n * 4};
     if (cell_momentum) copies[n_copies++] = {cell_momentum, h->cell_momentum, n * 8};
-    if (mean_density) copies[n_copies++] = {mean_density, h->mean_density, nc * 4};
-    if (mean_momentum) copies[n_copies++] = {mean_momentum, h->mean_momentum, nc * 8};
-    HIPCHK(h, h->copier.run(copies, n_copies, h->stream));
+    if (mean_density && !page) copies[n_copies++] = {mean_density, h->mean_density, nc * 4};
+    if (mean_momentum && !page) copies[n_copies++] = {mean_momentum, h->mean_momentum, nc * 8};
+    HIPCHK(h, h->copier.run(copies, n_copies, h->stream));  // returns with the stream idle
+    if (page) {
+        const char* at = h->page + kPageCoarse;
+        if (mean_density) std::memcpy(mean_density, at, nc * 4);
+        if (mean_momentum) std::memcpy(mean_momentum, at + nc * 4, nc * 8);
+    }
     return LGCA_OK;
 }
 

@@ -665,7 +665,8 @@ __device__ __forceinline__ void y_addends(uint32_t a1, uint32_t a2, uint32_t a4,
 template <int KIND>
 __global__ __launch_bounds__(64 * (1 + kCoarseProducers))
 void coarse_kernel(const uint32_t* __restrict__ planes, Geometry g, uint32_t r, uint32_t chunks, uint32_t chunk,
-                   float* __restrict__ md, float* __restrict__ mm, float* __restrict__ vel)
+                   float* __restrict__ md, float* __restrict__ mm, float* __restrict__ vel,
+                   float* __restrict__ host)
 {
     constexpr int Q = num_dir_of_kind(KIND);
     constexpr bool kChain = KIND != kHPP;
@@ -787,6 +788,11 @@ void coarse_kernel(const uint32_t* __restrict__ planes, Geometry g, uint32_t r, 
     md[c] = den;
     mm[2 * c] = ux;
     mm[2 * c + 1] = uy;
+    if (host) {
+        host[c] = den;
+        host[nc + 2 * c] = ux;
+        host[nc + 2 * c + 1] = uy;
+    }
     if (vel) {
         vel[2 * c] = den > 0.0f ? ux / den : 0.0f;
         vel[2 * c + 1] = den > 0.0f ? uy / den : 0.0f;
@@ -799,7 +805,7 @@ template <int KIND>
 __global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __restrict__ planes,
                                                           Geometry g, uint32_t r,
                                                           float* __restrict__ md, float* __restrict__ mm,
-                                                          float* __restrict__ vel)
+                                                          float* __restrict__ vel, float* __restrict__ host)
 {
     constexpr int Q = num_dir_of_kind(KIND);
     const uint32_t cdx = g.dim_x / (2 * r), cdy = g.dim_y / (2 * r);
@@ -845,6 +851,11 @@ __global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __rest
     md[c] = rho;
     mm[2 * c] = ux;
     mm[2 * c + 1] = uy;
+    if (host) {
+        host[c] = rho;
+        host[cdx * cdy + 2 * c] = ux;
+        host[cdx * cdy + 2 * c + 1] = uy;
+    }
     if (vel) {
         vel[2 * c] = rho > 0.0f ? ux / rho : 0.0f;
         vel[2 * c + 1] = rho > 0.0f ? uy / rho : 0.0f;
@@ -852,15 +863,15 @@ __global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __rest
 }
 
 hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, uint32_t r,
-                         float* mean_density, float* mean_momentum, float* velocity, hipStream_t s)
+                         float* mean_density, float* mean_momentum, float* velocity, float* host, hipStream_t s)
 {
     const uint32_t n = (g.dim_x / (2 * r)) * (g.dim_y / (2 * r));
     const dim3 grid(div_up(n, 64));
     if (r > kCoarseExactRadius) {
         switch (kind) {
-        case kHPP: hipLaunchKernelGGL(coarse_large_kernel<kHPP>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
-        case kFHP1: hipLaunchKernelGGL(coarse_large_kernel<kFHP1>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
-        default: hipLaunchKernelGGL(coarse_large_kernel<kFHP2>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity); break;
+        case kHPP: hipLaunchKernelGGL(coarse_large_kernel<kHPP>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
+        case kFHP1: hipLaunchKernelGGL(coarse_large_kernel<kFHP1>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
+        default: hipLaunchKernelGGL(coarse_large_kernel<kFHP2>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
         }
         return hipGetLastError();
     }
@@ -873,9 +884,9 @@ hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, ui
     // (the chain reads up to three times kChainAhead quads past the last one)
     const size_t lds = kind == kHPP ? 0 : (size_t)(2 * kCoarseProducers * chunk + 3 * 4 * kChainAhead) * 64 * sizeof(float);
     switch (kind) {
-    case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
-    case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
-    default: hipLaunchKernelGGL(coarse_kernel<kFHP2>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity); break;
+    case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity, host); break;
+    case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity, host); break;
+    default: hipLaunchKernelGGL(coarse_kernel<kFHP2>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity, host); break;
     }
     return hipGetLastError();
 }
@@ -1021,6 +1032,20 @@ hipError_t launch_mean_velocity(int kind, const uint32_t* planes, const uint32_t
     case kFHP1: hipLaunchKernelGGL(mean_velocity_kernel<kFHP1>, grid, block, 0, s, planes, mask, g, tw_log, acc); break;
     default: hipLaunchKernelGGL(mean_velocity_kernel<kFHP2>, grid, block, 0, s, planes, mask, g, tw_log, acc); break;
     }
+    return hipGetLastError();
+}
+
+// Counters to pinned memory, and zero for their next use.
+__global__ __launch_bounds__(64) void publish_kernel(unsigned long long* counters, unsigned long long* page, uint32_t n)
+{
+    if (threadIdx.x >= n) return;
+    page[threadIdx.x] = counters[threadIdx.x];
+    counters[threadIdx.x] = 0;
+}
+
+hipError_t launch_publish(unsigned long long* counters, unsigned long long* page, uint32_t n, hipStream_t s)
+{
+    hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(64), 0, s, counters, page, n);
     return hipGetLastError();
 }
 

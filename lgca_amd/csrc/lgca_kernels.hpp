@@ -274,11 +274,13 @@ hipError_t launch_cell_fields(int kind, const uint32_t* planes, const Geometry& 
                               float* density, float* momentum, hipStream_t s);
 hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, uint32_t r,
                          float* mean_density, float* mean_momentum, float* velocity,
-                         hipStream_t s);
+                         float* host, hipStream_t s);  // host: null, or density then momentum once more
 hipError_t launch_count(const uint32_t* words, uint64_t nwords, unsigned long long* out,
                         hipStream_t s);
 hipError_t launch_mean_velocity(int kind, const uint32_t* planes, const uint32_t* mask,
                                 const Geometry& g, long long* acc3, hipStream_t s);
+// n <= 64 counters to `page` (pinned memory), then cleared.
+hipError_t launch_publish(unsigned long long* counters, unsigned long long* page, uint32_t n, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 
 // Device-resident state of the viewers' forcing controller.

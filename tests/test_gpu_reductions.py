@@ -71,3 +71,26 @@ def test_coarse_fields_bit_exact_at_unit_edges(model, dx, dy, r):
                                      (710, 284, 71), (1000, 300, 72), (880, 450, 109)])
 def test_coarse_fields_bit_exact_at_long_units(model, dx, dy, r):
     test_coarse_fields_bit_exact_at_unit_edges(model, dx, dy, r)
+
+
+@pytest.mark.parametrize("dx,dy", [(582, 600), (584, 600)])  # coarse fields just below and above 1 MiB
+def test_small_results_in_turn(dx, dy):
+    """Counts, velocities, refused inputs and coarse fields one after another:
+    each result is its own call's."""
+    from lgca_amd import LgcaError
+    lat, state, types = make(2, dx, dy, 1, True)
+    velocity = lat.get_mean_velocity()
+    for _ in range(3):
+        assert lat.get_n_particles() == orc.count_particles(state)
+        assert lat.get_mean_velocity() == velocity
+        with pytest.raises(LgcaError):
+            lat.set_cell_types(np.full(dx * dy, 3, np.uint8))
+        lat.set_cell_types(types)
+        with pytest.raises(LgcaError):
+            lat.set_state_u8(np.full(dx * dy, 255, np.uint8))
+        lat.set_state_u8(state)
+        lat.post_process(cells=False)
+        _, _, md, mm = orc.post_process(2, dx, dy, 1, state)
+        np.testing.assert_array_equal(lat.mean_density().view(np.uint32), md.view(np.uint32))
+        np.testing.assert_array_equal(lat.mean_momentum().view(np.uint32), mm.view(np.uint32))
+    lat.close()
