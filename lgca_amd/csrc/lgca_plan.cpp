@@ -228,16 +228,17 @@ uint64_t block_count(const Geometry& g, int k, uint32_t tiles)
     return ((uint64_t)tiles * (g.W + 2 * h) + stride - 1) / stride;
 }
 
-// Lattices of up to 32 wave-rows (64 words of a row, packed as the blocks have
-// them) per SIMD.  us per step in blocks / walked, FHP-II: 4400 x 2200 1.9 /
-// 3.9, 8192 x 4096 (17,045 wave-rows) 3.6 / 5.3, 12000 x 4000 (24,323) 5.6 /
-// 6.3, 16384 x 4096 (33,957) 6.6 / 6.9, 32768 x 2048 (33,891) 6.8 / 6.6, 16384 x
-// 8192 (67,914) 12.6 / 10.5: the larger ones fill the GPU with walks, which
-// read and compute fewer halo rows.
+// Lattices of up to 36 wave-rows (64 words of a row, packed as the blocks have
+// them) per SIMD.  us per step in blocks / walked, FHP-II: 4400 x 2200 1.7 /
+// 2.9, 8192 x 4096 (17,045 wave-rows) 3.2 / 4.8, 12000 x 4000 (24,323) 4.7 /
+// 5.2, 32768 x 2048 (33,891) 5.8 / 6.0, 12000 x 6000 (36,484) 6.0 / 6.4, 13001 x
+// 6000 (39,581) 8.3 / 8.0 with walls and forced columns, 16384 x
+// 8192 (67,914) 11.2 / 9.5: the larger ones fill the GPU with walks, which read
+// and compute fewer halo rows.
 bool block_lattice(const Geometry& g)
 {
     const uint64_t wave_rows = tile_segments(g, 8) ? (uint64_t)g.dim_y / (64 / g.W) : block_count(g, 8, g.dim_y);
-    return wave_rows < 32768;
+    return wave_rows < 36864;
 }
 
 std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k)
