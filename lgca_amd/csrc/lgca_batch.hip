@@ -28,7 +28,7 @@
 // the live mix and keeps the fastest per site update, and tunes again when the
 // mix has changed by 2x.  16 FHP-II ensemble jobs of 1000-4000 steps: 24 ms in
 // walks, 9 ms with blocks; 120 serving jobs 380 and 300 ms; 512 ensemble jobs
-// 280 and 273 ms.
+// 280 and 273 ms (all with a 43-step collision; 260 and 230 ms now).
 // Results never depend on the shape: the hash is keyed by (seed, step, cell).
 #include "lgca.h"
 

@@ -8,15 +8,16 @@
 // are short), one 32-cell word per lane, and all its waves advance them one
 // step at a time.  A step needs two planes of the row above a wave's rows and
 // two of the row below (the rest it holds itself): they pass through LDS, with
-// one barrier per step.  The state crosses HBM once per pass.  Each lattice's
-// best walk against its best blocks, us per step: 256 x 256 HPP 0.78 -> 0.24,
-// 1001 x 754 FHP-I slip box 3.06 -> 0.82, 2048 x 512 FHP-II pipe 3.05 -> 1.13,
-// 4400 x 2200 FHP-III cylinder 5.2 -> 2.0, 6000 x 3000 FHP-II forced channel
-// 8.0 -> 4.3 (1.2 of it the force draws).
+// one barrier per step.  The state crosses HBM once per pass.  us per step
+// walked -> in blocks as they came -> now (packed lanes, 32-step collision):
+// 256 x 256 HPP 0.78 -> 0.24, 1001 x 754 FHP-I slip box 3.06 -> 0.82 -> 0.80,
+// 2048 x 512 FHP-II pipe 3.05 -> 1.13 -> 1.06, 4400 x 2200 FHP-III cylinder 5.2
+// -> 2.4 -> 1.85, 6000 x 3000 FHP-II forced channel 8.0 -> 5.4 -> 4.1 (1.2 of it
+// the force draws).
 //
 // What bounds it: on the small ones the launch and the first loads (3 us a
 // pass) and each step's chain of dependent instructions through one barrier;
-// on the larger ones VALU issue (62 instructions per wave-row and step, as the
+// on the larger ones VALU issue (51 instructions per wave-row and step, as the
 // walk) with the halo rows' share of it.
 //
 // y-halo: the block reads hk >= K extra rows on either side of its th stored
@@ -30,7 +31,8 @@
 // shares a wave with the start of the next one's.  Neighbours in the sequence
 // are neighbours in the row except at the halos' outer ends, where strips have
 // the same garbage.  A 188-word row takes 3.06 waves so, and 4 strips: 6000 x
-// 3000 FHP-II 3.2 -> 2.5 us a step, 4400 x 2200 (138 words) 2.4 -> 2.0.
+// 3000 FHP-II 3.2 -> 2.5 us a step, 4400 x 2200 (138 words) 2.4 -> 2.0 (both
+// with a 43-step collision; 2.2 and 1.85 now).
 //
 // Chirality: a row's Philox call serves its word for a group of four steps;
 // the words wait in LDS (read once a step), which costs no registers and no

@@ -1505,6 +1505,23 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
     return LGCA_OK;
 }
 
+// Room for the listed tries of a call whose amount is at most `most`.
+static lgca_status ensure_force_ws(lgca_lattice* h, int64_t most)
+{
+    const uint32_t tries = count_force_tries((uint64_t)h->dim_x * h->dim_y, most);
+    const size_t need = tries ? count_force_bytes(tries) : 0;
+    if (h->force_ws_bytes >= need) return LGCA_OK;
+    if (h->force_ws) {
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        HIPCHK(h, hipFree(h->force_ws));
+    }
+    h->force_ws = nullptr;
+    h->force_ws_bytes = 0;
+    HIPCHK(h, dalloc(&h->force_ws, need));
+    h->force_ws_bytes = need;
+    return LGCA_OK;
+}
+
 // Queues a count-mode force of the live state (lgca_force.hip).  most: the
 // largest amount that may be asked for.
 static lgca_status queue_count_force(lgca_lattice* h, CountForceArgs a, int dir, int64_t most)
@@ -1519,16 +1536,8 @@ static lgca_status queue_count_force(lgca_lattice* h, CountForceArgs a, int dir,
     a.cells_magic = UINT64_MAX / n;
     a.row_magic = UINT64_MAX / h->dim_x;
     a.tries = count_force_tries(n, most);
-    if (a.tries && h->force_ws_bytes < count_force_bytes(a.tries)) {
-        if (h->force_ws) {
-            HIPCHK(h, hipStreamSynchronize(h->stream));
-            HIPCHK(h, hipFree(h->force_ws));
-        }
-        h->force_ws = nullptr;
-        h->force_ws_bytes = 0;
-        HIPCHK(h, dalloc(&h->force_ws, count_force_bytes(a.tries)));
-        h->force_ws_bytes = count_force_bytes(a.tries);
-    }
+    lgca_status st = ensure_force_ws(h, most);
+    if (st) return st;
     a.ws = h->force_ws;
     HIPCHK(h, launch_count_force(h->kind, a, h->stream));
     return LGCA_OK;
@@ -1870,6 +1879,7 @@ extern "C" lgca_status lgca_load_checkpoint(lgca_lattice** out, const char* path
             h->ctrl_u = hd.ctrl_u;
             h->ctrl_eq = hd.ctrl_eq;
             h->ctrl_most = std::max(hd.ctrl_forcing, hd.ctrl_eq);
+            if (!st) st = ensure_force_ws(h, h->ctrl_most);
             h->calls_on_device = false;
         }
         if (!st) {
@@ -1902,6 +1912,8 @@ extern "C" lgca_status lgca_controller_set(lgca_lattice* h, int dir, float u, in
     DeviceGuard dg(h->device);
     lgca_status st = sync_force_calls(h);
     if (st) return st;
+    // the ticks' room now: a tick only launches
+    if ((st = ensure_force_ws(h, std::max(forcing, equilibrium_forcing)))) return st;
     if (!h->ctrl) HIPCHK(h, dalloc(&h->ctrl, sizeof(Controller)));
     HIPCHK(h, launch_fill_u32((uint32_t*)h->ctrl, 0u, sizeof(Controller) / 4, h->stream));
     // forcing (64-bit) as two words, written by fill kernels: no host buffer

@@ -264,7 +264,8 @@ std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k)
 // time of the rows a SIMD still works on.  Constants from passes of 5 to 28
 // steps on 256 x 256 HPP (0.12 us a step), the 2048 x 512 FHP-II pipe (0.45)
 // and 4400 x 2200 FHP-II (1.6); the best predicted shape was within 10 % of
-// the best measured one on each.
+// the best measured one on each, and is with the shorter collision (constants
+// a sixth smaller pick no better shapes).
 float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32_t k, const BlockShape& s)
 {
     const bool seg = tile_segments(g, (int)k);
