@@ -33,6 +33,7 @@
 #include "lgca.h"
 
 #include "lgca_dev.hpp"
+#include "lgca_hostcopy.hpp"
 #include "lgca_kernels.hpp"
 
 #include <algorithm>
@@ -77,6 +78,28 @@ __global__ __launch_bounds__(256) void upload_kernel(uint32_t* __restrict__ dst,
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < words) dst[i] = src[i];
+}
+
+// A finished job's arrays on their way to ordinary memory: a launch gathers as
+// much of them as a pinned slot holds, 16 bytes a lane, while the host copies
+// the other slot on.  A copy command of the runtime for each of the three arrays
+// takes, with its staging and its wait, 56 us for 16 K cells of FHP-II at radius
+// 8, 70 for 512 K and 4.1 ms for 64 M; this takes 16, 39 and 3.3 ms.  The host's
+// copy out of the slot bounds it (13 to 24 GB/s), the kernel reaches the link's
+// rate.  128 jobs of 0.6 M cells, run and fetched: 42.0 ms, 38.9 so.
+constexpr size_t kResultSlot = 512u << 10;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+struct ResultPiece {
+    const u32x4* src[3];
+    uint32_t at[3], n[3];  // in units of 16 bytes
+};
+
+__global__ __launch_bounds__(256) void result_kernel(u32x4* __restrict__ slot, ResultPiece p)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    for (int k = 0; k < 3; ++k)
+        if (i < p.n[k]) slot[p.at[k] + i] = p.src[k][i];
 }
 
 __global__ __launch_bounds__(256) void install_kernel(BatchJob* jobs, BatchState* state,
@@ -417,6 +440,10 @@ struct lgca_batch {
     uint64_t n_submitted = 0, n_done = 0;
     Arena arena;
 
+    // lgca_batch_result: the two slots behind the staging halves
+    std::mutex result_mu;
+    hipEvent_t result_ev[2] = {nullptr, nullptr};
+
     // tuning (under mu)
     int user_k = 0;
     uint32_t user_waves = 0;
@@ -441,7 +468,7 @@ struct lgca_batch {
     char* d_setup = nullptr;            // admission records and disc tables
     size_t setup_cap = 0;
     uint32_t* d_err = nullptr;          // sink for the codec kernels' flags
-    char* staging = nullptr;            // pinned, two halves
+    char* staging = nullptr;            // pinned, two halves, then two result slots
     char* staging_dev = nullptr;        // the same, for kernels
     size_t staging_used = 0;
     int staging_half = 0;
@@ -1374,11 +1401,13 @@ extern "C" lgca_status lgca_batch_create(lgca_batch** out, int device, uint64_t 
     if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess) return fail(e, "hipStreamCreate");
     if ((e = hipStreamCreateWithFlags(&b->copy_stream, hipStreamNonBlocking)) != hipSuccess) return fail(e, "hipStreamCreate");
     if ((e = hipStreamCreateWithFlags(&b->post_stream, hipStreamNonBlocking)) != hipSuccess) return fail(e, "hipStreamCreate");
-    if ((e = hipHostMalloc((void**)&b->staging, 2 * kStagingHalf, hipHostMallocDefault)) != hipSuccess)
+    if ((e = hipHostMalloc((void**)&b->staging, 2 * kStagingHalf + 2 * kResultSlot, hipHostMallocDefault)) != hipSuccess)
         return fail(e, "hipHostMalloc(staging)");
     if ((e = hipHostGetDevicePointer((void**)&b->staging_dev, b->staging, 0)) != hipSuccess)
         return fail(e, "hipHostGetDevicePointer(staging)");
     for (auto& ev : b->staging_ev)
+        if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return fail(e, "hipEventCreate");
+    for (auto& ev : b->result_ev)
         if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return fail(e, "hipEventCreate");
     // both halves start free
     for (auto& ev : b->staging_ev)
@@ -1417,6 +1446,8 @@ extern "C" lgca_status lgca_batch_destroy(lgca_batch* b)
     for (hipEvent_t e : b->event_pool) (void)hipEventDestroy(e);
     for (hipEvent_t e : b->tune_ev) (void)hipEventDestroy(e);
     for (hipEvent_t e : b->staging_ev)
+        if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : b->result_ev)
         if (e) (void)hipEventDestroy(e);
     b->arena.release_all();
     void* dptrs[] = {b->d_jobs, b->d_state, b->d_items[0], b->d_items[1], b->d_draw, b->d_err, b->d_setup};
@@ -1553,6 +1584,59 @@ extern "C" lgca_status lgca_batch_job_info(lgca_batch* b, uint64_t job_id, lgca_
     return LGCA_OK;
 }
 
+namespace {
+
+// Copies the parts to ordinary memory through the two result slots.  Parts
+// start at multiples of 256 bytes of a job's memory and are followed by room up
+// to the next one, so their last 16 bytes can be read whole.
+hipError_t fetch_parts(lgca_batch* b, const HostCopy* part, int n)
+{
+    struct Range {
+        char* dst;
+        size_t at, bytes;
+    };
+    Range range[2][3];
+    int ranges[2] = {0, 0};
+    size_t taken[3] = {0, 0, 0};
+    char* const host = b->staging + 2 * kStagingHalf;
+    char* const dev = b->staging_dev + 2 * kStagingHalf;
+    auto launch = [&](int q) {
+        ResultPiece p{};
+        size_t used = 0;
+        uint32_t most = 0;
+        ranges[q] = 0;
+        for (int k = 0; k < n; ++k) {
+            const size_t bytes = std::min(part[k].bytes - taken[k], kResultSlot - used);
+            if (!bytes) continue;
+            const int r = ranges[q]++;
+            range[q][r] = {(char*)part[k].dst + taken[k], used, bytes};
+            p.src[r] = (const u32x4*)((const char*)part[k].src + taken[k]);
+            p.at[r] = (uint32_t)(used / 16);
+            p.n[r] = (uint32_t)((bytes + 15) / 16);
+            most = std::max(most, p.n[r]);
+            used += align_up(bytes);
+            taken[k] += bytes;
+        }
+        if (!most) return hipSuccess;
+        hipLaunchKernelGGL(result_kernel, dim3((most + 255) / 256), dim3(256), 0, b->copy_stream,
+                           (u32x4*)(dev + q * kResultSlot), p);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : hipEventRecord(b->result_ev[q], b->copy_stream);
+    };
+    hipError_t e = launch(0);
+    for (int q = 0; e == hipSuccess && ranges[q]; q ^= 1) {
+        e = launch(q ^ 1);
+        if (e == hipSuccess) e = hipEventSynchronize(b->result_ev[q]);
+        if (e != hipSuccess) break;
+        for (int r = 0; r < ranges[q]; ++r)
+            std::memcpy(range[q][r].dst, host + q * kResultSlot + range[q][r].at, range[q][r].bytes);
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(b->copy_stream);
+    return e;
+}
+
+}  // namespace
+
 extern "C" lgca_status lgca_batch_result(lgca_batch* b, uint64_t job_id, uint8_t* state,
                                          float* mean_density, float* mean_momentum)
 {
@@ -1578,13 +1662,24 @@ extern "C" lgca_status lgca_batch_result(lgca_batch* b, uint64_t job_id, uint8_t
         nc = j->p.nc;
     }
     DevGuard dg(b->device);
+    HostCopy part[3];
+    int parts = 0;
+    if (state) part[parts++] = {state, m + L.bytes, n};
+    if (mean_density) part[parts++] = {mean_density, m + L.md, nc * 4};
+    if (mean_momentum) part[parts++] = {mean_momentum, m + L.mm, nc * 8};
+    bool slots = true;
+    for (int k = 0; k < parts; ++k) slots = slots && pageable(part[k].dst);
+    std::unique_lock<std::mutex> result_lk(b->result_mu, std::defer_lock);
     hipError_t e = hipSuccess;
-    if (state && e == hipSuccess) e = hipMemcpyAsync(state, m + L.bytes, n, hipMemcpyDeviceToHost, b->copy_stream);
-    if (mean_density && e == hipSuccess)
-        e = hipMemcpyAsync(mean_density, m + L.md, nc * 4, hipMemcpyDeviceToHost, b->copy_stream);
-    if (mean_momentum && e == hipSuccess)
-        e = hipMemcpyAsync(mean_momentum, m + L.mm, nc * 8, hipMemcpyDeviceToHost, b->copy_stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->copy_stream);
+    if (slots && result_lk.try_lock()) {
+        e = fetch_parts(b, part, parts);
+        result_lk.unlock();
+    } else {
+        for (int k = 0; k < parts && e == hipSuccess; ++k)
+            e = hipMemcpyAsync(part[k].dst, part[k].src, part[k].bytes, hipMemcpyDeviceToHost, b->copy_stream);
+        const hipError_t f = hipStreamSynchronize(b->copy_stream);
+        if (e == hipSuccess) e = f;
+    }
     {
         std::lock_guard<std::mutex> lk(b->mu);
         if (--j->readers == 0) b->cv_readers.notify_all();

@@ -22,8 +22,8 @@ namespace {
 // Below this, starting the threads (26 us each) costs what the chunks gain.
 constexpr size_t kStagedBytes = (size_t)6 << 20;
 
-// Only ordinary memory gains: pinned, managed and device memory is copied to
-// directly.
+}  // namespace
+
 bool pageable(const void* p)
 {
     hipPointerAttribute_t a{};
@@ -33,8 +33,6 @@ bool pageable(const void* p)
     }
     return a.type == hipMemoryTypeUnregistered;
 }
-
-}  // namespace
 
 bool HostCopier::prepare()
 {

@@ -13,6 +13,10 @@ struct HostCopy {
     size_t bytes;
 };
 
+// Whether a host copy goes through a staging buffer: pinned, managed and device
+// memory is copied to directly.
+bool pageable(const void* p);
+
 // Copies through pinned slots of its own, made on the first large copy and
 // given back by release() (or the destructor).  Not for several threads at
 // once: its owner's lock covers it.
