@@ -57,8 +57,8 @@ struct PipeCache {
 // word, then one finished-pass count per work item (row tile x strip).
 constexpr uint32_t kPipeQueue = 0, kPipeError = kMaxBands, kPipeDone = 16;
 constexpr uint32_t kCounters = 16;
-constexpr size_t kPageCoarse = 256;              // offset of the coarse fields in a handle's page
-constexpr size_t kPageMost = (size_t)1 << 20;    // largest such fields
+constexpr size_t kPageMore = 256;                // offset of the coarse fields or row ranges in a handle's page
+constexpr size_t kPageMost = (size_t)1 << 20;    // largest coarse fields there
 // steps_per_pass value that lets the trial choose it
 constexpr int kAutoSteps = -1;
 }  // namespace lgca
@@ -337,8 +337,10 @@ extern "C" lgca_status lgca_create(lgca_lattice** out, int model, uint32_t dim_x
     {
         const size_t coarse = (size_t)(dim_x / (2 * coarse_radius)) * (dim_y / (2 * coarse_radius)) * 12;
         h->page_coarse = coarse <= kPageMost;
+        // the row ranges (dim_y <= 65535) always have room
+        const size_t more = std::max(h->page_coarse ? coarse : 0, (size_t)dim_y * 8);
         void* p = nullptr;
-        if (hipHostMalloc(&p, kPageCoarse + (h->page_coarse ? coarse : 0), hipHostMallocDefault) == hipSuccess) {
+        if (hipHostMalloc(&p, kPageMore + more, hipHostMallocDefault) == hipSuccess) {
             h->page = (char*)p;
             if (hipHostGetDevicePointer((void**)&h->page_dev, p, 0) != hipSuccess) {
                 (void)hipHostFree(p);
@@ -493,6 +495,11 @@ static lgca_status upload_types(lgca_lattice* h, const uint8_t* types, hipMemcpy
     HIPCHK(h, launch_fill_u32((uint32_t*)h->row_range, 0x7FFFFFFFu, h->dim_y, h->stream));
     HIPCHK(h, launch_fill_u32((uint32_t*)h->row_range + h->dim_y, 0u, h->dim_y, h->stream));
     HIPCHK(h, launch_types(h->bytes, h->mask, h->row_range, h->g, (uint32_t*)h->counters, h->stream));
+    // The rows' ranges come through the page as well, under the flag's wait: a
+    // copy of the runtime for each half took 40 us and more (2050 rows).
+    if (h->page)
+        HIPCHK(h, launch_copy_u32((uint32_t*)(h->page_dev + kPageMore), (const uint32_t*)h->row_range,
+                                  2u * (uint64_t)h->dim_y, h->stream));
     unsigned long long flag = 0;
     if ((st = read_counters(h, &flag, 1))) return st;
     if (flag & 1ull) return fail(h, LGCA_ERR_INVALID_STATE, "cell types must be 0, 1 or 2");
@@ -505,6 +512,12 @@ static lgca_status upload_types(lgca_lattice* h, const uint8_t* types, hipMemcpy
     h->pipes.clear();
     h->row_lo.resize(h->dim_y);
     h->row_hi.resize(h->dim_y);
+    if (h->page) {
+        const char* at = h->page + kPageMore;
+        std::memcpy(h->row_lo.data(), at, (size_t)h->dim_y * 4);
+        std::memcpy(h->row_hi.data(), at + (size_t)h->dim_y * 4, (size_t)h->dim_y * 4);
+        return LGCA_OK;
+    }
     HIPCHK(h, hipMemcpy(h->row_lo.data(), h->row_range, (size_t)h->dim_y * 4, hipMemcpyDeviceToHost));
     HIPCHK(h, hipMemcpy(h->row_hi.data(), h->row_range + h->dim_y, (size_t)h->dim_y * 4, hipMemcpyDeviceToHost));
     return LGCA_OK;
@@ -1613,7 +1626,7 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
     }
     const bool coarse = mean_density || mean_momentum, page = h->page && h->page_coarse;
     if (coarse) {
-        lgca_status st = run_coarse(h, page ? (float*)(h->page_dev + kPageCoarse) : nullptr);
+        lgca_status st = run_coarse(h, page ? (float*)(h->page_dev + kPageMore) : nullptr);
         if (st) return st;
     }
     if (cell_density || cell_momentum)
@@ -1625,7 +1638,7 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
     if (mean_momentum && !page) copies[n_copies++] = {mean_momentum, h->mean_momentum, nc * 8};
     HIPCHK(h, h->copier.run(copies, n_copies, h->stream));  // returns with the stream idle
     if (page) {
-        const char* at = h->page + kPageCoarse;
+        const char* at = h->page + kPageMore;
         if (mean_density) std::memcpy(mean_density, at, nc * 4);
         if (mean_momentum) std::memcpy(mean_momentum, at + nc * 4, nc * 8);
     }

@@ -1049,6 +1049,19 @@ hipError_t launch_publish(unsigned long long* counters, unsigned long long* page
     return hipGetLastError();
 }
 
+__global__ __launch_bounds__(256) void copy_u32_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                                                       uint64_t n)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+hipError_t launch_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n, hipStream_t s)
+{
+    if (n) hipLaunchKernelGGL(copy_u32_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, dst, src, n);
+    return hipGetLastError();
+}
+
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, uint32_t v, uint64_t n)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256)

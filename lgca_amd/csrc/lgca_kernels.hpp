@@ -281,6 +281,7 @@ hipError_t launch_mean_velocity(int kind, const uint32_t* planes, const uint32_t
                                 const Geometry& g, long long* acc3, hipStream_t s);
 // n <= 64 counters to `page` (pinned memory), then cleared.
 hipError_t launch_publish(unsigned long long* counters, unsigned long long* page, uint32_t n, hipStream_t s);
+hipError_t launch_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 
 // Device-resident state of the viewers' forcing controller.

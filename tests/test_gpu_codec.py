@@ -128,3 +128,25 @@ def test_large_results_arrive_whole(dx, dy):
     assert not bad
     for lat in lats:
         lat.close()
+
+
+@pytest.mark.parametrize("dy", [34, 1000, 65534])
+def test_rows_solid_ranges_reach_the_walks(dy):
+    """The launch order is made from every row's range of solid cells: set twice
+    and walked against the oracle, up to the most rows there can be."""
+    dx, steps = 64, 9
+    rng = np.random.default_rng(dy)
+    state = rng.integers(0, 1 << Q[2], dx * dy, dtype=np.uint8)
+    lat = make(2, dx, dy)
+    lat.set_tuning(8, 16)
+    for _ in range(2):
+        types = np.zeros((dy, dx), dtype=np.uint8)
+        types[0], types[-1] = 1, 1
+        types[rng.integers(0, dy, max(2, dy // 50)), rng.integers(0, dx, max(2, dy // 50))] = 1
+        types = types.reshape(-1)
+        lat.set_cell_types(types)
+        lat.set_state_u8(state)
+        lat.set_step(0)
+        lat.step(steps)
+        assert np.array_equal(lat.get_state_u8(), orc.run(2, dx, dy, types, state, SEED, 0, steps, None, nthreads=8))
+    lat.close()
