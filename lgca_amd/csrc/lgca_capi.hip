@@ -57,8 +57,8 @@ struct PipeCache {
 // word, then one finished-pass count per work item (row tile x strip).
 constexpr uint32_t kPipeQueue = 0, kPipeError = kMaxBands, kPipeDone = 16;
 constexpr uint32_t kCounters = 16;
-constexpr size_t kPageMore = 256;                // offset of the coarse fields or row ranges in a handle's page
-constexpr size_t kPageMost = (size_t)1 << 20;    // largest coarse fields there
+constexpr size_t kPageRanges = 256;              // offset of the row ranges in a handle's page
+constexpr size_t kPageMost = (size_t)1 << 20;    // largest coarse fields that get a page of their own
 // steps_per_pass value that lets the trial choose it
 constexpr int kAutoSteps = -1;
 }  // namespace lgca
@@ -101,10 +101,13 @@ struct lgca_lattice {
     unsigned long long* counters = nullptr;  // 16 words: counters and flags
     bool counters_used = false;     // they may hold something
     // Pinned memory that kernels write small results to (null: copied instead):
-    // the counters, then the coarse fields (density, momentum) where they fit
+    // the counters and the rows' solid ranges, and from the first call that
+    // fetches them the coarse fields (density, momentum; 250 us to make for 400 KB,
+    // which a handle that never asks for fields is spared)
     char* page = nullptr;
     char* page_dev = nullptr;       // the same, for kernels
-    bool page_coarse = false;       // the coarse fields have room in it
+    char* coarse_page = nullptr;
+    char* coarse_page_dev = nullptr;
     uint64_t seed = 0, step = 0, force_calls = 0;
     int force_dir = LGCA_FORCE_NONE;
     uint64_t force_thr = 0;
@@ -211,6 +214,18 @@ lgca_status ensure_mask(lgca_lattice* h)
         HIPCHK(h, dalloc(&h->row_range, (size_t)h->dim_y * 2 * 4));
     }
     return LGCA_OK;
+}
+
+// Pinned memory and its address for kernels, or null.
+char* pinned_page(size_t bytes, char** dev)
+{
+    void* p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) {
+        if (hipHostGetDevicePointer((void**)dev, p, 0) == hipSuccess) return (char*)p;
+        (void)hipHostFree(p);
+    }
+    (void)hipGetLastError();
+    return nullptr;
 }
 
 // Counters to the host.  A kernel writes them to pinned memory and clears them
@@ -334,21 +349,7 @@ extern "C" lgca_status lgca_create(lgca_lattice** out, int model, uint32_t dim_x
     if ((e = dalloc(&h->counters, kCounters * sizeof(unsigned long long))) != hipSuccess)
         return bail(hip_fail(h, e, "hipMalloc(counters)"));
     h->counters_used = true;
-    {
-        const size_t coarse = (size_t)(dim_x / (2 * coarse_radius)) * (dim_y / (2 * coarse_radius)) * 12;
-        h->page_coarse = coarse <= kPageMost;
-        // the row ranges (dim_y <= 65535) always have room
-        const size_t more = std::max(h->page_coarse ? coarse : 0, (size_t)dim_y * 8);
-        void* p = nullptr;
-        if (hipHostMalloc(&p, kPageMore + more, hipHostMallocDefault) == hipSuccess) {
-            h->page = (char*)p;
-            if (hipHostGetDevicePointer((void**)&h->page_dev, p, 0) != hipSuccess) {
-                (void)hipHostFree(p);
-                h->page = nullptr;
-            }
-        }
-        if (!h->page) (void)hipGetLastError();
-    }
+    h->page = pinned_page(kPageRanges + (size_t)dim_y * 8, &h->page_dev);
     const uint64_t nw = (uint64_t)h->state_words;
     if ((e = launch_fill_u32(h->state[0], 0u, nw, h->stream)) != hipSuccess ||
         (e = launch_fill_u32(h->state[1], 0u, nw, h->stream)) != hipSuccess ||
@@ -378,6 +379,7 @@ extern "C" lgca_status lgca_destroy(lgca_lattice* h)
         for (hipEvent_t ev : h->trial_ev) (void)hipEventDestroy(ev);
         h->copier.release();
         if (h->page) (void)hipHostFree(h->page);
+        if (h->coarse_page) (void)hipHostFree(h->coarse_page);
         if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
     }
     delete h;
@@ -498,7 +500,7 @@ static lgca_status upload_types(lgca_lattice* h, const uint8_t* types, hipMemcpy
     // The rows' ranges come through the page as well, under the flag's wait: a
     // copy of the runtime for each half took 40 us and more (2050 rows).
     if (h->page)
-        HIPCHK(h, launch_copy_u32((uint32_t*)(h->page_dev + kPageMore), (const uint32_t*)h->row_range,
+        HIPCHK(h, launch_copy_u32((uint32_t*)(h->page_dev + kPageRanges), (const uint32_t*)h->row_range,
                                   2u * (uint64_t)h->dim_y, h->stream));
     unsigned long long flag = 0;
     if ((st = read_counters(h, &flag, 1))) return st;
@@ -513,7 +515,7 @@ static lgca_status upload_types(lgca_lattice* h, const uint8_t* types, hipMemcpy
     h->row_lo.resize(h->dim_y);
     h->row_hi.resize(h->dim_y);
     if (h->page) {
-        const char* at = h->page + kPageMore;
+        const char* at = h->page + kPageRanges;
         std::memcpy(h->row_lo.data(), at, (size_t)h->dim_y * 4);
         std::memcpy(h->row_hi.data(), at + (size_t)h->dim_y * 4, (size_t)h->dim_y * 4);
         return LGCA_OK;
@@ -1624,9 +1626,12 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
         if (cell_density && !h->cell_density) HIPCHK(h, dalloc(&h->cell_density, n * 4));
         if (cell_momentum && !h->cell_momentum) HIPCHK(h, dalloc(&h->cell_momentum, n * 8));
     }
-    const bool coarse = mean_density || mean_momentum, page = h->page && h->page_coarse;
+    const bool coarse = mean_density || mean_momentum;
+    if (coarse && !h->coarse_page && nc * 12 <= kPageMost)
+        h->coarse_page = pinned_page(nc * 12, &h->coarse_page_dev);
+    const bool page = coarse && h->coarse_page;
     if (coarse) {
-        lgca_status st = run_coarse(h, page ? (float*)(h->page_dev + kPageMore) : nullptr);
+        lgca_status st = run_coarse(h, page ? (float*)h->coarse_page_dev : nullptr);
         if (st) return st;
     }
     if (cell_density || cell_momentum)
@@ -1638,7 +1643,7 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
     if (mean_momentum && !page) copies[n_copies++] = {mean_momentum, h->mean_momentum, nc * 8};
     HIPCHK(h, h->copier.run(copies, n_copies, h->stream));  // returns with the stream idle
     if (page) {
-        const char* at = h->page + kPageMore;
+        const char* at = h->coarse_page;
         if (mean_density) std::memcpy(mean_density, at, nc * 4);
         if (mean_momentum) std::memcpy(mean_momentum, at + nc * 4, nc * 8);
     }
