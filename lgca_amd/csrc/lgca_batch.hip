@@ -292,6 +292,9 @@ JobParams job_params(const lgca_job_desc& d)
     return p;
 }
 
+// Decision words of a step, 0 where nothing is forced.
+uint64_t force_words(const JobParams& p) { return p.forced ? (uint64_t)(p.fy1 - p.fy0) * p.fwn : 0; }
+
 JobLayout job_layout(const lgca_job_desc& d, const JobParams& p, size_t n_halfw)
 {
     JobLayout L{};
@@ -406,15 +409,6 @@ struct ClassRange {
     uint32_t heavy;  // leading items that can take the general walk
 };
 
-// Launch shape of a round: k steps per pass; walks (m 0) with tiles tall enough
-// for about `waves` waves, or blocks of m rows per wave and `waves` waves per
-// workgroup.
-struct Candidate {
-    int k;
-    uint32_t waves;
-    uint32_t m = 0;
-};
-
 }  // namespace
 
 struct lgca_batch {
@@ -480,9 +474,9 @@ struct lgca_batch {
     std::vector<Job*> finishing;        // post-processed, waiting for their event
 
     // autotuner (worker-private)
-    Candidate cur{4, 4096, 0};
+    RoundShape cur{4, 4096, 0};
     uint64_t mix_key = 0;               // jobs the block shape was predicted for
-    std::vector<Candidate> cands;
+    std::vector<RoundShape> cands;
     size_t cand_i = 0;
     int cand_rounds = 0;
     std::vector<hipEvent_t> tune_ev;    // start/end per candidate
@@ -549,7 +543,7 @@ std::string validate(const lgca_job_desc& d)
         // a pass reads its steps' decisions through one buffer descriptor
         const uint64_t x1 = std::min(d.fx1, d.dim_x), y1 = std::min(d.fy1, d.dim_y);
         if (d.fx0 < x1 && d.fy0 < y1 &&
-            (y1 - d.fy0) * ((x1 + 31) / 32 - d.fx0 / 32) * 8u * 4u >= (1ull << 31))
+            force_pass_steps((y1 - d.fy0) * ((x1 + 31) / 32 - d.fx0 / 32)) < 8)
             return "force region too large (the decisions of an 8-step pass must stay under 2 GiB)";
     }
     return "";
@@ -864,72 +858,14 @@ uint32_t tile_rows_for(uint64_t wave_rows_total, uint32_t waves)
     return (uint32_t)th;
 }
 
-// Blocks of a job's k-step round: rows per block, row tiles, blocks.
-struct JobBlocks {
-    uint32_t th, tiles, blocks;
-};
-JobBlocks job_blocks(const Geometry& g, const Candidate& c, int k)
+// The running jobs as the round planner sees them (lgca_plan.cpp).
+std::vector<RoundJob> round_jobs(const lgca_batch* b)
 {
-    const bool seg = tile_segments(g, k);
-    const uint32_t held = c.m * c.waves * (seg ? 64 / g.W : 1);
-    const uint32_t most = (held - 2 * block_halo(c.m, (uint32_t)k)) & ~1u;
-    JobBlocks b;
-    b.tiles = (g.dim_y + most - 1) / most;
-    b.th = (g.dim_y + b.tiles - 1) / b.tiles;
-    b.th += b.th & 1u;
-    b.tiles = (g.dim_y + b.th - 1) / b.th;
-    b.blocks = (uint32_t)block_count(g, k, b.tiles);
-    return b;
-}
-
-// Predicted time (us) of a round of the running jobs in blocks of shape c:
-// block_pass_us over a mix, whose blocks share the CUs.
-float mix_round_us(const lgca_batch* b, const Candidate& c)
-{
-    const uint32_t fit = std::max(1u, std::min(16u / c.waves, 160u * 1024u / block_lds_bytes(kFHP2, c.m, c.waves)));
-    float work = 0.0f, wait = 0.0f, most = 0.0f, bytes = 0.0f;
-    for (const Job* j : b->active) {
-        const Geometry& g = j->p.g;
-        const int k = (int)std::min<uint64_t>((uint64_t)c.k, j->d.steps - j->step);
-        const JobBlocks n = job_blocks(g, c, k);
-        const uint32_t S = tile_segments(g, k) ? 64 / g.W : 1, group = S * c.m, held = group * c.waves;
-        float row = j->p.kind == kHPP ? 0.045f : j->p.kind == kFHP1 ? 0.090f : 0.119f;
-        if (j->p.has_mask || j->p.forced) row *= 1.1f;
-        const float chain = (j->p.kind == kHPP ? 0.04f : 0.16f) * (float)c.m;
-        float bw = 0.0f, bl = 0.0f;  // one block's VALU time, and its time alone on a CU
-        for (int left = 0; left < k; ++left) {
-            const uint32_t rows = std::min(held, n.th + 2 * (uint32_t)left);
-            const float w = (float)((rows + group - 1) / group * c.m) / 4.0f * row;
-            bw += w;
-            bl += 0.08f + std::max(w, chain);
-        }
-        const float blocks = (float)n.blocks;
-        work += blocks * bw;
-        wait += blocks * (bl - bw + 1.5f);
-        most = std::max(most, bl);
-        bytes += blocks * (float)(held + n.th) / (float)S * 256.0f * (float)g.Q;
-    }
-    return 4.5f + std::max(most, work / 256.0f + wait / (256.0f * (float)fit)) + 0.5f * bytes / 4.5e6f;
-}
-
-// The block shapes a round may take, those with the least predicted time per
-// step first.  Steps are multiples of 4, so that a round of walks may follow,
-// and divide the force window when a job is forced.
-std::vector<Candidate> block_candidates(const lgca_batch* b)
-{
-    std::vector<std::pair<float, Candidate>> v;
-    const bool forced = std::any_of(b->active.begin(), b->active.end(), [](const Job* j) { return j->p.forced; });
-    for (int k = 4; k <= 24; k += 4)
-        for (uint32_t m : {2u, 4u})
-            for (uint32_t waves : {4u, 8u, 12u, 16u}) {
-                const Candidate c{k, waves, m};
-                if (m * waves < 2 * (uint32_t)k + 2 || (forced && kWindow % (uint32_t)k)) continue;
-                v.emplace_back(mix_round_us(b, c) / (float)k, c);
-            }
-    std::sort(v.begin(), v.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-    std::vector<Candidate> out;
-    for (const auto& x : v) out.push_back(x.second);
-    return out;
+    std::vector<RoundJob> v;
+    v.reserve(b->active.size());
+    for (const Job* j : b->active)
+        v.push_back(RoundJob{j->p.g, j->p.kind, j->p.has_mask || j->p.forced, force_words(j->p), j->d.steps - j->step});
+    return v;
 }
 
 // Whether a work item reading rows [a, b) of a job (on the torus) can take
@@ -962,7 +898,7 @@ bool rows_heavy(const Job* j, int64_t a, int64_t b)
 }
 
 // Builds this round's work items if the mix changed.
-void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th, const Candidate& shape)
+void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th, const RoundShape& shape)
 {
     const size_t n = b->active.size();
     b->sig.clear();
@@ -989,6 +925,8 @@ void build_round(lgca_batch* b, const std::vector<int>& ks, uint32_t th, const C
         const uint32_t halo = seg ? 0u : tile_halo(g, k);
         if (shape.m) {
             // a launch for every k: the items hold their job's
+            if ((uint64_t)k > force_pass_steps(force_words(j->p)))
+                throw WorkerError{"a round's force decisions reach 2 GiB"};
             const JobBlocks n = job_blocks(g, shape, k);
             const uint64_t key = g.nb != 32 ? 1u : 0u;
             std::vector<WorkItem>& vh = cls[key];
@@ -1114,23 +1052,23 @@ void start_tuning(lgca_batch* b, int user_k, uint32_t user_waves, uint64_t wr)
     if (!user_k && !user_waves) {
         // the blocks predicted fastest against the walks that win on mixes
         // which fill the GPU
-        const std::vector<Candidate> blocks = block_candidates(b);
+        const std::vector<RoundShape> blocks = round_shapes(round_jobs(b), kWindow);
         for (size_t i = 0; i < blocks.size() && i < 3; ++i) b->cands.push_back(blocks[i]);
         for (int k : ks)
-            for (uint32_t w : {2048u, 4096u}) b->cands.push_back(Candidate{k, w});
+            for (uint32_t w : {2048u, 4096u}) b->cands.push_back(RoundShape{k, w});
     } else {
         for (int k : ks) {
             if (user_k && k != user_k) continue;
             for (uint32_t w : ws) {
                 if (user_waves && w != user_waves) continue;
-                b->cands.push_back(Candidate{k, w});
+                b->cands.push_back(RoundShape{k, w});
             }
         }
     }
     if (user_k && b->cands.empty())
         for (uint32_t w : ws)
-            if (!user_waves || w == user_waves) b->cands.push_back(Candidate{user_k, w});
-    if (user_waves && b->cands.empty()) b->cands.push_back(Candidate{user_k ? user_k : 4, user_waves});
+            if (!user_waves || w == user_waves) b->cands.push_back(RoundShape{user_k, w});
+    if (user_waves && b->cands.empty()) b->cands.push_back(RoundShape{user_k ? user_k : 4, user_waves});
     b->tuned_wave_rows = wr;
     b->rounds_since_tune = 0;
     if (b->cands.size() <= 1) {
@@ -1198,7 +1136,7 @@ void run_round(lgca_batch* b)
         for (const Job* j : b->active) key = key * 0x100000001B3ull ^ j->id;
         if (key != b->mix_key) {
             b->mix_key = key;
-            b->cur = block_candidates(b).front();
+            b->cur = round_shapes(round_jobs(b), kWindow).front();
         }
         b->tuned_wave_rows = 0;  // a mix that grows past this is tuned at once
     } else if (!b->tuning && !b->evaluating) {
@@ -1217,12 +1155,12 @@ void run_round(lgca_batch* b)
     for (size_t i = 0; i < n; ++i) {
         const Job* j = b->active[i];
         // (blocks may start a pass at any step)
-        ks[i] = b->cur.m ? (int)std::min<uint64_t>((uint64_t)b->cur.k, j->d.steps - j->step)
+        ks[i] = b->cur.m ? round_steps(b->cur, j->d.steps - j->step, force_words(j->p))
                          : pick_k(b->cur.k, j->d.steps - j->step, j->step);
         su += (uint64_t)j->d.dim_x * j->d.dim_y * (uint64_t)ks[i];
     }
     const uint32_t th = b->cur.m ? 0 : tile_rows_for(wave_rows(b, b->cur.k), b->cur.waves);
-    const Candidate shape = b->cur;
+    const RoundShape shape = b->cur;
     build_round(b, ks, th, shape);
     draw_windows(b, ks);
 

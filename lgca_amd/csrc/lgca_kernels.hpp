@@ -174,6 +174,10 @@ float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32
 std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k);
 // Whether passes of this lattice are better held in blocks than walked.
 bool block_lattice(const Geometry& g);
+// Most steps of a pass whose force decisions, `words` of them a step, stay below
+// 2 GiB: a pass reads them through one buffer descriptor, past whose end the
+// offsets of unforced words must lie (kOutside in lgca_block.hpp).
+inline uint64_t force_pass_steps(uint64_t words) { return words ? (((uint64_t)1 << 31) - 1) / (4 * words) : UINT64_MAX; }
 hipError_t launch_block(int kind, const BlockShape& s, const BlockArgs& b, hipStream_t st);
 template <int KIND, int M>
 hipError_t launch_block_km(const BlockArgs& b, uint32_t waves, uint32_t blocks, bool ragged, int seg, hipStream_t s);
@@ -218,6 +222,35 @@ inline uint32_t block_shape_bits(uint32_t th, uint32_t halo, uint32_t k, BlockLa
 }
 hipError_t launch_tile_batch(int k, bool ragged, const BatchJob* jobs, BatchState* state,
                              const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s);
+
+// Launch shape of a batch's round: k steps per pass; walks (m 0) with tiles tall
+// enough for about `waves` waves, or blocks of m rows per wave and `waves` waves
+// per workgroup.
+struct RoundShape {
+    int k;
+    uint32_t waves;
+    uint32_t m = 0;
+};
+// What the shape of a round of blocks depends on of a running job.
+struct RoundJob {
+    Geometry g;
+    int kind;
+    bool feat;             // solids or forcing
+    uint64_t force_words;  // decision words of a step (0: not forced)
+    uint64_t left;         // steps to go
+};
+// Blocks of a job's k-step round: rows per block, row tiles, blocks.
+struct JobBlocks {
+    uint32_t th, tiles, blocks;
+};
+JobBlocks job_blocks(const Geometry& g, const RoundShape& s, int k);
+// Steps that a job with `left` to go makes in a round of blocks of shape s.
+int round_steps(const RoundShape& s, uint64_t left, uint64_t force_words);
+// Predicted time (us) of a round of the jobs in blocks of shape s.
+float round_us(const std::vector<RoundJob>& jobs, const RoundShape& s);
+// The block shapes that a round of the jobs may take, those with the least
+// predicted time per step first; never none.  window: steps of a force window.
+std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window);
 
 // Launchers of one (model, K) pair and of one K's batch kernel, instantiated
 // by lgca_tile_inst.hip; grid and shapes come checked from launch_tile /

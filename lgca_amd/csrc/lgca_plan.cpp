@@ -1,6 +1,6 @@
 // lgca_plan.cpp -- host-only launch planning: lattice geometry, the tiled
-// step's halo and strip counts, the strip-mode wave dispatch order and the
-// band plan of multi-pass launches.  Plain C++ (no device code), so that test
+// step's halo and strip counts, the strip-mode wave dispatch order, the band
+// plan of multi-pass launches, and the shapes of block passes and rounds.  Plain C++ (no device code), so that test
 // programs can build it with the host compiler and check the plans without a
 // GPU.
 #include "lgca_kernels.hpp"
@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdint>
+#include <utility>
 
 namespace lgca {
 
@@ -292,6 +293,83 @@ float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32
     // them overlap other blocks' steps
     const float bytes = (float)blocks * (float)((s.m * s.waves) + (s.th + S - 1) / S) * 256.0f * (float)g.Q;
     return 3.2f + (feat ? 1.3f : 0.0f) + (float)rounds * us + 0.5f * bytes / 4.5e6f;
+}
+
+// ------------------------------------------------- rounds of a batch in blocks
+
+JobBlocks job_blocks(const Geometry& g, const RoundShape& s, int k)
+{
+    const bool seg = tile_segments(g, k);
+    const uint32_t held = s.m * s.waves * (seg ? 64 / g.W : 1);
+    const uint32_t most = (held - 2 * block_halo(s.m, (uint32_t)k)) & ~1u;
+    JobBlocks b;
+    b.tiles = (g.dim_y + most - 1) / most;
+    b.th = (g.dim_y + b.tiles - 1) / b.tiles;
+    b.th += b.th & 1u;
+    b.tiles = (g.dim_y + b.th - 1) / b.th;
+    b.blocks = (uint32_t)block_count(g, k, b.tiles);
+    return b;
+}
+
+// A shape chosen before a job with a large force region came may have more
+// steps than that job's decisions allow.  Jobs are accepted with 8 or more, and
+// a multiple of 4 keeps the job's step one, as walks need it.
+int round_steps(const RoundShape& s, uint64_t left, uint64_t force_words)
+{
+    uint64_t k = (uint64_t)s.k;
+    if (force_pass_steps(force_words) < k) k = force_pass_steps(force_words) & ~(uint64_t)3;
+    return (int)std::min(k, left);
+}
+
+// block_pass_us over a mix, whose blocks share the CUs.
+float round_us(const std::vector<RoundJob>& jobs, const RoundShape& s)
+{
+    const uint32_t fit = std::max(1u, std::min(16u / s.waves, 160u * 1024u / block_lds_bytes(2, s.m, s.waves)));
+    float work = 0.0f, wait = 0.0f, most = 0.0f, bytes = 0.0f;
+    for (const RoundJob& j : jobs) {
+        const Geometry& g = j.g;
+        const int k = round_steps(s, j.left, j.force_words);
+        const JobBlocks n = job_blocks(g, s, k);
+        const uint32_t S = tile_segments(g, k) ? 64 / g.W : 1, group = S * s.m, held = group * s.waves;
+        float row = j.kind == 0 ? 0.045f : j.kind == 1 ? 0.090f : 0.119f;
+        if (j.feat) row *= 1.1f;
+        const float chain = (j.kind == 0 ? 0.04f : 0.16f) * (float)s.m;
+        float bw = 0.0f, bl = 0.0f;  // one block's VALU time, and its time alone on a CU
+        for (int left = 0; left < k; ++left) {
+            const uint32_t rows = std::min(held, n.th + 2 * (uint32_t)left);
+            const float w = (float)((rows + group - 1) / group * s.m) / 4.0f * row;
+            bw += w;
+            bl += 0.08f + std::max(w, chain);
+        }
+        const float blocks = (float)n.blocks;
+        work += blocks * bw;
+        wait += blocks * (bl - bw + 1.5f);
+        most = std::max(most, bl);
+        bytes += blocks * (float)(held + n.th) / (float)S * 256.0f * (float)g.Q;
+    }
+    return 4.5f + std::max(most, work / 256.0f + wait / (256.0f * (float)fit)) + 0.5f * bytes / 4.5e6f;
+}
+
+// Steps are multiples of 4, so that a round of walks may follow, and with a
+// forced job they divide the window and keep its decisions in bounds.
+std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window)
+{
+    std::vector<std::pair<float, RoundShape>> v;
+    uint64_t most_words = 0;
+    for (const RoundJob& j : jobs) most_words = std::max(most_words, j.force_words);
+    for (int k = 4; k <= 24; k += 4) {
+        if (most_words && (window % (uint32_t)k || (uint64_t)k > force_pass_steps(most_words))) continue;
+        for (uint32_t m : {2u, 4u})
+            for (uint32_t waves : {4u, 8u, 12u, 16u}) {
+                const RoundShape s{k, waves, m};
+                if (m * waves < 2 * (uint32_t)k + 2) continue;
+                v.emplace_back(round_us(jobs, s) / (float)k, s);
+            }
+    }
+    std::sort(v.begin(), v.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+    std::vector<RoundShape> out;
+    for (const auto& x : v) out.push_back(x.second);
+    return out;
 }
 
 }  // namespace lgca

@@ -73,7 +73,7 @@ hipError_t launch_block(int kind, const BlockShape& sh, const BlockArgs& b, hipS
     if (b.a.th < 2 || (b.a.th & 1u) || (m > 1 && (b.hk & 1u)) || b.hk < b.k || held < b.a.th + 2 * b.hk)
         return hipErrorInvalidValue;
     if (!seg && (b.a.halo < tile_halo(g, (int)b.k) || b.a.halo > 16 || b.k > 32)) return hipErrorInvalidValue;
-    if (b.a.fdec && (uint64_t)b.k * b.a.fdec_stride * 4u >= ((uint64_t)1 << 31)) return hipErrorInvalidValue;
+    if (b.a.fdec && b.k > force_pass_steps(b.a.fdec_stride)) return hipErrorInvalidValue;
     const uint64_t blocks = block_count(g, (int)b.k, (g.dim_y + b.a.th - 1) / b.a.th);
     if (blocks >= ((uint64_t)1 << 31) || blocks % b.nstrips) return hipErrorInvalidValue;
     const bool ragged = g.nb != 32;
