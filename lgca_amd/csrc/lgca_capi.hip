@@ -1627,9 +1627,11 @@ extern "C" lgca_status lgca_post_process(lgca_lattice* h, float* cell_density, f
         if (cell_momentum && !h->cell_momentum) HIPCHK(h, dalloc(&h->cell_momentum, n * 8));
     }
     const bool coarse = mean_density || mean_momentum;
-    if (coarse && !h->coarse_page && nc * 12 <= kPageMost)
+    // (other than ordinary memory the runtime copies to itself)
+    const bool ordinary = coarse && (!mean_density || pageable(mean_density)) && (!mean_momentum || pageable(mean_momentum));
+    if (ordinary && !h->coarse_page && nc * 12 <= kPageMost)
         h->coarse_page = pinned_page(nc * 12, &h->coarse_page_dev);
-    const bool page = coarse && h->coarse_page;
+    const bool page = ordinary && h->coarse_page;
     if (coarse) {
         lgca_status st = run_coarse(h, page ? (float*)h->coarse_page_dev : nullptr);
         if (st) return st;
