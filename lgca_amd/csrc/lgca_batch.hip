@@ -413,6 +413,7 @@ struct ClassRange {
 
 struct lgca_batch {
     int device = 0;
+    uint32_t ncu = 0;                   // CUs of the device
     uint64_t budget = 0;
     hipStream_t stream = nullptr;       // worker: set-up and rounds
     hipStream_t post_stream = nullptr;  // worker: post-processing of finished jobs
@@ -780,7 +781,7 @@ void finish(lgca_batch* b, Job* j)
     j->last_ev = take_event(b);
     hipchk(hipEventRecord(j->last_ev, b->stream), "hipEventRecord");
     hipchk(hipStreamWaitEvent(b->post_stream, j->last_ev, 0), "hipStreamWaitEvent");
-    hipchk(launch_coarse(p.kind, st, p.g, j->d.coarse_radius, (float*)(m + j->L.md), (float*)(m + j->L.mm),
+    hipchk(launch_coarse(p.kind, st, p.g, j->d.coarse_radius, b->ncu, (float*)(m + j->L.md), (float*)(m + j->L.mm),
                          (float*)(m + j->L.vel), nullptr, b->post_stream),
            "coarse");
     hipchk(launch_unpack(st, (uint8_t*)(m + j->L.bytes), p.g, b->post_stream), "unpack");
@@ -1330,6 +1331,9 @@ extern "C" lgca_status lgca_batch_create(lgca_batch** out, int device, uint64_t 
     b->budget = hbm_budget_bytes;
     b->arena.block_bytes = (size_t)std::min<uint64_t>((uint64_t)1 << 30, align_up(hbm_budget_bytes));
     DevGuard dg(device);
+    int ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && ncu >= 1)
+        b->ncu = (uint32_t)ncu;
     auto fail = [&](hipError_t e, const char* what) {
         g_batch_create_error = std::string(what) + ": " + hipGetErrorString(e);
         lgca_batch_destroy(b);

@@ -1607,7 +1607,7 @@ static lgca_status run_coarse(lgca_lattice* h, float* host = nullptr)
         HIPCHK(h, dalloc(&h->mean_momentum, nc * 8));
         HIPCHK(h, dalloc(&h->velocity, nc * 8));
     }
-    HIPCHK(h, launch_coarse(h->kind, h->snap, h->g, h->r, h->mean_density, h->mean_momentum,
+    HIPCHK(h, launch_coarse(h->kind, h->snap, h->g, h->r, h->ncu, h->mean_density, h->mean_momentum,
                             h->velocity, host, h->stream));
     return LGCA_OK;
 }

@@ -633,8 +633,6 @@ hipError_t launch_cell_fields(int kind, const uint32_t* planes, const Geometry& 
 // loads' latency count), 26 us so (4400 x 2200 at r = 20: 113, 25 and 15 us;
 // 1480 x 740 at r = 10: 36, 9.9 and 7.8 us).  The producers' arithmetic bounds
 // it: loads two stages ahead in place of one make no difference.
-constexpr uint32_t kCoarseExactRadius = 1023;
-constexpr uint32_t kCoarseProducers = 7, kCoarseColumns = 36, kChainAhead = 4;
 
 // Addends of the y-momentum chain for the cells of one unit, zeros past its
 // end: bit j of the four planes is cell j; out[j] = ky * sin(pi/3), ky = a1 + a2 - a4 - a5,
@@ -799,10 +797,11 @@ void coarse_kernel(const uint32_t* __restrict__ planes, Geometry g, uint32_t r, 
     }
 }
 
-// The same one cell at a time, one thread per coarse cell, for radii whose
-// density sums FP32 may round (more than 2^24 particles in a window).
+// The same one cell at a time, one thread per coarse cell: for radii whose
+// density sums FP32 may round (more than 2^24 particles in a window), and where
+// many small cells fill the GPU with lanes (coarse_in_units).
 template <int KIND>
-__global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __restrict__ planes,
+__global__ __launch_bounds__(64) void coarse_lane_kernel(const uint32_t* __restrict__ planes,
                                                           Geometry g, uint32_t r,
                                                           float* __restrict__ md, float* __restrict__ mm,
                                                           float* __restrict__ vel, float* __restrict__ host)
@@ -862,31 +861,25 @@ __global__ __launch_bounds__(64) void coarse_large_kernel(const uint32_t* __rest
     }
 }
 
-hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, uint32_t r,
+hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, uint32_t r, uint32_t ncu,
                          float* mean_density, float* mean_momentum, float* velocity, float* host, hipStream_t s)
 {
     const uint32_t n = (g.dim_x / (2 * r)) * (g.dim_y / (2 * r));
     const dim3 grid(div_up(n, 64));
-    if (r > kCoarseExactRadius) {
+    if (!coarse_in_units(kind, r, n, ncu)) {
         switch (kind) {
-        case kHPP: hipLaunchKernelGGL(coarse_large_kernel<kHPP>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
-        case kFHP1: hipLaunchKernelGGL(coarse_large_kernel<kFHP1>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
-        default: hipLaunchKernelGGL(coarse_large_kernel<kFHP2>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
+        case kHPP: hipLaunchKernelGGL(coarse_lane_kernel<kHPP>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
+        case kFHP1: hipLaunchKernelGGL(coarse_lane_kernel<kFHP1>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
+        default: hipLaunchKernelGGL(coarse_lane_kernel<kFHP2>, grid, dim3(64), 0, s, planes, g, r, mean_density, mean_momentum, velocity, host); break;
         }
         return hipGetLastError();
     }
-    // the r + 1 columns in units of at most kCoarseColumns, of about equal size,
-    // whole quads of addends: two stages of them take 126 KiB of LDS at most
-    const uint32_t chunks = (r + kCoarseColumns) / kCoarseColumns;
-    const uint32_t chunk = ((r + 1 + chunks - 1) / chunks + 3) & ~3u;
-    const uint32_t used = (r + chunk) / chunk;  // chunks that hold a column
+    const CoarseUnits u = coarse_units(kind, r);
     const dim3 block(64 * (1 + kCoarseProducers));
-    // (the chain reads up to three times kChainAhead quads past the last one)
-    const size_t lds = kind == kHPP ? 0 : (size_t)(2 * kCoarseProducers * chunk + 3 * 4 * kChainAhead) * 64 * sizeof(float);
     switch (kind) {
-    case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity, host); break;
-    case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity, host); break;
-    default: hipLaunchKernelGGL(coarse_kernel<kFHP2>, grid, block, lds, s, planes, g, r, used, chunk, mean_density, mean_momentum, velocity, host); break;
+    case kHPP: hipLaunchKernelGGL(coarse_kernel<kHPP>, grid, block, u.lds, s, planes, g, r, u.chunks, u.chunk, mean_density, mean_momentum, velocity, host); break;
+    case kFHP1: hipLaunchKernelGGL(coarse_kernel<kFHP1>, grid, block, u.lds, s, planes, g, r, u.chunks, u.chunk, mean_density, mean_momentum, velocity, host); break;
+    default: hipLaunchKernelGGL(coarse_kernel<kFHP2>, grid, block, u.lds, s, planes, g, r, u.chunks, u.chunk, mean_density, mean_momentum, velocity, host); break;
     }
     return hipGetLastError();
 }

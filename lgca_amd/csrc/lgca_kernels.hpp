@@ -305,7 +305,19 @@ hipError_t launch_init_fill(uint32_t* planes, const uint32_t* mask, const uint8_
                             hipStream_t s);
 hipError_t launch_cell_fields(int kind, const uint32_t* planes, const Geometry& g,
                               float* density, float* momentum, hipStream_t s);
-hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, uint32_t r,
+// Coarse fields.  One kernel takes 64 coarse cells a workgroup, its producers
+// reading the rows in units of columns (up to kCoarseExactRadius, whose sums FP32
+// holds exactly); the other a lane per coarse cell.
+constexpr uint32_t kCoarseExactRadius = 1023;
+constexpr uint32_t kCoarseProducers = 7, kCoarseColumns = 36, kChainAhead = 4;
+struct CoarseUnits {
+    uint32_t chunks, chunk;  // units of a row and columns of a unit
+    uint32_t lds;            // bytes
+};
+CoarseUnits coarse_units(int kind, uint32_t r);
+// Whether the first is predicted to be the faster for `cells` coarse cells.
+bool coarse_in_units(int kind, uint32_t r, uint64_t cells, uint32_t ncu);
+hipError_t launch_coarse(int kind, const uint32_t* planes, const Geometry& g, uint32_t r, uint32_t ncu,
                          float* mean_density, float* mean_momentum, float* velocity,
                          float* host, hipStream_t s);  // host: null, or density then momentum once more
 hipError_t launch_count(const uint32_t* words, uint64_t nwords, unsigned long long* out,

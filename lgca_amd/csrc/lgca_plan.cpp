@@ -372,4 +372,44 @@ std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t
     return out;
 }
 
+// ------------------------------------------------------------- coarse fields
+
+CoarseUnits coarse_units(int kind, uint32_t r)
+{
+    // the r + 1 columns in units of at most kCoarseColumns, of about equal size,
+    // whole quads of addends: two stages of them take 126 KiB of LDS at most
+    const uint32_t chunks = (r + kCoarseColumns) / kCoarseColumns;
+    CoarseUnits u;
+    u.chunk = ((r + 1 + chunks - 1) / chunks + 3) & ~3u;
+    u.chunks = (r + u.chunk) / u.chunk;  // those that hold a column
+    // (the chain reads up to three times kChainAhead quads past the last one)
+    u.lds = kind == 0 ? 0 : (2 * kCoarseProducers * u.chunk + 3 * 4 * kChainAhead) * 64 * 4;
+    return u;
+}
+
+// Predicted times of the two kernels.  In units a workgroup's stages follow each
+// other, so the time goes by rounds of workgroups on the CUs; a lane per
+// coarse cell waits for its chain, or, with enough of them, for the cells'
+// arithmetic.  FHP-II, us in units / a lane each: 4096 x 2048 at r = 1 137.5 / 22.2,
+// r = 4 18.3 / 10.5, r = 6 11.4 / 16.0, r = 16 11.6 / 63; 8192 x 4096 at r = 2
+// 140 / 36.8, r = 5 41.1 / 31.8, r = 8 29.3 / 25.6, r = 16 21.4 / 69; 32768 x
+// 8192 at r = 16 154 / 125, r = 32 98 / 247.  On none of 248 sizes (HPP, FHP-I and
+// FHP-II, 512 x 256 to 32768 x 8192, r 1 to 32) does it take a kernel that is
+// more than a twentieth slower than the other.
+bool coarse_in_units(int kind, uint32_t r, uint64_t cells, uint32_t ncu)
+{
+    if (r > kCoarseExactRadius) return false;
+    const float wgs = (float)((cells + 63) / 64), cus = (float)std::max(ncu, 1u);
+    if (wgs <= cus) return true;
+    const CoarseUnits u = coarse_units(kind, r);
+    const uint32_t stages = ((2 * r + 1) * u.chunks + kCoarseProducers - 1) / kCoarseProducers;
+    const uint32_t fit = std::min(4u, 160u * 1024u / (u.lds + 6u * 1024u));
+    const float wg = kind == 0 ? 2.8f + 1.1f * (float)stages : 4.2f + 0.06f * (float)(stages * u.chunk);
+    const float units = 1.8f + wg * std::max(1.0f, wgs / (cus * (float)fit));
+    const float visits = (float)(2 * r + 1) * (float)(r + 1);
+    const float latency = 4.5f + (kind == 0 ? 0.075f : 0.1f) * visits;
+    const float flow = wgs * (0.077f + 0.013f * visits) / cus;
+    return units * units <= latency * latency + flow * flow;
+}
+
 }  // namespace lgca
