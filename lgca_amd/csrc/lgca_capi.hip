@@ -1085,7 +1085,8 @@ static const PipeCache* pipe_plan(lgca_lattice* h, int k, const TileArgs& a)
 }
 
 // Whether lgca_step runs passes in blocks (lgca_block.hpp): with automatic
-// steps and rows, on lattices that walks cannot fill the GPU with.
+// steps and rows, on lattices that walks cannot fill the GPU with (but for
+// calls of a few steps, short_walk_rows).
 static bool uses_blocks(const lgca_lattice* h)
 {
     return h->tile_k == kAutoSteps && !h->tile_th && block_lattice(h->g);
@@ -1388,10 +1389,13 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
     if (blocks) plan_blocks(h);
     while (left > 0) {
         int k = 1, ev_start = -1, ev_end = -1;
-        uint32_t th = 0;
-        if (blocks) {
+        uint32_t th = blocks ? short_walk_rows(h->g, h->kind, left) : 0;
+        const bool block = blocks && !th;
+        if (block) {
             k = (int)block_steps(h, left);
             if (forcing && ext_dec) k = (int)std::min<uint64_t>((uint64_t)k, ext_words / per_step);
+        } else if (blocks) {
+            k = (int)left;  // a walk
         } else if (h->tile_k != 0 && ext_dec) {
             const LaunchShape sh = kept_shape(h);
             k = steps_for_launch(sh.k, left);
@@ -1404,7 +1408,7 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
         // descriptor of under 2 GiB: lattices whose forced region is larger
         // than that per pass (some 2 G forced cells at 8 steps) take fewer
         // steps per pass (a trial launch so cut is timed with its group).
-        if (forcing && !blocks && h->tile_k != 0 && (uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes) {
+        if (forcing && !block && h->tile_k != 0 && (uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes) {
             while (k > 1 && (uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes) k /= 2;
             if ((uint64_t)k * per_step * 4u >= kMaxPassDecisionBytes)
                 return fail(h, LGCA_ERR_INVALID_ARGUMENT, "lgca_step: the force region's decisions of one step exceed 2 GiB");
@@ -1479,7 +1483,7 @@ static lgca_status step_locked(lgca_lattice* h, uint64_t nsteps, uint32_t* ext_d
             left -= span;
             continue;
         }
-        if (blocks) {
+        if (block) {
             HIPCHK(h, launch_block_pass(h, (uint32_t)k, h->block[k], fdec, (uint32_t)h->step));
         } else if (h->tile_k == 0) {
             StepArgs a{};

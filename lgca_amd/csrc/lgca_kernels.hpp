@@ -174,6 +174,9 @@ float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32
 std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k);
 // Whether passes of this lattice are better held in blocks than walked.
 bool block_lattice(const Geometry& g);
+// Rows per tile of the walk that a whole call of `steps` steps had better be on
+// such a lattice, or 0.
+uint32_t short_walk_rows(const Geometry& g, int kind, uint64_t steps);
 // Most steps of a pass whose force decisions, `words` of them a step, stay below
 // 2 GiB: a pass reads them through one buffer descriptor, past whose end the
 // offsets of unforced words must lie (kOutside in lgca_block.hpp).

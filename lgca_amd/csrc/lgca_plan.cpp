@@ -229,8 +229,14 @@ uint64_t block_count(const Geometry& g, int k, uint32_t tiles)
     return ((uint64_t)tiles * (g.W + 2 * h) + stride - 1) / stride;
 }
 
-// Lattices of up to 36 wave-rows (64 words of a row, packed as the blocks have
-// them) per SIMD.  us per step in blocks / walked, FHP-II: 4400 x 2200 1.7 /
+// Rows of 64 words (or the whole rows that a wave holds), packed as the blocks
+// have them.
+static uint64_t block_wave_rows(const Geometry& g)
+{
+    return tile_segments(g, 8) ? (uint64_t)g.dim_y / (64 / g.W) : block_count(g, 8, g.dim_y);
+}
+
+// Lattices of up to 36 wave-rows per SIMD.  us per step in blocks / walked, FHP-II: 4400 x 2200 1.7 /
 // 2.9, 8192 x 4096 (17,045 wave-rows) 3.2 / 4.8, 12000 x 4000 (24,323) 4.7 /
 // 5.2, 32768 x 2048 (33,891) 5.8 / 6.0, 12000 x 6000 (36,484) 6.0 / 6.4, 13001 x
 // 6000 (39,581) 8.3 / 8.0 with walls and forced columns, 16384 x
@@ -238,8 +244,27 @@ uint64_t block_count(const Geometry& g, int k, uint32_t tiles)
 // and compute fewer halo rows.
 bool block_lattice(const Geometry& g)
 {
-    const uint64_t wave_rows = tile_segments(g, 8) ? (uint64_t)g.dim_y / (64 / g.W) : block_count(g, 8, g.dim_y);
-    return wave_rows < 36864;
+    return block_wave_rows(g) < 36864;
+}
+
+// A call of 1, 2 or 4 steps is one pass either way.  A block pass starts all its
+// loads at once and stores only when its steps are done, so on many rows, for few
+// steps, walks over tiles of 4 or 8 rows, whose loads and stores overlap, are
+// faster; other counts take a walk two launches or more.  us per call in
+// blocks / walked: 4096 x 2048 FHP-II (4,295 wave-rows) 1 step 6.7 / 6.0, 2 steps
+// 7.4 / 7.2, 4 steps 9.2 / 10.9; 6000 x 3000 (9,194) 11.0 / 8.6, 11.7 / 10.1, 13.5 /
+// 14.9; 7000 x 3500 with walls (12,476) 14.9 / 10.2, 16.6 / 11.2, 18.2 / 16.3;
+// 8192 x 4096 (17,045) 16.1 / 11.7, 17.1 / 12.6, 22.1 / 18.6, HPP 8.8 / 7.6, 9.1 / 8.3,
+// 11.7 / 9.2; 12000 x 5800 forced everywhere (35,268) 41.3 / 36.3, 54 / 40, 53 /
+// 51.  Blocks keep flat lattices (1000000 x 16, 1 step 5.5 / 6.7) and HPP rows that
+// a wave holds whole (2048 x 16384, 4 steps 8.7 / 10.0).
+uint32_t short_walk_rows(const Geometry& g, int kind, uint64_t steps)
+{
+    if (steps != 1 && steps != 2 && steps != 4) return 0;
+    if (g.dim_y < 256 || (kind == 0 && tile_segments(g, (int)steps))) return 0;
+    const uint64_t wave_rows = block_wave_rows(g);
+    if (wave_rows < (steps == 4 ? 12288 : 4096 * steps)) return 0;
+    return wave_rows < 8192 ? 4 : 8;
 }
 
 std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k)

@@ -48,9 +48,32 @@ static void check_coarse()
     }
 }
 
+static void check_short_calls()
+{
+    struct {
+        int kind;
+        uint32_t dim_x, dim_y;
+        bool walk[3];  // 1, 2, 4 steps
+    } cases[] = {
+        {2, 2048, 2048, {false, false, false}}, {0, 2048, 512, {false, false, false}}, {2, 4096, 2048, {true, false, false}},
+        {2, 6000, 3000, {true, true, false}},   {2, 7000, 3500, {true, true, true}},   {0, 8192, 4096, {true, true, true}},
+        {1, 8192, 4096, {true, true, true}},    {2, 12000, 5800, {true, true, true}},  {2, 512, 65534, {true, true, true}},
+        {0, 2048, 16384, {false, false, false}}, {2, 1000000, 16, {false, false, false}}, {0, 1000000, 64, {false, false, false}}};
+    for (const auto& c : cases) {
+        const Geometry g = make_geometry(c.dim_x, c.dim_y, c.kind == 0 ? 4 : c.kind == 1 ? 6 : 7);
+        CHECK(block_lattice(g), "%u x %u runs in blocks", c.dim_x, c.dim_y);
+        for (uint32_t i = 0; i < 3; ++i) {
+            const uint32_t th = short_walk_rows(g, c.kind, 1u << i);
+            CHECK((th != 0) == c.walk[i] && th % 2 == 0 && th <= g.dim_y, "kind %d, %u x %u, %u steps", c.kind, c.dim_x, c.dim_y, 1u << i);
+        }
+        for (uint64_t n : {0u, 3u, 5u, 6u, 7u, 8u, 12u, 100u}) CHECK(!short_walk_rows(g, c.kind, n), "a walk of %u steps", (uint32_t)n);
+    }
+}
+
 int main()
 {
     check_coarse();
+    check_short_calls();
     if (failures) {
         std::printf("%d checks failed\n", failures);
         return 1;
