@@ -1089,7 +1089,7 @@ static const PipeCache* pipe_plan(lgca_lattice* h, int k, const TileArgs& a)
 // calls of a few steps, short_walk_rows).
 static bool uses_blocks(const lgca_lattice* h)
 {
-    return h->tile_k == kAutoSteps && !h->tile_th && block_lattice(h->g);
+    return h->tile_k == kAutoSteps && !h->tile_th && block_lattice(h->g, h->mask != nullptr);
 }
 
 // Decides the block shapes from the pass-time model: the best for every number

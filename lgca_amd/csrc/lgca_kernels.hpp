@@ -173,7 +173,7 @@ float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32
 // out equal.
 std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k);
 // Whether passes of this lattice are better held in blocks than walked.
-bool block_lattice(const Geometry& g);
+bool block_lattice(const Geometry& g, bool solids);
 // Rows per tile of the walk that a whole call of `steps` steps had better be on
 // such a lattice, or 0.
 uint32_t short_walk_rows(const Geometry& g, int kind, uint64_t steps);

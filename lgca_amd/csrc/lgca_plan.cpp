@@ -242,8 +242,12 @@ static uint64_t block_wave_rows(const Geometry& g)
 // 6000 (39,581) 8.3 / 8.0 with walls and forced columns, 16384 x
 // 8192 (67,914) 11.2 / 9.5: the larger ones fill the GPU with walks, which read
 // and compute fewer halo rows.
-bool block_lattice(const Geometry& g)
+// Nor do flat ones whose strips alone do, without solids: 4000000 x 2 FHP-II 3.3
+// us a step in blocks and 2.3 walked, x 4 3.8 / 2.9, x 6 4.3 / 4.8, 2000000 x 2 1.97 /
+// 1.82, x 4 2.2 / 2.3, 4000000 x 4 with walls 4.2 / 4.7.
+bool block_lattice(const Geometry& g, bool solids)
 {
+    if (g.dim_y <= 4 && !solids && !tile_segments(g, 8) && tile_strips(g, 8) >= 500 * g.dim_y) return false;
     return block_wave_rows(g) < 36864;
 }
 

@@ -61,7 +61,7 @@ static void check_short_calls()
         {0, 2048, 16384, {false, false, false}}, {2, 1000000, 16, {false, false, false}}, {0, 1000000, 64, {false, false, false}}};
     for (const auto& c : cases) {
         const Geometry g = make_geometry(c.dim_x, c.dim_y, c.kind == 0 ? 4 : c.kind == 1 ? 6 : 7);
-        CHECK(block_lattice(g), "%u x %u runs in blocks", c.dim_x, c.dim_y);
+        CHECK(block_lattice(g, false) && block_lattice(g, true), "%u x %u runs in blocks", c.dim_x, c.dim_y);
         for (uint32_t i = 0; i < 3; ++i) {
             const uint32_t th = short_walk_rows(g, c.kind, 1u << i);
             CHECK((th != 0) == c.walk[i] && th % 2 == 0 && th <= g.dim_y, "kind %d, %u x %u, %u steps", c.kind, c.dim_x, c.dim_y, 1u << i);
@@ -70,8 +70,25 @@ static void check_short_calls()
     }
 }
 
+static void check_block_lattices()
+{
+    struct {
+        uint32_t dim_x, dim_y;
+        bool open, solids;  // in blocks without and with solids
+    } cases[] = {
+        {256, 256, true, true}, {1480, 740, true, true}, {12000, 6000, true, true}, {16384, 8192, false, false},
+        {32768, 8192, false, false}, {300000, 40, true, true}, {1000000, 2, true, true}, {2000000, 2, false, true},
+        {2000000, 4, true, true}, {4000000, 2, false, true}, {4000000, 4, false, true}, {4000000, 6, true, true},
+        {8000000, 4, false, true}, {20, 2, true, true}};
+    for (const auto& c : cases) {
+        const Geometry g = make_geometry(c.dim_x, c.dim_y, 7);
+        CHECK(block_lattice(g, false) == c.open && block_lattice(g, true) == c.solids, "%u x %u in blocks", c.dim_x, c.dim_y);
+    }
+}
+
 int main()
 {
+    check_block_lattices();
     check_coarse();
     check_short_calls();
     if (failures) {
