@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void setup_kernel(const JobInstall* __restrict
 __global__ __launch_bounds__(kDrawThreads) void batch_draw_kernel(const BatchJob* __restrict__ jobs,
                                                                   BatchState* state,
                                                                   const uint32_t* __restrict__ slots,
-                                                                  uint32_t nsteps)
+                                                                  uint32_t nsteps, bool few)
 {
     __shared__ DrawShared sh;
     const uint32_t slot = slots[blockIdx.y];
@@ -202,11 +202,12 @@ __global__ __launch_bounds__(kDrawThreads) void batch_draw_kernel(const BatchJob
     r.fw0 = j.a.fw0;
     r.fwn = j.a.fwn;
     r.dim_x = j.a.g.dim_x;
+    r.words = draw_words(few, j.force_q);
     const uint32_t groups = ((r.step0 & 3u) + nsteps + 3u) / 4u;
-    const uint64_t items = (r.plane + kDrawWords - 1) / kDrawWords * groups;
+    const uint64_t items = (r.plane + r.words - 1) / r.words * groups;
     for (uint64_t it = blockIdx.x; it < items; it += gridDim.x) {
         const uint64_t chunk = it / groups;
-        draw_chunk(r, chunk * kDrawWords, (uint32_t)(it - chunk * groups), sh);
+        draw_chunk(r, chunk * r.words, (uint32_t)(it - chunk * groups), sh);
     }
     // fdec_step0 is not the field the other blocks read
     if (blockIdx.x == 0 && threadIdx.x == 0) state[slot].fdec_step0 = r.step0;
@@ -1027,19 +1028,23 @@ void draw_windows(lgca_batch* b, const std::vector<int>& ks)
         hipchk(hipMalloc((void**)&b->d_draw, b->draw_cap * 4), "hipMalloc(draw list)");
     }
     upload(b, b->d_draw, slots.data(), slots.size() * 4);
-    uint64_t most = 0;
-    for (uint32_t s : slots) {
-        const Job* j = b->slot_job[s];
-        most = std::max<uint64_t>(most, (uint64_t)(j->p.fy1 - j->p.fy0) * j->p.fwn);
-    }
     // one workgroup per item of the largest region (9 groups when the window
     // starts inside one), as far as 1024
-    const uint32_t bx = (uint32_t)std::min<uint64_t>((most + kDrawWords - 1) / kDrawWords * (kWindow / 4 + 1), 1024);
+    constexpr uint64_t kGroups = kWindow / 4 + 1;
+    uint64_t chunks = 0, most = 0;
+    for (uint32_t s : slots) chunks += (force_words(b->slot_job[s]->p) + kDrawWords - 1) / kDrawWords;
+    const bool few = chunks * (kWindow / 4) < kDrawFew;
+    for (uint32_t s : slots) {
+        const JobParams& p = b->slot_job[s]->p;
+        const uint32_t words = draw_words(few, force_q(p.force_thr));
+        most = std::max(most, (force_words(p) + words - 1) / words * kGroups);
+    }
+    const uint32_t bx = (uint32_t)std::min<uint64_t>(most, 1024);
     // blockIdx.y covers at most 65535 jobs per launch
     for (size_t o = 0; o < slots.size(); o += 65535) {
         const uint32_t ny = (uint32_t)std::min<size_t>(65535, slots.size() - o);
         hipLaunchKernelGGL(batch_draw_kernel, dim3(bx, ny), dim3(kDrawThreads), 0, b->stream, b->d_jobs, b->d_state,
-                           b->d_draw + o, kWindow);
+                           b->d_draw + o, kWindow, few);
         hipchk(hipGetLastError(), "batch_draw_kernel");
     }
 }

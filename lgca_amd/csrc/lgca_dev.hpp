@@ -315,7 +315,22 @@ __device__ __forceinline__ uint32_t force_columns(uint32_t w, uint32_t fx0, uint
 // 6000 x 3000 cells forced at p = 5e-3, 28 steps: 59 -> 32 us (searching the
 // table by a logarithm and two reads: 41 for 39 at the time; results through
 // LDS to whole-line stores: 42).
+//
+// 1024 words leave the second pass few idle lanes where few words fire.  Where
+// most do (p >= 0.05, by q), or chunks of 1024 are fewer than two a CU (`few`), a
+// lane would walk four words' fires one after the other, and takes one.  64 steps
+// of FHP-II, us with chunks of 1024 / 256: 512 x 256 at p = 5e-3 65 / 59, p = 0.5
+// 305 / 123; 2048 x 512 at p = 1e-3 83 / 86, p = 0.5 343 / 201; 6000 x 3000 at p =
+// 5e-3 259 / 291, p = 0.5 1550 / 1435; 8192 x 4096 at p = 0.02 610 / 651, p = 0.1
+// 1101 / 1079.
 constexpr uint32_t kDrawThreads = 256, kDrawWords = 1024;
+constexpr uint64_t kDrawFew = 512;  // chunks
+__host__ __device__ inline bool draw_dense(uint32_t q) { return q <= 4080218932u; }
+__host__ __device__ inline uint32_t draw_words(bool few, uint32_t q)
+{
+    return few || draw_dense(q) ? kDrawThreads : kDrawWords;
+}
+
 struct DrawShared {
     uint32_t nQ[32];
     uint32_t count;
@@ -327,6 +342,7 @@ struct DrawRegion {
     uint64_t plane;             // (row, word) pairs
     uint32_t nsteps, step0, key0, key1;
     uint32_t fx0, fx1, fy0, fw0, fwn, dim_x;
+    uint32_t words;             // words of a chunk (draw_words)
 };
 
 // force_table has filled sh.nQ.  Group `group` is counted from step0 & ~3;
@@ -359,7 +375,7 @@ __device__ __forceinline__ void draw_chunk(const DrawRegion& a, uint64_t first_p
     };
     if (tid == 0) sh.count = 0;
     __syncthreads();
-    for (uint32_t k = 0; k < kDrawWords; k += kDrawThreads) {
+    for (uint32_t k = 0; k < a.words; k += kDrawThreads) {
         const uint64_t at = first_pair + k + tid;
         bool fires = false;
         U4 r{0, 0, 0, 0};

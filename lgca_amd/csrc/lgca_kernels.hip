@@ -223,15 +223,18 @@ __global__ __launch_bounds__(kDrawThreads) void force_draw_kernel(ForceDrawArgs 
     r.fw0 = a.fw0;
     r.fwn = a.fwn;
     r.dim_x = a.dim_x;
-    draw_chunk(r, (uint64_t)blockIdx.x * kDrawWords, blockIdx.y, sh);
+    r.words = a.words;
+    draw_chunk(r, (uint64_t)blockIdx.x * a.words, blockIdx.y, sh);
 }
 
-hipError_t launch_force_draw(const ForceDrawArgs& a, hipStream_t s)
+hipError_t launch_force_draw(const ForceDrawArgs& args, hipStream_t s)
 {
+    ForceDrawArgs a = args;
     const uint32_t groups = ((a.step0 & 3u) + a.nsteps + 3u) / 4u;
     const uint64_t n = (uint64_t)(a.fy1 - a.fy0) * a.fwn;
-    if ((n + kDrawWords - 1) / kDrawWords >= ((uint64_t)1 << 31) || groups > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(force_draw_kernel, dim3(div_up(n, kDrawWords), groups), dim3(kDrawThreads), 0, s, a);
+    a.words = draw_words((n + kDrawWords - 1) / kDrawWords * groups < kDrawFew, a.q);
+    if ((n + a.words - 1) / a.words >= ((uint64_t)1 << 31) || groups > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(force_draw_kernel, dim3(div_up(n, a.words), groups), dim3(kDrawThreads), 0, s, a);
     return hipGetLastError();
 }
 

@@ -281,6 +281,7 @@ struct ForceDrawArgs {
     uint32_t q;                 // first-fire sampling parameter, see force_q
     uint32_t fx0, fx1, fy0, fy1, fw0, fwn;
     uint32_t dim_x;
+    uint32_t words;             // words of a chunk, set at the launch
 };
 hipError_t launch_force_draw(const ForceDrawArgs& a, hipStream_t s);
 
