@@ -695,11 +695,12 @@ static lgca_status draw_decisions(lgca_lattice* h, uint32_t* dec, uint32_t nstep
 
 // Force decisions are drawn for a window of upcoming steps at once; a window
 // always starts at the current step and covers at least `need` steps.
+constexpr size_t kWindowWords = (size_t)(64ull << 20) / 4;
 static lgca_status prepare_decisions(lgca_lattice* h, uint64_t remaining, uint32_t need)
 {
     const size_t per_step = decision_words_per_step(h);
     // up to 64 steps, capped at 64 MiB of decision words, never fewer than `need`
-    size_t k = (size_t)(64ull << 20) / 4 / per_step;
+    size_t k = kWindowWords / per_step;
     if (k > 64) k = 64;
     if (k > remaining) k = (size_t)remaining;
     else if (k > need) k -= k % need;  // whole passes: a window's rest would be drawn again
@@ -1120,11 +1121,18 @@ static void plan_blocks(lgca_lattice* h)
 
 // Steps of the next block pass of `left` steps to go: whole passes, the rest
 // spread evenly over as many (an even split costs less than a short last
-// pass, whose launch and loads are the same).
+// pass, whose launch and loads are the same).  Where most words fire, drawing
+// them is most of the time, and a window that holds one pass draws whole groups
+// of four steps whatever it uses of them: passes are cut to whole groups there
+// (8192 x 4096 FHP-II forced everywhere, 64 steps at p = 0.5 2863 -> 2518 us).
 static uint32_t block_steps(const lgca_lattice* h, uint64_t left)
 {
     const uint64_t passes = (left + h->block_k - 1) / h->block_k;
-    return (uint32_t)((left + passes - 1) / passes);
+    const uint32_t k = (uint32_t)((left + passes - 1) / passes);
+    if (k > 4 && h->force_dir != LGCA_FORCE_NONE && draw_dense(force_q(h->force_thr)) &&
+        2 * k * decision_words_per_step(h) > kWindowWords)
+        return k & ~3u;
+    return k;
 }
 
 // A pass of k steps in blocks of shape s from the live state into the other

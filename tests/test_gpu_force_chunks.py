@@ -36,3 +36,23 @@ def test_large_draws_match_the_oracle(words, rows, p):
         b.wait(timeout=60)
         for i in ids:
             np.testing.assert_array_equal(b.result(i)[0], want)
+
+
+@pytest.mark.parametrize("p", [0.049, 0.5])
+def test_windows_of_one_pass(p):
+    """A region whose windows hold one pass: passes of whole groups of steps
+    where most words fire, and any number else, against a fixed shape."""
+    from lgca_amd import Lattice
+    dx, dy = 8200, 4000
+    print(f"[window] {dx}x{dy} p={p}", flush=True)
+    lats = [Lattice(2, dim_x=dx, dim_y=dy, coarse_graining_radius=1, seed=5) for _ in range(2)]
+    lats[1].set_tuning(4, 16)
+    for lat in lats:
+        lat.init_random(0.3)
+        lat.set_step(2)
+        lat.set_forcing("y", p)
+        for n in (3, 61, 14):
+            lat.step(n)
+    np.testing.assert_array_equal(lats[0].get_state_u8(), lats[1].get_state_u8())
+    for lat in lats:
+        lat.close()
