@@ -852,6 +852,9 @@ static std::vector<LaunchShape> trial_candidates(const lgca_lattice* h)
     for (uint32_t r : {4u, 8u, 12u, 16u, 20u, 24u, 32u}) add(base_k, r);
     if (h->tile_k == kAutoSteps) {  // (smaller lattices run in blocks)
         for (uint32_t r : {16u, 24u, 32u, 40u, 48u, 64u}) add(8, r);
+        // flat ones (block_lattice), which have no such tiles
+        if (h->dim_y < 16)
+            for (uint32_t r : {2u, 4u}) add(8, r);
         // Tiles tall enough that a pass's waves fill the GPU's wave slots
         // once (or twice) and no more: a pass with a few waves past a whole
         // number of rounds ends with a tail of them on an otherwise idle GPU
