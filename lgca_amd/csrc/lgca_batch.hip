@@ -334,6 +334,7 @@ struct Job {
     uint64_t step = 0;       // steps queued
     uint32_t cur = 0;        // buffer holding the state after the queued steps
     uint64_t window_end = 0; // force decisions exist for steps < window_end
+    std::unique_ptr<RoundTerms> terms;  // for the round planner, from its first prediction on
     hipEvent_t done_ev = nullptr;
     hipEvent_t last_ev = nullptr;  // end of the job's last round on the main stream
 };
@@ -865,8 +866,14 @@ std::vector<RoundJob> round_jobs(const lgca_batch* b)
 {
     std::vector<RoundJob> v;
     v.reserve(b->active.size());
-    for (const Job* j : b->active)
+    for (Job* j : b->active) {
         v.push_back(RoundJob{j->p.g, j->p.kind, j->p.has_mask || j->p.forced, force_words(j->p), j->d.steps - j->step});
+        if (!j->terms) {
+            j->terms = std::make_unique<RoundTerms>();
+            round_terms(v.back(), *j->terms);
+        }
+        v.back().terms = j->terms.get();
+    }
     return v;
 }
 

@@ -230,8 +230,8 @@ hipError_t launch_tile_batch(int k, bool ragged, const BatchJob* jobs, BatchStat
 // enough for about `waves` waves, or blocks of m rows per wave and `waves` waves
 // per workgroup.
 struct RoundShape {
-    int k;
-    uint32_t waves;
+    int k = 0;
+    uint32_t waves = 0;
     uint32_t m = 0;
 };
 // What the shape of a round of blocks depends on of a running job.
@@ -241,7 +241,14 @@ struct RoundJob {
     bool feat;             // solids or forcing
     uint64_t force_words;  // decision words of a step (0: not forced)
     uint64_t left;         // steps to go
+    const struct RoundTerms* terms = nullptr;  // round_terms, or null
 };
+// A job's part of a round's predicted time, for each of the shapes considered.
+constexpr uint32_t kRoundShapes = 21;
+struct RoundTerms {
+    float work[kRoundShapes], wait[kRoundShapes], most[kRoundShapes], bytes[kRoundShapes];
+};
+void round_terms(const RoundJob& job, RoundTerms& terms);
 // Blocks of a job's k-step round: rows per block, row tiles, blocks.
 struct JobBlocks {
     uint32_t th, tiles, blocks;
@@ -249,8 +256,6 @@ struct JobBlocks {
 JobBlocks job_blocks(const Geometry& g, const RoundShape& s, int k);
 // Steps that a job with `left` to go makes in a round of blocks of shape s.
 int round_steps(const RoundShape& s, uint64_t left, uint64_t force_words);
-// Predicted time (us) of a round of the jobs in blocks of shape s.
-float round_us(const std::vector<RoundJob>& jobs, const RoundShape& s);
 // The block shapes that a round of the jobs may take, those with the least
 // predicted time per step first; never none.  window: steps of a force window.
 std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window);

@@ -3,10 +3,16 @@
 // through one buffer descriptor, in which offset 2^31 and up must mean "no
 // decision" (kOutside in lgca_block.hpp), so the decisions of any pass stay
 // below 2 GiB, whatever was running when the shape was chosen.
+// A prediction from the jobs' kept terms chooses what one from the start does, at
+// a small part of its cost, which the worker pays whenever a job comes or ends.
 // Prints "ROUNDS PASSED" and exits 0 when every check holds.
 #include "lgca_kernels.hpp"
 
+#include <algorithm>
+#include <chrono>
 #include <cstdio>
+#include <memory>
+#include <random>
 #include <vector>
 
 using namespace lgca;
@@ -66,9 +72,51 @@ static void check_force_bound()
         CHECK(round_steps(s, 1000, 64 * 1024) == s.k, "steps of an ordinary job");
 }
 
+static void check_kept_terms()
+{
+    std::mt19937 rng(7);
+    for (int mix = 0; mix < 60; ++mix) {
+        std::vector<RoundJob> fresh, kept;
+        std::vector<std::unique_ptr<RoundTerms>> terms;
+        const uint32_t n = 1 + rng() % 40;
+        for (uint32_t i = 0; i < n; ++i) {
+            const uint32_t dim_x = 20 + rng() % (mix % 3 ? 400 : 9000), dim_y = 2 + 2 * (rng() % 800);
+            RoundJob j = job((int)(rng() % 3), dim_x, dim_y, mix % 4 == 3 && rng() % 2 ? rng() % 100000 + 1 : 0, 1000);
+            if (mix == 59 && !i) j = job(2, 65536, 32768, 2000ull * 32768, 1000);  // cut to 8 steps
+            terms.push_back(std::make_unique<RoundTerms>());
+            round_terms(j, *terms.back());
+            j.left = rng() % 4 ? 24 + rng() % 500 : 1 + rng() % 30;
+            fresh.push_back(j);
+            j.terms = terms.back().get();
+            kept.push_back(j);
+        }
+        const std::vector<RoundShape> a = round_shapes(fresh, kWindow), b = round_shapes(kept, kWindow);
+        CHECK(a.size() == b.size() && !a.empty(), "shapes of mix %d", mix);
+        for (size_t i = 0; i < std::min(a.size(), b.size()); ++i)
+            CHECK(a[i].k == b[i].k && a[i].m == b[i].m && a[i].waves == b[i].waves, "mix %d, shape %zu", mix, i);
+    }
+    std::vector<RoundJob> jobs(4000, job(2, 64, 64, 0, 1000));
+    auto seconds = [&] {
+        double best = 1e9;
+        for (int rep = 0; rep < 10; ++rep) {
+            const auto t0 = std::chrono::steady_clock::now();
+            (void)round_shapes(jobs, kWindow);
+            best = std::min(best, std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+        }
+        return best;
+    };
+    const double anew = seconds();
+    RoundTerms terms;
+    round_terms(jobs[0], terms);
+    for (RoundJob& j : jobs) j.terms = &terms;
+    const double kept = seconds();
+    CHECK(kept * 5 < anew, "4000 jobs: %.0f us with kept terms, %.0f anew", kept * 1e6, anew * 1e6);
+}
+
 int main()
 {
     check_force_bound();
+    check_kept_terms();
     if (failures) {
         std::printf("%d checks failed\n", failures);
         return 1;
