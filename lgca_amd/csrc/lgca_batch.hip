@@ -223,6 +223,7 @@ constexpr size_t kAlign = 256;
 constexpr size_t kStagingHalf = 32u << 20;  // pinned upload staging, two halves
 constexpr uint32_t kMinTileRows = 8, kMaxTileRows = 512;
 constexpr int kTuneRounds = 3;            // rounds timed per candidate
+constexpr uint64_t kPredictedRows = 26112;  // wave-rows below which block shapes are predicted, not timed
 
 size_t align_up(size_t v) { return (v + kAlign - 1) & ~(kAlign - 1); }
 
@@ -1065,7 +1066,7 @@ void start_tuning(lgca_batch* b, int user_k, uint32_t user_waves, uint64_t wr)
     if (!user_k && !user_waves) {
         // the blocks predicted fastest against the walks that win on mixes
         // which fill the GPU
-        const std::vector<RoundShape> blocks = round_shapes(round_jobs(b), kWindow);
+        const std::vector<RoundShape> blocks = round_shapes(round_jobs(b), kWindow, b->ncu);
         for (size_t i = 0; i < blocks.size() && i < 3; ++i) b->cands.push_back(blocks[i]);
         for (int k : ks)
             for (uint32_t w : {2048u, 4096u}) b->cands.push_back(RoundShape{k, w});
@@ -1139,8 +1140,10 @@ void run_round(lgca_batch* b)
     // restarts only when the mix has grown 4x since it began.
     // A mix too small to fill the GPU with walks takes the block shape predicted
     // fastest for the jobs still running, untimed: its rounds are short and its
-    // jobs keep ending.
-    if (!user_k && !user_waves && wr_now < 3 * 8704) {
+    // jobs keep ending.  Whole runs, predicted / timed: ensembles of 10,542
+    // wave-rows 9.0 / 9.5 ms, 22,104 13.5 / 14.5, 35,014 19.6 / 19.6, 76,336 37.5 / 37.7;
+    // serving mixes of 8,714 9.4 / 10.3, 35,196 20.9 / 22.4, 70,600 41.0 / 39.7.
+    if (!user_k && !user_waves && wr_now < kPredictedRows) {
         if (b->tuning || b->evaluating) {
             b->tuning = b->evaluating = false;
             b->mix_key = 0;
@@ -1149,7 +1152,7 @@ void run_round(lgca_batch* b)
         for (const Job* j : b->active) key = key * 0x100000001B3ull ^ j->id;
         if (key != b->mix_key) {
             b->mix_key = key;
-            b->cur = round_shapes(round_jobs(b), kWindow).front();
+            b->cur = round_shapes(round_jobs(b), kWindow, b->ncu).front();
         }
         b->tuned_wave_rows = 0;  // a mix that grows past this is tuned at once
     } else if (!b->tuning && !b->evaluating) {

@@ -258,7 +258,7 @@ JobBlocks job_blocks(const Geometry& g, const RoundShape& s, int k);
 int round_steps(const RoundShape& s, uint64_t left, uint64_t force_words);
 // The block shapes that a round of the jobs may take, those with the least
 // predicted time per step first; never none.  window: steps of a force window.
-std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window);
+std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window, uint32_t ncu);
 
 // Launchers of one (model, K) pair and of one K's batch kernel, instantiated
 // by lgca_tile_inst.hip; grid and shapes come checked from launch_tile /

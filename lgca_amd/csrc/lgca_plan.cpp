@@ -406,7 +406,7 @@ void round_terms(const RoundJob& job, RoundTerms& terms)
 // whenever a job comes or ends, with the GPU at most a few rounds behind.  A
 // prediction from the start / from the terms: 1000 jobs of 128 x 128 1.1 ms / 10 us
 // (rounds of 37 us), 4000 of 64 x 64 4.6 ms / 44 us (rounds of 122).
-std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window)
+std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t window, uint32_t ncu)
 {
     constexpr uint64_t kMostSteps = kShapes.shape[kRoundShapes - 1].k;
     RoundTerms sum{};
@@ -426,13 +426,14 @@ std::vector<RoundShape> round_shapes(const std::vector<RoundJob>& jobs, uint32_t
             sum.bytes[i] += t->bytes[i];
         }
     }
+    const float cus = (float)std::max(ncu, 1u);
     std::vector<std::pair<float, RoundShape>> v;
     for (uint32_t i = 0; i < kRoundShapes; ++i) {
         const RoundShape& s = kShapes.shape[i];
         // with a forced job the steps divide the window and keep its decisions in bounds
         if (most_words && (window % (uint32_t)s.k || (uint64_t)s.k > force_pass_steps(most_words))) continue;
         const uint32_t fit = std::max(1u, std::min(16u / s.waves, 160u * 1024u / block_lds_bytes(2, s.m, s.waves)));
-        const float us = 4.5f + std::max(sum.most[i], sum.work[i] / 256.0f + sum.wait[i] / (256.0f * (float)fit)) +
+        const float us = 4.5f + std::max(sum.most[i], sum.work[i] / cus + sum.wait[i] / (cus * (float)fit)) +
                          0.5f * sum.bytes[i] / 4.5e6f;
         v.emplace_back(us / (float)s.k, s);
     }

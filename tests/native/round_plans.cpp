@@ -28,7 +28,7 @@ static int failures = 0;
         }                                        \
     } while (0)
 
-constexpr uint32_t kWindow = 32;
+constexpr uint32_t kWindow = 32, kCus = 256;
 
 static RoundJob job(int kind, uint32_t dim_x, uint32_t dim_y, uint64_t force_words, uint64_t left)
 {
@@ -51,7 +51,7 @@ static void check_force_bound()
             CHECK(words * 8 * 4 < (1ull << 31) && force_pass_steps(words) >= 8, "an accepted region (%u x %u words)", r.words, r.rows);
             std::vector<std::vector<RoundJob>> mixes = {{forced}, {job(2, 512, 512, 0, 100), forced, job(0, 64, 64, 128, 7)}};
             for (const auto& mix : mixes) {
-                const std::vector<RoundShape> shapes = round_shapes(mix, kWindow);
+                const std::vector<RoundShape> shapes = round_shapes(mix, kWindow, kCus);
                 CHECK(!shapes.empty(), "a shape for every mix");
                 for (const RoundShape& s : shapes) {
                     CHECK(s.k * words * 4 < (1ull << 31), "%d steps of %u x %u words", s.k, r.words, r.rows);
@@ -59,7 +59,7 @@ static void check_force_bound()
                 }
             }
             // shapes chosen before the job was admitted
-            for (const RoundShape& s : round_shapes({job(kind, 2048, 1024, 0, 1000)}, kWindow))
+            for (const RoundShape& s : round_shapes({job(kind, 2048, 1024, 0, 1000)}, kWindow, kCus))
                 for (uint64_t left : {1ull, 3ull, 7ull, 8ull, 15ull, 16ull, 1000ull}) {
                     const int k = round_steps(s, left, words);
                     CHECK(k >= 1 && (uint64_t)k <= left && k <= s.k, "%d of %d steps", k, s.k);
@@ -68,7 +68,7 @@ static void check_force_bound()
                 }
         }
     // small regions change nothing
-    for (const RoundShape& s : round_shapes({job(2, 2048, 1024, 0, 1000)}, kWindow))
+    for (const RoundShape& s : round_shapes({job(2, 2048, 1024, 0, 1000)}, kWindow, kCus))
         CHECK(round_steps(s, 1000, 64 * 1024) == s.k, "steps of an ordinary job");
 }
 
@@ -90,7 +90,7 @@ static void check_kept_terms()
             j.terms = terms.back().get();
             kept.push_back(j);
         }
-        const std::vector<RoundShape> a = round_shapes(fresh, kWindow), b = round_shapes(kept, kWindow);
+        const std::vector<RoundShape> a = round_shapes(fresh, kWindow, kCus), b = round_shapes(kept, kWindow, kCus);
         CHECK(a.size() == b.size() && !a.empty(), "shapes of mix %d", mix);
         for (size_t i = 0; i < std::min(a.size(), b.size()); ++i)
             CHECK(a[i].k == b[i].k && a[i].m == b[i].m && a[i].waves == b[i].waves, "mix %d, shape %zu", mix, i);
@@ -100,7 +100,7 @@ static void check_kept_terms()
         double best = 1e9;
         for (int rep = 0; rep < 10; ++rep) {
             const auto t0 = std::chrono::steady_clock::now();
-            (void)round_shapes(jobs, kWindow);
+            (void)round_shapes(jobs, kWindow, kCus);
             best = std::min(best, std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
         }
         return best;
@@ -113,8 +113,20 @@ static void check_kept_terms()
     CHECK(kept * 5 < anew, "4000 jobs: %.0f us with kept terms, %.0f anew", kept * 1e6, anew * 1e6);
 }
 
+// A device with fewer CUs takes longer over the same work: a mix that leaves
+// 256 of them half idle takes tall blocks of few redundant rows on 16.
+static void check_cus()
+{
+    const std::vector<RoundJob> mix = {job(2, 2048, 512, 0, 1000), job(2, 1024, 1024, 0, 1000)};
+    const RoundShape wide = round_shapes(mix, kWindow, 256).front(), narrow = round_shapes(mix, kWindow, 16).front();
+    const JobBlocks a = job_blocks(mix[0].g, wide, wide.k), b = job_blocks(mix[0].g, narrow, narrow.k);
+    const double da = (double)(wide.m * wide.waves) / a.th, db = (double)(narrow.m * narrow.waves) / b.th;  // rows held per stored one
+    CHECK(db < da, "16 CUs: %.2f rows held per stored one, 256: %.2f", db, da);
+}
+
 int main()
 {
+    check_cus();
     check_force_bound();
     check_kept_terms();
     if (failures) {
