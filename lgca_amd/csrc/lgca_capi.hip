@@ -1590,6 +1590,7 @@ extern "C" lgca_status lgca_apply_body_force_count(lgca_lattice* h, int dir, int
     if (st0) return st0;
     lgca_status st = clear_counters(h);
     if (st) return st;
+    if ((st = ensure_force_ws(h, target))) return st;  // before the call counts
     CountForceArgs a{};
     a.call = (uint32_t)h->force_calls++;
     a.amount = target;
