@@ -415,6 +415,7 @@ extern "C" lgca_status lgca_get_info(const lgca_lattice* h, lgca_info* info)
     if (h->cell_momentum) dev += info->num_cells * 8;
     if (h->mean_density) dev += info->num_coarse_cells * 20;
     if (h->bytes) dev += info->num_cells;
+    dev += h->force_ws_bytes;
     info->device_bytes = dev;
     info->step = h->step;
     info->seed = h->seed;
