@@ -1183,7 +1183,8 @@ static lgca_status tune_blocks(lgca_lattice* h)
     if (cand.size() > kTuneBlocks) cand.resize(kTuneBlocks);
     const uint32_t* fdec = nullptr;
     if (forcing) {
-        const uint32_t need = kBlockMaxSteps;
+        uint32_t need = 1;
+        for (const Candidate& c : cand) need = std::max(need, c.k);
         if (h->dec_count == 0 || h->step < h->dec_step0 || h->step + need > h->dec_step0 + h->dec_count) {
             lgca_status st = prepare_decisions(h, 64, need);
             if (st) return st;
