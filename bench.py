@@ -170,7 +170,7 @@ def time_steps(w, steps: int, warmup: int, tuning=None, tune: bool = True):
     end.record(stream)
     end.synchronize()
     coarse_ms = start.elapsed_ms(end)
-    info = lat.info()
+    shape = lat.pass_shape()
     lat.close()
     start.close()
     end.close()
@@ -178,7 +178,7 @@ def time_steps(w, steps: int, warmup: int, tuning=None, tune: bool = True):
     sups = n * steps / (ms / 1e3)
     achieved = n * 2 * Q[w["model"]] / 8 * steps / (ms / 1e3) / 1e9
     return dict(ms=ms, wall=wall, sups=sups, achieved=achieved, conserved=n0 == n1,
-                steps_per_pass=int(info.steps_per_pass), tile_rows=int(info.tile_rows),
+                steps_per_pass=int(shape.steps), tile_rows=int(shape.rows), blocks=bool(shape.blocks),
                 coarse_ms=coarse_ms)
 
 
@@ -192,7 +192,7 @@ def other_configs():
         out[key] = {
             "workload": w["label"], "steps": steps, "ms_per_step": round(r["ms"] / steps, 6),
             "value": round(r["sups"] / 1e9, 3), "unit": "GSUP/s",
-            "steps_per_pass": r["steps_per_pass"], "tile_rows": r["tile_rows"],
+            "steps_per_pass": r["steps_per_pass"], "tile_rows": r["tile_rows"], "blocks": r["blocks"],
             "roofline": {"bound": "hbm", "achieved": round(r["achieved"], 1),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(r["achieved"] / HBM_PEAK_GBS, 4)},

@@ -61,8 +61,8 @@ typedef struct lgca_info {
     uint32_t tile_rows;      /* rows per tile of the tiled kernel's steps_per_pass
                                 launches: lgca_set_tuning's value, else the height
                                 the timed trial of the first launches chose (0
-                                until it has); lattices that run in blocks
-                                (lgca_set_tuning) report the fixed rule's       */
+                                until it has); lattices that run in blocks report
+                                the fixed rule's (lgca_get_pass: what they run) */
     uint64_t num_cells;
     uint64_t num_coarse_cells;
     uint64_t state_bytes;    /* one state buffer: dim_y * Q * row_pitch * 4   */
@@ -75,6 +75,16 @@ typedef struct lgca_info {
     uint32_t pass_pipeline;  /* 1 when lgca_set_pipeline has turned on launches
                                 of several passes                               */
 } lgca_info;
+
+/* The passes that longer lgca_step calls make as the handle stands. */
+typedef struct lgca_pass {
+    int32_t blocks;          /* 1: in blocks (lgca_set_tuning), 0: the tiled kernel
+                                or the one-step kernel                          */
+    uint32_t steps;          /* steps per pass; 0 until the first call or lgca_tune
+                                has decided                                     */
+    uint32_t rows;           /* rows stored per block or tile (one-step kernel: 0) */
+    uint32_t waves;          /* waves per workgroup of a block (tiles: 1)        */
+} lgca_pass;
 
 /* Creates a lattice of dim_x x dim_y cells on GPU `device`, all FLUID and
  * empty.  Replaces the constructors Lattice(...) / OMP_Lattice(...)
@@ -91,6 +101,7 @@ LGCA_API lgca_status lgca_destroy(lgca_lattice* h);
 /* Text of the last failure on h (or of the last failed lgca_create when h is NULL). */
 LGCA_API const char* lgca_last_error(const lgca_lattice* h);
 LGCA_API lgca_status lgca_get_info(const lgca_lattice* h, lgca_info* info);
+LGCA_API lgca_status lgca_get_pass(const lgca_lattice* h, lgca_pass* pass);
 
 /* Queue work on an external HIP stream (a hipStream_t; NULL restores the
  * handle's own stream). */

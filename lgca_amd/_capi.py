@@ -33,6 +33,10 @@ class Info(C.Structure):
     ]
 
 
+class Pass(C.Structure):
+    _fields_ = [("blocks", C.c_int32), ("steps", C.c_uint32), ("rows", C.c_uint32), ("waves", C.c_uint32)]
+
+
 GEOM_PERIODIC, GEOM_PIPE, GEOM_CYLINDER, GEOM_TYPES = range(4)
 JOB_QUEUED, JOB_RUNNING, JOB_DONE, JOB_RELEASED, JOB_FAILED = range(5)
 ALL_JOBS = 2 ** 64 - 1
@@ -71,6 +75,7 @@ SIGNATURES = {
     "lgca_create": [C.POINTER(_h), C.c_int, C.c_uint32, C.c_uint32, C.c_uint32, C.c_int],
     "lgca_destroy": [_h],
     "lgca_get_info": [_h, C.POINTER(Info)],
+    "lgca_get_pass": [_h, C.POINTER(Pass)],
     "lgca_set_stream": [_h, C.c_void_p],
     "lgca_synchronize": [_h],
     "lgca_set_seed": [_h, C.c_uint64],

@@ -1097,6 +1097,21 @@ static bool uses_blocks(const lgca_lattice* h)
     return h->tile_k == kAutoSteps && !h->tile_th && block_lattice(h->g, h->mask != nullptr);
 }
 
+extern "C" lgca_status lgca_get_pass(const lgca_lattice* h, lgca_pass* pass)
+{
+    if (!h || !pass) return LGCA_ERR_INVALID_ARGUMENT;
+    if (uses_blocks(h)) {
+        const BlockShape s = h->block_k ? h->block[h->block_k] : BlockShape{0, 0, 0};
+        *pass = lgca_pass{1, h->block_k, s.th, s.waves};
+    } else if (h->tile_k == 0) {
+        *pass = lgca_pass{0, 1, 0, 1};
+    } else {
+        const LaunchShape s = h->tile_th ? LaunchShape{h->tile_k == kAutoSteps ? 4 : h->tile_k, h->tile_th + (h->tile_th & 1u)} : h->tuned;
+        *pass = lgca_pass{0, s.th ? (uint32_t)s.k : 0u, s.th, 1};
+    }
+    return LGCA_OK;
+}
+
 // Decides the block shapes from the pass-time model: the best for every number
 // of steps, and the steps per pass with the least time per step.  lgca_info
 // reports the walk's rule for such lattices, which run no trial.

@@ -212,6 +212,12 @@ class Lattice:
         self._check(lib().lgca_get_info(self._h, C.byref(inf)))
         return inf
 
+    def pass_shape(self) -> capi.Pass:
+        """The passes that longer step calls make as the lattice stands."""
+        p = capi.Pass()
+        self._check(lib().lgca_get_pass(self._h, C.byref(p)))
+        return p
+
     # -------------------------------------------------------------- extras
     def set_seed(self, seed: int) -> None:
         self._check(lib().lgca_set_seed(self._h, int(seed) & (2**64 - 1)))
