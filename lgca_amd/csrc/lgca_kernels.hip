@@ -956,7 +956,7 @@ hipError_t launch_count(const uint32_t* words, uint64_t nwords, unsigned long lo
 // A word of 32 cells is summed at once: the density's three bits come from a
 // chain of full adders, and for every density the momentum of its cells is a
 // few popcounts (about 100 operations a word, against 30 for each cell taken
-// one by one).  A workgroup covers 1 << tw_log words of 1024 >> tw_log rows.
+// one by one).  A workgroup covers 1 << tw_log words of 1024 >> tw_log rows at a time.
 template <int KIND>
 __global__ __launch_bounds__(kReduceThreads) void mean_velocity_kernel(const uint32_t* __restrict__ planes,
                                                                        const uint32_t* __restrict__ mask,
@@ -967,7 +967,7 @@ __global__ __launch_bounds__(kReduceThreads) void mean_velocity_kernel(const uin
     const uint32_t tw = 1u << tw_log, rows = kReduceThreads >> tw_log;
     unsigned long long sum[3] = {0, 0, 0};
     for (uint32_t y = blockIdx.x * rows + (threadIdx.x >> tw_log); y < g.dim_y; y += gridDim.x * rows) {
-        for (uint32_t w = threadIdx.x & (tw - 1u); w < g.W; w += tw) {
+        for (uint32_t w = blockIdx.y * tw + (threadIdx.x & (tw - 1u)); w < g.W; w += gridDim.y * tw) {
             uint32_t fluid = valid_mask(g, w);
             if (mask)
                 fluid &= ~(mask[((size_t)y * 2 + 0) * g.P + w] | mask[((size_t)y * 2 + 1) * g.P + w]);
@@ -1021,7 +1021,10 @@ hipError_t launch_mean_velocity(int kind, const uint32_t* planes, const uint32_t
 {
     uint32_t tw_log = 0;
     while ((1u << tw_log) < g.W && (1u << tw_log) < kReduceThreads) ++tw_log;
-    const dim3 grid(std::min(div_up(g.dim_y, kReduceThreads >> tw_log), kReduceBlocks)), block(kReduceThreads);
+    // a workgroup per row (or rows); flat lattices share long rows out too (20000000 x
+    // 2 FHP-II 936 us a call with a workgroup per row, 28 so)
+    dim3 grid(std::min(div_up(g.dim_y, kReduceThreads >> tw_log), kReduceBlocks)), block(kReduceThreads);
+    grid.y = std::max(1u, std::min(div_up(g.W, 1u << tw_log), kReduceBlocks / grid.x));
     unsigned long long* acc = (unsigned long long*)acc3;
     switch (kind) {
     case kHPP: hipLaunchKernelGGL(mean_velocity_kernel<kHPP>, grid, block, 0, s, planes, mask, g, tw_log, acc); break;
