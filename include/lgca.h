@@ -171,7 +171,8 @@ LGCA_API lgca_status lgca_step_noalloc(lgca_lattice* h, uint64_t nsteps);
  * automatic, the trial chooses 4 or 8 steps per pass on a lattice large enough
  * to fill the GPU with tiles; smaller ones run in blocks of rows held in
  * registers, up to 28 steps per pass, in shapes predicted from the size (and
- * timed by lgca_tune).  Results do not depend on it.  No counterpart in the reference; used by the autotuner and
+ * timed by lgca_tune); their calls of 1, 2 or 4 steps take one pass of tiles
+ * where that is faster.  Results do not depend on it.  No counterpart in the reference; used by the autotuner and
  * benchmarks. */
 LGCA_API lgca_status lgca_set_tuning(lgca_lattice* h, int steps_per_pass, uint32_t tile_rows);
 /* Several passes of 4 or 8 steps per launch (on = 1; 0, the default, launches

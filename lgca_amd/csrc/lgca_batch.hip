@@ -3,11 +3,11 @@
 //
 // A batch keeps every admitted job's bit-planes resident in one device arena
 // and advances all of them together.  A round gives each running job k steps
-// (k = the tuned steps per pass, less at a job's end) and is one launch of
-// tile_batch_kernel per (model, k, ragged width) class; the wave that finishes
-// a job's last work item of the round moves the job's step and buffer parity
-// on the device.
-// Work items (one per wave: job, x-strip, row tile, tile shape) are rebuilt
+// (k = the round's steps, less at a job's end) in one launch of
+// block_batch_kernel per ragged or whole width, or of tile_batch_kernel per (k,
+// ragged or whole width); the workgroup that finishes a job's last work item of
+// the round moves the job's step and buffer parity on the device.
+// Work items (one per workgroup: job, x-strip, row tile, its shape) are rebuilt
 // only when the set of running jobs or the tuning changes, so a steady stretch
 // of rounds is launches alone.  Per-cell force decisions are drawn for windows
 // of kWindow steps by one launch over all forced jobs that need a new window.

@@ -188,7 +188,7 @@ hipError_t launch_block_km(const BlockArgs& b, uint32_t waves, uint32_t blocks, 
 // Batched ensembles.  BatchJob is a job's static descriptor (its TileArgs
 // without src/dst/t0/th/halo, which come from BatchState and WorkItem);
 // BatchState is the job's dynamic state on the device; a WorkItem is one
-// wave's tile.
+// workgroup's tile (one wave) or block.
 struct BatchJob {
     TileArgs a;            // geometry, masks, keys, force region and window base
     uint32_t* buf0;
@@ -200,20 +200,19 @@ struct BatchState {
     uint32_t step;         // absolute step (mod 2^32)
     uint32_t cur;          // 0: state in buf0, 1: in buf1
     uint32_t fdec_step0;   // step of the first decision plane at a.fdec
-    uint32_t done;         // waves of the current round that have finished
+    uint32_t done;         // workgroups of the current round that have finished
 };
 struct WorkItem {
-    uint32_t job, strip, tile;  // segment mode: strip 0, tile = group of 64 / W row tiles
-    uint32_t shape;        // rows per tile | halo << 16 | segment mode << 31
+    // segment mode: strip 0, tile = group of 64 / W row tiles (blocks: row tile);
+    // packed blocks: strip = the block's share of the sequence, tile 0
+    uint32_t job, strip, tile;
+    uint32_t shape;        // rows per tile | halo << 16 | segment mode << 31; blocks: block_shape_bits
     uint32_t job_items;    // items of this job in the round
 };
-// One class launch of a round: every item (all of one K and raggedness, any
-// models) advances its job K steps reading its BatchState.  The wave that
-// finishes a job's last item of the round moves the job K steps on and swaps
-// its buffers, for the next round's launches to read.
-// n_heavy: the class's leading items that can take the general walk.
-// The same in blocks of m rows per wave, `waves` waves per workgroup (one per
-// item; item shapes are block_shape_bits, steps included).
+// One class launch of a round of blocks of m rows per wave, `waves` waves per
+// workgroup: every item (any models, steps in its shape) advances its job
+// reading its BatchState.  n_heavy: the leading items that can take the general
+// walk, or hold solids or forcing.
 hipError_t launch_block_batch(uint32_t m, uint32_t waves, bool ragged, const BatchJob* jobs, BatchState* state,
                               const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s);
 template <int M>
@@ -223,6 +222,9 @@ inline uint32_t block_shape_bits(uint32_t th, uint32_t halo, uint32_t k, BlockLa
 {
     return th | (halo << 16) | (lanes == kLanesPacked ? 1u << 23 : 0u) | (k << 24) | (lanes == kLanesRows ? 1u << 31 : 0u);
 }
+// One class launch of a round of walks: the same for items all of one K and
+// raggedness.  In both, whoever finishes a job's last item of the round moves
+// the job on and swaps its buffers, for the next round's launches to read.
 hipError_t launch_tile_batch(int k, bool ragged, const BatchJob* jobs, BatchState* state,
                              const WorkItem* items, uint32_t n_items, uint32_t n_heavy, hipStream_t s);
 

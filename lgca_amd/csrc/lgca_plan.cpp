@@ -295,7 +295,10 @@ std::vector<BlockShape> block_shapes(const Geometry& g, int kind, uint32_t k)
 // steps on 256 x 256 HPP (0.12 us a step), the 2048 x 512 FHP-II pipe (0.45)
 // and 4400 x 2200 FHP-II (1.6); the best predicted shape was within 10 % of
 // the best measured one on each, and is with the shorter collision (constants
-// a sixth smaller pick no better shapes).
+// a sixth smaller pick no better shapes).  Forced lattices past 8192 x 4096 are
+// the exception: the model does not know that six rows a wave spill with solids
+// or forcing (10000 x 4000 FHP-II forced everywhere 7.9 us a step, 6.3 in the
+// four-row shape that lgca_tune finds; 8192 x 4096 6.0 and 5.5).
 float block_pass_us(const Geometry& g, int kind, bool feat, uint32_t ncu, uint32_t k, const BlockShape& s)
 {
     const bool seg = tile_segments(g, (int)k);
