@@ -1198,7 +1198,7 @@ static lgca_status tune_blocks(lgca_lattice* h)
     if (cand.size() > kTuneBlocks) cand.resize(kTuneBlocks);
     const uint32_t* fdec = nullptr;
     if (forcing) {
-        uint32_t need = 1;
+        uint32_t need = 4;
         for (const Candidate& c : cand) need = std::max(need, c.k);
         if (h->dec_count == 0 || h->step < h->dec_step0 || h->step + need > h->dec_step0 + h->dec_count) {
             lgca_status st = prepare_decisions(h, 64, need);
@@ -1231,6 +1231,16 @@ static lgca_status tune_blocks(lgca_lattice* h)
         h->block[best.k] = best.s;
         for (uint32_t k = 1; k < best.k && e == hipSuccess; ++k)
             if (h->block[k].m) e = launch_block_pass(h, k, h->block[k], fdec, t0);
+    }
+    // the walks of short calls, whose kernels are compiled per step offset
+    for (int k = 1; k <= 4 && e == hipSuccess; k *= 2) {
+        const uint32_t th = short_walk_rows(h->g, h->kind, (uint64_t)k);
+        for (uint32_t o = 0; th && o < 4 && (k > 1 || o == 0) && e == hipSuccess; ++o) {
+            TileArgs a = with_k(tile_args(h, th, fdec), k);
+            a.t0 += o;
+            const OrderRef ord = wave_order(h, k, a, true);
+            e = launch_tile(h->kind, k, a, h->stream, ord.dev, ord.n);
+        }
     }
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     for (hipEvent_t v : ev)
